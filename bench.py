@@ -103,10 +103,10 @@ def kernel_bytes(p):
         "correct_velocity": 7 * R, "correct_pressure": 3 * R,
         "max_cfl": 3 * R, "max_div": 3 * R,
         # RK3 substep 1: ro = 0, the history ru is written but not read
-        "helm_fwd": 10 * R,          # qt qr qz pr | ru1 ru2 ru3 yt yr yz
+        "helm_fwd": 10 * R,          # qt qr qz pr | ru1 ru2 ru3 gt gr gz
         # substeps 2 and 3: the previous substep's correction applied on the fly
-        "helm_fwd_corr": 15 * R,     # qt qr qz pr dph ru1 ru2 ru3 | ru1 ru2 ru3 yt yr yz pr
-        "helm_bwd": 6 * R,           # yt yr yz (U q + y) | qt qr qz
+        "helm_fwd_corr": 15 * R,     # qt qr qz pr dph ru1 ru2 ru3 | ru1 ru2 ru3 gt gr gz pr
+        "helm_bwd": 6 * R,           # gt gr gz (sc*rhs + A q) | qt qr qz
         "diagnostics": 3 * R,        # qt qr qz -> 10 scalars
         # last correction of a logging step with the diagnostics on the
         # corrected fields: qt qr qz pr dph | qt qr qz pr
@@ -431,22 +431,23 @@ def served_leg(tc, njobs):
 
 
 def _kernel_short(name):
-    """'void tc::k_helm_fwd<true, 2>(tc::GridDev, ...)' -> 'k_helm_fwd<true, 2>'."""
+    """'void tc::k_helm_rhs<true, 2>(tc::GridDev, ...)' -> 'k_helm_rhs<true, 2>'."""
     name = name.replace("void ", "").split("(")[0]
     return name.split("::", 1)[1] if "::" in name else name
 
 
 # device kernels whose timer name differs from the kernel name
-_KERNEL_TIMER = {"k_correct_both2": "correct_both"}
+_KERNEL_TIMER = {"k_correct_both2": "correct_both", "k_helm_rhs": "helm_fwd",
+                 "k_helm_solve": "helm_bwd"}
 
 
 def _timer_of(kernel):
     """Kernel timer name (the kernel_bytes key) of a device kernel name."""
     base = kernel.split("<")[0]
+    if base == "k_helm_rhs" and kernel.replace(" ", "").endswith(",true>"):
+        return "helm_fwd_corr"  # k_helm_rhs<UNIFORM, LPT, CORR = true>
     if base in _KERNEL_TIMER:
         return _KERNEL_TIMER[base]
-    if base == "k_helm_fwd" and kernel.replace(" ", "").endswith(",true>"):
-        return "helm_fwd_corr"  # k_helm_fwd<UNIFORM, LPT, CORR = true>
     return base[2:] if base.startswith("k_") else base
 
 

@@ -83,7 +83,9 @@ void write_table(double *T, int nt, int n, std::vector<double> &dl, std::vector<
 }
 
 // Row-normalised matrix of the q_theta / q_z solves (mask variant ic, oc).
-void build_wall_table(const tc::Grid &g, int comp, int ic, int oc, double betadx, double *T, int nt) {
+// rows: the records of the right-hand sides, filled by the no-slip variant.
+void build_wall_table(const tc::Grid &g, int comp, int ic, int oc, double betadx, double *T, int nt,
+                      tc::RhsRow *rows) {
   const int n = g.nrm;
   const bool is_qt = (comp == tc::LU_QT);
   const std::vector<double> &ap = is_qt ? g.ap1j : g.ap3j;
@@ -116,10 +118,23 @@ void build_wall_table(const tc::Grid &g, int comp, int ic, int oc, double betadx
   for (int q = 0; q < n; q++) d[q] = ackl[q + 1];
   // right-hand side row scaling uses the unblended diagonal
   for (int kc = 1; kc <= n; kc++) sc[kc - 1] = 1.0 / (1. - ac[kc] * betadx);
+  if (ic == 1 && oc == 1) {
+    double tc::RhsRow::*const f[4] = {is_qt ? &tc::RhsRow::sc_t : &tc::RhsRow::sc_z,
+                                      is_qt ? &tc::RhsRow::am_t : &tc::RhsRow::am_z,
+                                      is_qt ? &tc::RhsRow::ap_t : &tc::RhsRow::ap_z,
+                                      is_qt ? &tc::RhsRow::x_t : &tc::RhsRow::x_z};
+    for (int kc = 1; kc <= n; kc++) {
+      rows[kc].*f[0] = sc[kc - 1];
+      rows[kc].*f[1] = kc > 1 ? amkl[kc] : 0.0;
+      rows[kc].*f[2] = kc < n ? apkl[kc] : 0.0;
+    }
+    rows[1].*f[3] = -ap[1] * betadx * (1.0 / (1.0 - ac_fs1 * betadx));
+    rows[n].*f[3] = -am[n] * betadx * (1.0 / (1.0 - ac_fs2 * betadx));
+  }
   write_table(T, nt, n, dl, d, du, sc);
 }
 
-void build_qr_table(const tc::Grid &g, double betadx, double *T, int nt) {
+void build_qr_table(const tc::Grid &g, double betadx, double *T, int nt, tc::RhsRow *rows) {
   const int n = g.nr, nrm = g.nrm;
   std::vector<double> amkl((size_t)n + 2), ackl((size_t)n + 2), apkl((size_t)n + 2);
   amkl[1] = 0.;
@@ -140,7 +155,12 @@ void build_qr_table(const tc::Grid &g, double betadx, double *T, int nt) {
     du[q] = apkl[q + 1];
   }
   for (int q = 0; q < n; q++) d[q] = ackl[q + 1];
-  for (int kc = 2; kc <= nrm; kc++) sc[kc - 1] = 1.0 / (1.0 - g.ac2j[kc] * betadx);
+  for (int kc = 2; kc <= nrm; kc++) {
+    sc[kc - 1] = 1.0 / (1.0 - g.ac2j[kc] * betadx);
+    rows[kc].sc_r = sc[kc - 1];
+    rows[kc].am_r = kc > 2 ? amkl[kc] : 0.0;
+    rows[kc].ap_r = kc < nrm ? apkl[kc] : 0.0;
+  }
   write_table(T, nt, n, dl, d, du, sc);
 }
 
@@ -154,17 +174,24 @@ int refresh_tables(tc_ctx *c) {
   if (!any) return 0;
   // the previous upload must have left the staging buffer
   HIPCHK(hipEventSynchronize(c->lu_copied));
-  const size_t per_slot = (size_t)3 * 4 * c->lu_nt;
+  const size_t per_slot = tc::lu_slot_doubles(c);
+  bool pivots = false;
   for (int s = 0; s < nsst; s++) {
     const double betadx = c->beta * c->g.alm[s + 1];
     double *base = c->lu_host + (size_t)s * per_slot;
+    tc::RhsRow *rows = reinterpret_cast<tc::RhsRow *>(base + (size_t)3 * 4 * c->lu_nt);
     for (int v = all_variants ? 0 : 3; v < 4; v++) {
       build_wall_table(c->g, tc::LU_QT, v & 1, v >> 1, betadx,
-                       base + ((size_t)tc::LU_QT * 4 + v) * c->lu_nt, c->lu_nt);
+                       base + ((size_t)tc::LU_QT * 4 + v) * c->lu_nt, c->lu_nt, rows);
       build_wall_table(c->g, tc::LU_QZ, v & 1, v >> 1, betadx,
-                       base + ((size_t)tc::LU_QZ * 4 + v) * c->lu_nt, c->lu_nt);
+                       base + ((size_t)tc::LU_QZ * 4 + v) * c->lu_nt, c->lu_nt, rows);
     }
-    build_qr_table(c->g, betadx, base + (size_t)tc::LU_QR * 4 * c->lu_nt, c->lu_nt);
+    build_qr_table(c->g, betadx, base + (size_t)tc::LU_QR * 4 * c->lu_nt, c->lu_nt, rows);
+    for (int t = 0; t < 12; t++) {
+      const bool used = t / 4 == tc::LU_QR ? t % 4 == 0 : (all_variants || t % 4 == 3);
+      for (int r = 0; used && r < c->nr; r++)
+        pivots = pivots || base[(size_t)t * c->lu_nt + tc::LU_ROW * r + 5] != 0.0;
+    }
     c->lu_key[s] = betadx;
   }
   HIPCHK(hipMemcpyAsync(c->lu, c->lu_host, sizeof(double) * per_slot * nsst, hipMemcpyHostToDevice,
@@ -172,6 +199,7 @@ int refresh_tables(tc_ctx *c) {
   HIPCHK(hipEventRecord(c->lu_copied, c->stream));
   c->lu_valid = true;
   c->lu_all_variants = all_variants;
+  c->lu_pivots = pivots;
   return 0;
 }
 
@@ -585,9 +613,10 @@ int tc_create_tuned(const tc_params *p, const tc_tuning *tun, tc_ctx **out) {
   // LU tables
   c->lu_nt = tc::LU_ROW * c->nr;
   {
-    const size_t n = (size_t)3 * 3 * 4 * c->lu_nt;
+    const size_t n = 3 * tc::lu_slot_doubles(c);
     TRY(dev_alloc(c, (void **)&c->lu, sizeof(double) * n));
     HTRY(hipHostMalloc((void **)&c->lu_host, sizeof(double) * n, hipHostMallocDefault));
+    std::fill(c->lu_host, c->lu_host + n, 0.0);
     HTRY(hipEventCreateWithFlags(&c->lu_copied, hipEventDisableTiming));
     HTRY(hipEventRecord(c->lu_copied, c->stream));
   }
@@ -620,7 +649,7 @@ int tc_create_tuned(const tc_params *p, const tc_tuning *tun, tc_ctx **out) {
     c->last_nute = std::nan("");
   }
   set_substep(c, 1);
-  c->helm_lpt = t.helm_lpt ? t.helm_lpt : tc::choose_helm_lpt(c);
+  tc::choose_helm_schedule(c, t.helm_lpt);
   c->poisson_pq = t.poisson_pq;
   {
     const char *dfs = std::getenv("TC_DIVFFT_STAGE");
@@ -640,7 +669,7 @@ int tc_set_tuning(tc_ctx *c, const tc_tuning *t) {
   const tc_tuning r = resolve_tuning(t, c->nrm);
   const std::string e = apply_plans(c, r);
   if (!e.empty()) return fail(e);
-  c->helm_lpt = r.helm_lpt ? r.helm_lpt : tc::choose_helm_lpt(c);
+  tc::choose_helm_schedule(c, r.helm_lpt);
   c->poisson_pq = r.poisson_pq;
   return tc::set_deferral(c, r.defer);
 }

@@ -61,7 +61,7 @@ using Key = std::tuple<int, int, int, int, int, int, int, int, int, int, int, in
 
 Key group_key(const tc_ctx *c) {
   return Key(c->nthm, c->nzm, c->nrm, c->p.nsst, c->helm_lpt, c->poisson_pq,
-             c->masks_uniform_one ? 1 : 0, c->plan_t.lines, c->plan_t.me, c->plan_t.padsh,
+             (c->masks_uniform_one ? 1 : 0) + (c->lu_pivots ? 2 : 0), c->plan_t.lines, c->plan_t.me, c->plan_t.padsh,
              c->plan_z.lines, c->plan_z.me * 1000 + c->plan_z.nt, c->plan_z.padsh,
              tc::defers_correction(c) ? 1 : 0);
 }
@@ -204,10 +204,10 @@ StepDesc make_desc(tc_ctx *c, int ns) {
   d.spec = c->spec;
   d.icyl = c->mask;
   d.ocyl = c->mask + c->P;
-  const size_t slot = (size_t)(ns - 1) * 3;
-  d.lut = c->lu + (slot + tc::LU_QT) * 4 * (size_t)c->lu_nt;
-  d.lur = c->lu + (slot + tc::LU_QR) * 4 * (size_t)c->lu_nt;
-  d.luz = c->lu + (slot + tc::LU_QZ) * 4 * (size_t)c->lu_nt;
+  d.lut = tc::lu_table(c, ns, tc::LU_QT);
+  d.lur = tc::lu_table(c, ns, tc::LU_QR);
+  d.luz = tc::lu_table(c, ns, tc::LU_QZ);
+  d.rows = tc::rhs_rows(c, ns);
   d.lu_nt = c->lu_nt;
   d.dt = dt;
   d.al = al;

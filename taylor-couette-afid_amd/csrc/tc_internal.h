@@ -63,6 +63,17 @@ struct FFTPlan {
 enum { LU_QT = 0, LU_QR = 1, LU_QZ = 2 };
 constexpr int LU_ROW = 8;
 
+// What the right-hand sides need of the Helmholtz matrices of plane k (row
+// k of each component), one record per plane and substep slot: the scaling
+// of the right-hand side and the off-diagonals of the row-normalised matrix
+// (unit diagonal).  x_t, x_z: the off-diagonal towards the interior of the
+// two wall rows where the wall is free-slip (k = 1: ap, k = nrm: am).
+// The q_r rows next to the walls do not couple to them (q_r is fixed there).
+struct RhsRow {
+  double sc_t, am_t, ap_t, sc_r, am_r, ap_r, sc_z, am_z, ap_z, x_t, x_z, pad;
+};
+static_assert(sizeof(RhsRow) == 96, "RhsRow is twelve doubles");
+
 struct Timer {
   std::string name;
   hipEvent_t a, b;
@@ -86,6 +97,7 @@ struct StepDesc {
   double2 *spec;
   const unsigned char *icyl, *ocyl;
   const double *lut, *lur, *luz;  // LU tables of this substep
+  const RhsRow *rows;           // [k], k = 1..nrm, of this substep
   int lu_nt;
   double dt, al, beta, usdt, inv_norm;
   FFTPlan pt, pz;
@@ -189,6 +201,7 @@ struct tc_ctx {
   double lu_key[3] = {-1, -1, -1};
   bool lu_valid = false;
   bool lu_all_variants = false;  // all four mask variants built (else only variant 3)
+  bool lu_pivots = false;        // some table exchanges rows (helm_solve needs the serial sweep)
   // FFT
   tc::FFTPlan plan_t, plan_z;
   double2 *tw_t = nullptr, *tw_z = nullptr;
@@ -212,6 +225,7 @@ struct tc_ctx {
   int divfft_stage = 1;  // fused divergence FFT: stage the divergence rows in LDS first
   int poisson_pq = 13;  // rows per thread of the radial Poisson solve (13 or 26)
   int helm_lpt = 1;  // radial lines per thread in the fused Helmholtz kernel (1 or 2)
+  int helm_slots[2] = {512, 512};  // its blocks resident on the device at once (plain, corrected)
   tc_tuning tuning{};  // effective tuning (helm_lpt 0 = chosen by occupancy)
   // statistics accumulators (TC_NSTATS x nrm x nzm) and per-line partials
   double *stats = nullptr, *stat_part = nullptr;
@@ -243,7 +257,7 @@ void launch_explicit_qr(tc_ctx *c);
 void launch_explicit_qz(tc_ctx *c);
 void launch_helmholtz_fused(tc_ctx *c);
 void launch_helmholtz_fused_corr(tc_ctx *c, const double *pr_in, double *pr_out, double al_prev);
-int choose_helm_lpt(const tc_ctx *c);
+void choose_helm_schedule(tc_ctx *c, int lpt);
 void launch_implicit_qt(tc_ctx *c);
 void launch_implicit_qr(tc_ctx *c);
 void launch_implicit_qz(tc_ctx *c);
@@ -276,6 +290,9 @@ bool defers_correction(const tc_ctx *c);
 int set_deferral(tc_ctx *c, int mode);
 // the dt and step recorded in a restart file's header (nothing else is read)
 int restart_file_info(const char *path, double *dt, int *ntime);
+size_t lu_slot_doubles(const tc_ctx *c);
+const double *lu_table(const tc_ctx *c, int ns, int comp);
+const RhsRow *rhs_rows(const tc_ctx *c, int ns);
 void launch_helmholtz_fused_g(tc_ctx *c, const StepDesc *tab, const BatchDyn *dyn, int ns, int n,
                               hipStream_t s, bool corr);
 void launch_correct_both_g(tc_ctx *c, const StepDesc *tab, int n, hipStream_t s);

@@ -20,6 +20,35 @@ DEVI long long IX(const GridDev &g, int k, int j, int i) {
 DEVI int wrap_p(int i, int n) { return (i + 1 == n) ? 0 : i + 1; }
 DEVI int wrap_m(int i, int n) { return (i == 0) ? n - 1 : i - 1; }
 
+// Workgroups are dispatched round-robin over the XCDs; hand each XCD a
+// contiguous run of tiles so neighbouring tiles share one L2.
+DEVI int xcd_tile(int b, int nb) {
+  constexpr int NX = 8;
+  const int q = nb / NX, r = nb - q * NX;
+  const int x = b % NX, local = b / NX;
+  return x * q + (x < r ? x : r) + local;
+}
+
+// A load from a table that no kernel writes while it is read.  In the
+// constant address space a load at a wave-uniform address is a scalar load
+// whatever else the kernel stores; through a plain pointer it is one only
+// where the compiler can rule out every store, and else a vector load whose
+// wait also drains the loads in flight.
+DEVI double ldk(const double *p) {
+  typedef __attribute__((address_space(4))) const double CT;
+  return *(CT *)(unsigned long long)p;
+}
+template <class T>
+DEVI T ldk_record(const T *p) {
+  constexpr int N = sizeof(T) / sizeof(double);
+  struct {
+    double v[N];
+  } a;
+#pragma unroll
+  for (int q = 0; q < N; q++) a.v[q] = ldk(reinterpret_cast<const double *>(p) + q);
+  return __builtin_bit_cast(T, a);
+}
+
 // Non-temporal access for arrays streamed once per kernel (no other block
 // re-reads them soon): a streaming copy runs 5.8% faster with both.
 DEVI double ld_nt(const double *p) { return __builtin_nontemporal_load(p); }
@@ -215,15 +244,9 @@ struct LUView {
   DEVI double du(int r) const { return b[LU_ROW * r + 1]; }
   DEVI double du2(int r) const { return b[LU_ROW * r + 2]; }
   DEVI double rd(int r) const { return b[LU_ROW * r + 3]; }
-  DEVI double sc(int r) const { return b[LU_ROW * r + 4]; }
   DEVI double pv(int r) const { return b[LU_ROW * r + 5]; }
-  DEVI double ud(int r) const { return b[LU_ROW * r + 6]; }
-  // row r of U q for q_r, q_(r+1), q_(r+2)
-  DEVI double uq(int r, double q0, double q1, double q2) const {
-    return ud(r) * q0 + du(r) * q1 + du2(r) * q2;
-  }
 };
-DEVI LUView lu_view(const double *base, int nt) {
+DEVI LUView lu_view(const double *base) {
   LUView v;
   v.b = base;
   return v;
@@ -301,219 +324,302 @@ DEVI double rhs_qz(const GridDev &g, const HelmPlane &c, const ImpArgs &a, int k
   return (a.ga * qcv + a.ro * hist + a.alre * d33 - dpx) * a.dt;
 }
 
-// ImplicitAndUpdateQT.F90:40-117 + SolveImpEqnUpdate_QT.F90:34-78
-__global__ __launch_bounds__(256) void k_implicit_qt(GridDev g, ImpArgs a, double *__restrict__ qt,
-                                                     const double *__restrict__ pr,
-                                                     const double *__restrict__ dq,
-                                                     double *__restrict__ ru1,
-                                                     double *__restrict__ y,
-                                                     const unsigned char *__restrict__ icyl,
-                                                     const unsigned char *__restrict__ ocyl,
-                                                     const double *__restrict__ lu, int nt) {
-  const long long l = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (l >= g.P) return;
-  const int j = (int)(l / g.nthm), i = (int)(l - (long long)j * g.nthm);
-  const long long lim = (long long)j * g.nthm + wrap_m(i, g.nthm);
-  const int n = g.nrm;
-  const int ic = icyl[l], oc = ocyl[l];
-  const double fic = (double)ic, foc = (double)oc;
-  const LUView T = lu_view(lu + (size_t)(ic + 2 * oc) * nt, nt);
-  const long long P = g.P;
-  double qm = 0.0, q0 = qt[l], qp = qt[l + P];
-  double carry = 0.0, yprev;
-  for (int k = 1; k <= n; k++) {
-    const long long o = (long long)(k - 1) * P + l;
-    if (k > 1) {
-      qm = q0;
-      q0 = qp;
-      qp = (k < n) ? qt[o + P] : 0.0;
-    }
-    const double dqv = dq[o];
-    const double r = rhs_qt(g, g.hp[k], a, k, qm, q0, qp, pr[o], pr[o - l + lim], dqv, ru1[o], fic, foc);
-    ru1[o] = dqv;
-    if (k == 1) {
-      carry = (r + a.bc1) * T.sc(0);
+// Routine-level right-hand sides, one point per thread: component WHICH of
+// ImplicitAndUpdateQT/QR/QZ (F90:40-117, :39-63, :36-115) with the history
+// update, scaled as SolveImpEqnUpdate_* scales its rows.
+template <int WHICH>
+__global__ __launch_bounds__(256) void k_implicit(GridDev g, ImpArgs a, const double *__restrict__ q,
+                                                  const double *__restrict__ pr,
+                                                  const double *__restrict__ expl,
+                                                  double *__restrict__ ru, double *__restrict__ y,
+                                                  const unsigned char *__restrict__ icyl,
+                                                  const unsigned char *__restrict__ ocyl,
+                                                  const RhsRow *__restrict__ rows) {
+  const int i = blockIdx.x * 64 + threadIdx.x;
+  const int j = blockIdx.y * 4 + threadIdx.y;
+  if (i >= g.nthm || j >= g.nzm) return;
+  const int k = blockIdx.z + (WHICH == 1 ? 2 : 1), n = g.nrm;
+  const long long l = (long long)j * g.nthm + i, o = (long long)(k - 1) * g.P + l;
+  const HelmPlane &hc = g.hp[k];
+  const RhsRow &t = rows[k];
+  const bool wr = WHICH == 1;  // q_r has both walls as planes
+  const double q0 = q[o], qm = (wr || k > 1) ? q[o - g.P] : 0.0, qp = (wr || k < n) ? q[o + g.P] : 0.0;
+  const double e = expl[o];
+  double r;
+  if (WHICH == 1) {
+    r = rhs_qr(hc, a, qm, q0, qp, pr[o], pr[o - g.P], e, ru[o]) * t.sc_r;
+  } else {
+    const double fic = (double)icyl[l], foc = (double)ocyl[l];
+    if (WHICH == 0) {
+      const double pim = pr[o - i + wrap_m(i, g.nthm)];
+      r = rhs_qt(g, hc, a, k, qm, q0, qp, pr[o], pim, e, ru[o], fic, foc);
+      if (k == 1) r = r + a.bc1;
+      r = r * t.sc_t;
     } else {
-      lsolve_step(T, k - 2, r * T.sc(k - 1), carry, yprev);
-      y[o - P] = yprev;
+      const double pjm = pr[o + (long long)(wrap_m(j, g.nzm) - j) * g.nthm];
+      r = rhs_qz(g, hc, a, k, qm, q0, qp, pr[o], pjm, e, ru[o], fic, foc) * t.sc_z;
     }
   }
-  y[(long long)(n - 1) * P + l] = carry;
+  ru[o] = e;
+  y[o] = r;
 }
 
-// ImplicitAndUpdateQR.F90:39-63 + the forward half of SolveImpEqnUpdate_QR:
-// nr rows with identity rows (zero right-hand side) at both walls.
-__global__ __launch_bounds__(256) void k_implicit_qr(GridDev g, ImpArgs a,
-                                                     const double *__restrict__ qr,
-                                                     const double *__restrict__ pr,
-                                                     const double *__restrict__ dph,
-                                                     double *__restrict__ ru2,
-                                                     double *__restrict__ y,
-                                                     const double *__restrict__ lu, int nt) {
-  const long long l = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (l >= g.P) return;
-  const int n = g.nr;
-  const LUView T = lu_view(lu, nt);
-  const long long P = g.P;
-  double qm, q0 = qr[l], qp = qr[l + P];
-  double carry = 0.0, yprev;  // row 0: zero right-hand side
-  for (int k = 2; k <= g.nrm; k++) {
-    const long long o = (long long)(k - 1) * P + l;
-    qm = q0;
-    q0 = qp;
-    qp = qr[o + P];
-    const double dv = dph[o];
-    const double r = rhs_qr(g.hp[k], a, qm, q0, qp, pr[o], pr[o - P], dv, ru2[o]);
-    ru2[o] = dv;
-    lsolve_step(T, k - 2, r * T.sc(k - 1), carry, yprev);
-    y[o - P] = yprev;
+// ---------------------------------------------------------------------------
+// Tridiagonal solves of the radial Helmholtz systems.  FOLD: the right-hand
+// sides are sc*rhs + A q, so the solution of A x' = sc*rhs + A q is
+// x' = q + x, the updated velocity itself, and q is not read (a few ulps of
+// q more rounding); otherwise q += x, as the reference adds it.
+//
+// Partitioned over the block: a block owns 64 lines (lanes along theta) and
+// each of its waves a segment of at most R rows of them, held in registers,
+// so a line's rows are loaded as one batch and its dependent chain is as
+// long as a segment instead of the line.  Without row exchanges the factors
+// are A = L U with y_r = g_r - dl_(r-1) y_(r-1) and x_r = (y_r - du_r x_(r+1))
+// rd_r.  Each wave sweeps its segment with a zero incoming value and leaves
+// the outgoing value and the product of its factors in LDS; the waves then
+// chain those (at most 15 terms) to their true incoming value, whose
+// contribution down the segment is the same recurrence on one number.  Twice:
+// downwards for L, upwards for U.  The factor products of a diagonally
+// dominant matrix stay below one, so this is as stable as the sweeps.
+//
+// The factors of a segment's rows are the same for all lanes (UNIFORM): the
+// lanes hold those of one row each and broadcast them by readlane.
+// ---------------------------------------------------------------------------
+DEVI double rlane(double v, int i) {
+  union {
+    double d;
+    int w[2];
+  } u, r;
+  u.d = v;
+  r.w[0] = __builtin_amdgcn_readlane(u.w[0], i);
+  r.w[1] = __builtin_amdgcn_readlane(u.w[1], i);
+  return r.d;
+}
+
+// comp: 0 q_theta, 1 q_r (rows 2..nrm; both walls are set to zero), 2 q_z
+template <int R, bool UNIFORM, bool FOLD>
+DEVI void helm_solve_body(const long long lgrp, const int comp, const GridDev &g,
+                          double *__restrict__ q, const double *__restrict__ y,
+                          const unsigned char *__restrict__ icyl,
+                          const unsigned char *__restrict__ ocyl, const double *__restrict__ lu,
+                          int nt, double *ex) {
+  const int lane = threadIdx.x, NS = blockDim.y;
+  const int p = __builtin_amdgcn_readfirstlane(threadIdx.y);
+  const long long P = g.P, l = lgrp * 64 + lane;
+  const bool ok = l < P;
+  const long long lc = ok ? l : P - 1;
+  const int first = comp == 1 ? 1 : 0, n = g.nrm - first, last = first + n - 1;
+  const int lo = first + p * n / NS, S = first + (p + 1) * n / NS - lo;
+  double v[R];
+  {
+    const double *yp = y + (long long)lo * P + lc;
+#pragma unroll
+    for (int i = 0; i < R; i++) v[i] = ld_nt(yp + (long long)min(i, S - 1) * P);
   }
-  lsolve_step(T, n - 2, 0.0, carry, yprev);  // row nr: zero right-hand side
-  y[(long long)(n - 2) * P + l] = yprev;
-  y[(long long)(n - 1) * P + l] = carry;
-}
-
-// ImplicitAndUpdateQZ.F90:36-115 + SolveImpEqnUpdate_QZ.F90:32-68.
-__global__ __launch_bounds__(256) void k_implicit_qz(GridDev g, ImpArgs a,
-                                                     const double *__restrict__ qz,
-                                                     const double *__restrict__ pr,
-                                                     const double *__restrict__ qcap,
-                                                     double *__restrict__ ru3,
-                                                     double *__restrict__ y,
-                                                     const unsigned char *__restrict__ icyl,
-                                                     const unsigned char *__restrict__ ocyl,
-                                                     const double *__restrict__ lu, int nt) {
-  const long long l = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (l >= g.P) return;
-  const int j = (int)(l / g.nthm), i = (int)(l - (long long)j * g.nthm);
-  const long long ljm = (long long)wrap_m(j, g.nzm) * g.nthm + i;
-  const int n = g.nrm;
-  const int ic = icyl[l], oc = ocyl[l];
-  const double fic = (double)ic, foc = (double)oc;
-  const LUView T = lu_view(lu + (size_t)(ic + 2 * oc) * nt, nt);
-  const long long P = g.P;
-  double qm = 0.0, q0 = qz[l], qp = qz[l + P];
-  double carry = 0.0, yprev;
-  for (int k = 1; k <= n; k++) {
-    const long long o = (long long)(k - 1) * P + l;
-    if (k > 1) {
-      qm = q0;
-      q0 = qp;
-      qp = (k < n) ? qz[o + P] : 0.0;
-    }
-    const double qv = qcap[o];
-    const double r = rhs_qz(g, g.hp[k], a, k, qm, q0, qp, pr[o], pr[o - l + ljm], qv, ru3[o], fic, foc);
-    ru3[o] = qv;
-    if (k == 1) {
-      carry = r * T.sc(0);
-    } else {
-      lsolve_step(T, k - 2, r * T.sc(k - 1), carry, yprev);
-      y[o - P] = yprev;
+  const int var = comp == 1 ? 0 : (UNIFORM ? 3 : icyl[lc] + 2 * ocyl[lc]);
+  const LUView T = lu_view(lu + (size_t)var * nt);
+  // -dl_(r-1), rd_r and -du_r rd_r of row lo + i (UNIFORM: of rows lo + lane
+  // and, past 64 rows, lo + 64 + lane)
+  constexpr int NK = (R + 63) / 64;
+  double kdl[NK], kdu[NK], krd[NK];
+  if constexpr (UNIFORM) {
+#pragma unroll
+    for (int u = 0; u < NK; u++) {
+      const int r = lo + min(lane + 64 * u, S - 1);
+      kdl[u] = r > first ? -T.dl(r - 1) : 0.0;
+      krd[u] = T.rd(r);
+      kdu[u] = r < last ? -T.du(r) * krd[u] : 0.0;
     }
   }
-  y[(long long)(n - 1) * P + l] = carry;
+  auto dl = [&](int i) {
+    if constexpr (UNIFORM) return rlane(kdl[i >> 6], i & 63);
+    else return lo + i > first ? -T.dl(lo + i - 1) : 0.0;
+  };
+  auto rd = [&](int i) {
+    if constexpr (UNIFORM) return rlane(krd[i >> 6], i & 63);
+    else return T.rd(lo + i);
+  };
+  auto ud = [&](int i) {
+    if constexpr (UNIFORM) return rlane(kdu[i >> 6], i & 63);
+    else return lo + i < last ? -T.du(lo + i) * T.rd(lo + i) : 0.0;
+  };
+  double *exc = ex, *exw = ex + NS * 64;  // outgoing values and factors
+  double c = 0.0, w = 1.0;
+#pragma unroll
+  for (int i = 0; i < R; i++)
+    if (i < S) {
+      const double d = dl(i);
+      c = v[i] + d * c;
+      v[i] = c;
+      w = w * d;
+    }
+  exc[p * 64 + lane] = c;
+  exw[p * 64 + lane] = w;
+  __syncthreads();
+  w = 0.0;
+  for (int s = 0; s < p; s++) w = exc[s * 64 + lane] + exw[s * 64 + lane] * w;
+#pragma unroll
+  for (int i = 0; i < R; i++)
+    if (i < S) {
+      w = w * dl(i);
+      v[i] = v[i] + w;
+    }
+  exc += 2 * NS * 64;
+  exw += 2 * NS * 64;
+  c = 0.0;
+  w = 1.0;
+#pragma unroll
+  for (int i = R - 1; i >= 0; i--)
+    if (i < S) {
+      const double u = ud(i);
+      c = v[i] * rd(i) + u * c;
+      v[i] = c;
+      w = w * u;
+    }
+  exc[p * 64 + lane] = c;
+  exw[p * 64 + lane] = w;
+  __syncthreads();
+  w = 0.0;
+  for (int s = NS - 1; s > p; s--) w = exc[s * 64 + lane] + exw[s * 64 + lane] * w;
+  if (!ok) return;
+  double *qp = q + (long long)lo * P + l;
+#pragma unroll
+  for (int i = R - 1; i >= 0; i--)
+    if (i < S) {
+      w = w * ud(i);
+      double *o = qp + (long long)i * P;
+      st_nt(o, FOLD ? v[i] + w : *o + (v[i] + w));
+    }
+  if (comp == 1) {  // ImplicitAndUpdateQR.F90:70-71
+    if (p == 0) q[l] = 0.0;
+    if (p == NS - 1) q[(long long)(g.nr - 1) * P + l] = 0.0;
+  }
 }
 
-// Backward substitution (dgtts2) of one line: q += x, rows first..n-1 (the
-// q_r wall rows are reset instead).  Loads are issued a chunk of rows ahead
+struct SolveIO {
+  double *q[3];
+  const double *y[3];
+  const double *lu[3];
+};
+
+// The components of a line group are consecutive, and the groups contiguous
+// per XCD: the six arrays then move together (1024x1024x769: 7.8 ms against
+// 8.2 with one component after the other, 512x512x385: 885 against 960 us).
+template <int R, bool UNIFORM, bool FOLD>
+__global__ __launch_bounds__(R > 32 ? 512 : 1024) void k_helm_solve(
+    GridDev g, SolveIO io, const unsigned char *__restrict__ icyl,
+    const unsigned char *__restrict__ ocyl, int nt, int comp0) {
+  extern __shared__ double ex[];
+  const int lin = xcd_tile(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+  const int comp = lin % (int)gridDim.y + comp0;
+  helm_solve_body<R, UNIFORM, FOLD>(lin / (int)gridDim.y, comp, g,
+                              comp == 0 ? io.q[0] : (comp == 1 ? io.q[1] : io.q[2]),
+                              comp == 0 ? io.y[0] : (comp == 1 ? io.y[1] : io.y[2]), icyl, ocyl,
+                              comp == 0 ? io.lu[0] : (comp == 1 ? io.lu[1] : io.lu[2]), nt, ex);
+}
+
+// Grouped: blockIdx.z = instance; right-hand sides in rhs, dq, qcap.
+template <int R, bool UNIFORM>
+__global__ __launch_bounds__(R > 32 ? 512 : 1024) void k_helm_solve_g(
+    const StepDesc *__restrict__ tab) {
+  extern __shared__ double ex[];
+  const StepDesc &d = tab[blockIdx.z];
+  if (inst_stopped(d)) return;
+  const int lin = xcd_tile(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * 3);
+  const int comp = lin % 3;
+  helm_solve_body<R, UNIFORM, true>(
+      lin / 3, comp, glob(d.g),
+      glob(d.f[comp == 0 ? TC_QT : (comp == 1 ? TC_QR : TC_QZ)]),
+      glob(d.f[comp == 0 ? TC_RHS : (comp == 1 ? TC_DQ : TC_QCAP)]), glob(d.icyl), glob(d.ocyl),
+      glob(comp == 0 ? d.lut : (comp == 1 ? d.lur : d.luz)), d.lu_nt, ex);
+}
+
+// Serial form, one line per lane: dgttrs as it is, for factors with row
+// exchanges and for lines longer than the partitioned form holds.  y is
+// overwritten by the forward sweep.  Loads are issued a chunk of rows ahead
 // of the dependent recurrence.
-// FOLD: y already holds U q + y (the forward sweep added it), so the
-// solution of U x' = y' is x' = q + x itself and q is not read.
-template <bool FOLD>
-DEVI void usolve_line(const LUView &T, int n, int first, double *__restrict__ q,
-                      const double *__restrict__ y, long long l, long long P) {
+DEVI void helm_solve_serial_body(const long long l, const int comp, const GridDev &g,
+                                 double *__restrict__ q, double *__restrict__ y,
+                                 const unsigned char *__restrict__ icyl,
+                                 const unsigned char *__restrict__ ocyl,
+                                 const double *__restrict__ lu, int nt, bool fold) {
   constexpr int CH = 16;
-  auto put = [&](long long o, double qv, double x) { st_nt(q + o, FOLD ? x : qv + x); };
-  double x1 = y[(long long)(n - 1) * P + l] * T.rd(n - 1);
-  if (n - 1 >= first) {
-    const long long o = (long long)(n - 1) * P + l;
-    put(o, FOLD ? 0.0 : q[o], x1);
-  }
-  double x0 = (y[(long long)(n - 2) * P + l] - T.du(n - 2) * x1) * T.rd(n - 2);
-  if (n - 2 >= first) {
-    const long long o = (long long)(n - 2) * P + l;
-    put(o, FOLD ? 0.0 : q[o], x0);
-  }
-  for (int r0 = n - 3; r0 >= first; r0 -= CH) {
-    double yv[CH], qv[CH];
+  if (l >= g.P) return;
+  const long long P = g.P;
+  const int var = comp == 1 ? 0 : icyl[l] + 2 * ocyl[l];
+  const LUView T = lu_view(lu + (size_t)var * nt);
+  const int first = comp == 1 ? 1 : 0, last = g.nrm - 1;
+  double carry = y[(long long)first * P + l], out;
+  for (int r0 = first + 1; r0 <= last; r0 += CH) {
+    double f[CH];
+#pragma unroll
+    for (int u = 0; u < CH; u++)
+      if (r0 + u <= last) f[u] = y[(long long)(r0 + u) * P + l];
 #pragma unroll
     for (int u = 0; u < CH; u++) {
-      const int r = r0 - u;
-      if (r >= first) {
-        const long long o = (long long)r * P + l;
-        yv[u] = ld_nt(y + o);
-        qv[u] = FOLD ? 0.0 : q[o];
+      const int r = r0 + u;
+      if (r <= last) {
+        lsolve_step(T, r - 1, f[u], carry, out);
+        y[(long long)(r - 1) * P + l] = out;
       }
     }
+  }
+  // q_r: x' is zero at both walls, so row nrm couples to nothing above it
+  double x1 = 0.0, x0 = carry * T.rd(last);
+  auto put = [&](int r, double x) {
+    double *o = q + (long long)r * P + l;
+    *o = fold ? x : *o + x;
+  };
+  put(last, x0);
+  for (int r0 = last - 1; r0 >= first; r0 -= CH) {
+    double f[CH];
+#pragma unroll
+    for (int u = 0; u < CH; u++)
+      if (r0 - u >= first) f[u] = y[(long long)(r0 - u) * P + l];
 #pragma unroll
     for (int u = 0; u < CH; u++) {
       const int r = r0 - u;
       if (r >= first) {
-        const double x = (yv[u] - T.du(r) * x0 - T.du2(r) * x1) * T.rd(r);
-        put((long long)r * P + l, qv[u], x);
+        const double x = (f[u] - T.du(r) * x0 - T.du2(r) * x1) * T.rd(r);
+        put(r, x);
         x1 = x0;
         x0 = x;
       }
     }
   }
+  if (comp == 1) q[l] = q[(long long)(g.nr - 1) * P + l] = 0.0;
 }
 
-// which: bit 0 q_theta, bit 1 q_r, bit 2 q_z
-template <bool FOLD>
-DEVI void helm_bwd_body(const long long l, const GridDev &g, double *__restrict__ qt,
-                        double *__restrict__ qr, double *__restrict__ qz,
-                        const double *__restrict__ yt, const double *__restrict__ yr,
-                        const double *__restrict__ yz, const unsigned char *__restrict__ icyl,
-                        const unsigned char *__restrict__ ocyl, const double *__restrict__ lut,
-                        const double *__restrict__ lur, const double *__restrict__ luz, int nt,
-                        int which) {
-  if (l >= g.P) return;
-  const int v = icyl[l] + 2 * ocyl[l];
-  if (which & 1) usolve_line<FOLD>(lu_view(lut + (size_t)v * nt, nt), g.nrm, 0, qt, yt, l, g.P);
-  if (which & 2) {
-    // SolveImpEqnUpdate_QR.F90:63-65 adds rows 2..nrm; walls reset
-    // (ImplicitAndUpdateQR.F90:70-71)
-    usolve_line<FOLD>(lu_view(lur, nt), g.nr, 1, qr, yr, l, g.P);
-    qr[l] = 0.0;
-    qr[(long long)(g.nr - 1) * g.P + l] = 0.0;
-  }
-  if (which & 4) usolve_line<FOLD>(lu_view(luz + (size_t)v * nt, nt), g.nrm, 0, qz, yz, l, g.P);
+__global__ __launch_bounds__(256) void k_helm_solve_serial(GridDev g, SolveIO io,
+                                                           const unsigned char *__restrict__ icyl,
+                                                           const unsigned char *__restrict__ ocyl,
+                                                           int nt, int comp0, bool fold) {
+  const int comp = blockIdx.y + comp0;
+  helm_solve_serial_body((long long)blockIdx.x * 256 + threadIdx.x, comp, g,
+                         comp == 0 ? io.q[0] : (comp == 1 ? io.q[1] : io.q[2]),
+                         const_cast<double *>(comp == 0 ? io.y[0] : (comp == 1 ? io.y[1] : io.y[2])),
+                         icyl, ocyl, comp == 0 ? io.lu[0] : (comp == 1 ? io.lu[1] : io.lu[2]), nt, fold);
 }
 
-template <bool FOLD>
-__global__ __launch_bounds__(256) void k_helm_bwd(GridDev g, double *__restrict__ qt,
-                                                  double *__restrict__ qr,
-                                                  double *__restrict__ qz,
-                                                  const double *__restrict__ yt,
-                                                  const double *__restrict__ yr,
-                                                  const double *__restrict__ yz,
-                                                  const unsigned char *__restrict__ icyl,
-                                                  const unsigned char *__restrict__ ocyl,
-                                                  const double *__restrict__ lut,
-                                                  const double *__restrict__ lur,
-                                                  const double *__restrict__ luz, int nt,
-                                                  int which) {
-  helm_bwd_body<FOLD>((long long)blockIdx.x * blockDim.x + threadIdx.x, g, qt, qr, qz, yt, yr, yz,
-                      icyl, ocyl, lut, lur, luz, nt, which);
-}
-
-// Grouped fused backward sweep: blockIdx.y = instance; y' = rhs, dq, qcap.
-__global__ __launch_bounds__(256) void k_helm_bwd_g(const StepDesc *__restrict__ tab) {
-  const StepDesc &d = tab[blockIdx.y];
+__global__ __launch_bounds__(256) void k_helm_solve_serial_g(const StepDesc *__restrict__ tab) {
+  const StepDesc &d = tab[blockIdx.z];
   if (inst_stopped(d)) return;
-  helm_bwd_body<true>((long long)blockIdx.x * blockDim.x + threadIdx.x, glob(d.g),
-                      glob(d.f[TC_QT]), glob(d.f[TC_QR]), glob(d.f[TC_QZ]), glob(d.f[TC_RHS]),
-                      glob(d.f[TC_DQ]), glob(d.f[TC_QCAP]), glob(d.icyl), glob(d.ocyl),
-                      glob(d.lut), glob(d.lur), glob(d.luz), d.lu_nt, 7);
+  const int comp = blockIdx.y;
+  helm_solve_serial_body((long long)blockIdx.x * 256 + threadIdx.x, comp, glob(d.g),
+                         glob(d.f[comp == 0 ? TC_QT : (comp == 1 ? TC_QR : TC_QZ)]),
+                         glob(d.f[comp == 0 ? TC_RHS : (comp == 1 ? TC_DQ : TC_QCAP)]),
+                         glob(d.icyl), glob(d.ocyl),
+                         glob(comp == 0 ? d.lut : (comp == 1 ? d.lur : d.luz)), d.lu_nt, true);
 }
 
 // ---------------------------------------------------------------------------
-// Fused substep front: explicit terms + right-hand sides + forward
-// substitution of all three components in one march along r.  A block owns
-// a 64 (theta) x 4 (z) tile of radial lines; the planes k-1, k, k+1 of
-// qt, qr, qz (with a one-point periodic halo) rotate through an LDS ring and
-// plane k+2 is fetched into registers while plane k is computed.  The
-// explicit terms never reach HBM.
+// Fused substep front: explicit terms and right-hand sides of all three
+// components.  A block owns a 64 (theta) x 4*LPT (z) tile of radial lines
+// over a segment of r planes; the planes k-1, k, k+1 of qt, qr, qz (with a
+// one-point periodic halo) rotate through an LDS ring and plane k+2 is
+// fetched into registers while plane k is computed.  The explicit terms
+// never reach HBM.  Every value is local to its point, so the segments and
+// tiles of a launch do not change the results.
 // ---------------------------------------------------------------------------
 // One point of CorrectVelocity.F90:32-40 and CorrectPressure.F90:37-46
 // (amm = apph), without FMA contraction: the pair kernel and the Helmholtz
@@ -521,11 +627,11 @@ __global__ __launch_bounds__(256) void k_helm_bwd_g(const StepDesc *__restrict__
 // dm: the dph neighbour at i-1 (qt), k-1 (qr), j-1 (qz).
 DEVI double corr_qt(const GridDev &g, int kc, double t, double d, double dm, double dt, double al) {
 #pragma clang fp contract(off)
-  return t - (d - dm) * dt * al * g.dxt * g.usrm[kc];
+  return t - (d - dm) * dt * al * g.dxt * ldk(g.usrm + kc);
 }
 DEVI double corr_qr(const GridDev &g, int kc, double r, double d, double dm, double dt, double al) {
 #pragma clang fp contract(off)
-  return r - (d - dm) * dt * al * g.rudx2c[kc];
+  return r - (d - dm) * dt * al * ldk(g.rudx2c + kc);
 }
 DEVI double corr_qz(const GridDev &g, double z, double d, double dm, double dt, double al) {
 #pragma clang fp contract(off)
@@ -534,13 +640,13 @@ DEVI double corr_qz(const GridDev &g, double z, double d, double dm, double dt, 
 DEVI double corr_pr(const GridDev &g, int kc, double p, double d, double dim, double dip, double djm,
                     double djp, double dkm, double dkp, double be) {
 #pragma clang fp contract(off)
-  const double amm = g.apph[kc], acc = g.acph[kc], app = g.apph[kc];
+  const double amm = ldk(g.apph + kc), acc = ldk(g.acph + kc), app = amm;
   return p + d -
-         be * ((dip - 2.0 * d + dim) * g.udx1qm[kc] + (djp - 2.0 * d + djm) * g.dxzq +
+         be * ((dip - 2.0 * d + dim) * ldk(g.udx1qm + kc) + (djp - 2.0 * d + djm) * g.dxzq +
                (dkp * app + d * acc + dkm * amm));
 }
 
-constexpr int FT_I = 64, FT_W = FT_I + 2;
+constexpr int FT_N = 256, FT_I = 64, FT_J = FT_N / FT_I, FT_W = FT_I + 2;
 
 // A pressure correction still to be applied: the Helmholtz kernel of the
 // next substep applies it to every plane it stages (velocity and pressure)
@@ -572,66 +678,55 @@ struct LAcc {
   }
 };
 
-// Workgroups are dispatched round-robin over the XCDs; hand each XCD a
-// contiguous run of tiles so neighbouring tiles share one L2.
-DEVI int xcd_tile(int b, int nb) {
-  constexpr int NX = 8;
-  const int q = nb / NX, r = nb - q * NX;
-  const int x = b % NX, local = b / NX;
-  return x * q + (x < r ? x : r) + local;
-}
-
-// A block of 256 threads owns a 64 (theta) x 4*LPT (z) tile of radial lines,
-// LPT lines per thread (rows ty and ty+4).  UNIFORM: every wall mask is 1
-// (no-slip everywhere, the SlipBCs default), so all lines share one table
-// entry and the table pointers stay scalar.
+// A block of 256 threads owns a 64 (theta) x 4*LPT (z) tile of radial lines
+// from plane k0 to plane k1, LPT lines per thread (rows ty and ty+4).
+// UNIFORM: every wall mask is 1 (no-slip everywhere, the SlipBCs default).
 // CORR: qt, qr, qz hold the previous substep's velocity before its pressure
 // correction and pr its pressure before the correction; the correction
 // (dph of that substep) is applied to each plane as it is staged, from a
 // ring of dph planes with a two-point theta/z halo, so the corrected fields
 // are the ones the per-substep path would have stored, bit for bit.
 template <bool UNIFORM, int LPT, bool CORR>
-DEVI void helm_fwd_body(
-    const int tile, const GridDev &g, const ImpArgs &a, const double *__restrict__ qt,
-    const double *__restrict__ qr, const double *__restrict__ qz, const double *__restrict__ pr,
-    double *__restrict__ ru1, double *__restrict__ ru2, double *__restrict__ ru3,
-    double *__restrict__ yt, double *__restrict__ yr, double *__restrict__ yz,
-    const unsigned char *__restrict__ icyl, const unsigned char *__restrict__ ocyl,
-    const double *__restrict__ lut, const double *__restrict__ lur,
-    const double *__restrict__ luz, int nt, int ntx, const CorrIn &ci,
-    const double *__restrict__ dph, double *__restrict__ pr_out) {
-  constexpr int TJ = 4 * LPT, H = TJ + 2, S = FT_W * H, NE = (S + 255) / 256;
-  constexpr int W2 = FT_I + 4, S2 = W2 * (TJ + 4), NE2 = (S2 + 255) / 256;
+DEVI void helm_rhs_body(
+    const int tile, const int k0, const int k1, const GridDev &g, const ImpArgs &a,
+    const double *__restrict__ qt, const double *__restrict__ qr, const double *__restrict__ qz,
+    const double *__restrict__ pr, double *__restrict__ ru1, double *__restrict__ ru2,
+    double *__restrict__ ru3, double *__restrict__ yt, double *__restrict__ yr,
+    double *__restrict__ yz, const unsigned char *__restrict__ icyl,
+    const unsigned char *__restrict__ ocyl, const RhsRow *__restrict__ rows, int ntx,
+    const CorrIn &ci, const double *__restrict__ dph, double *__restrict__ pr_out) {
+  constexpr int TJ = FT_J * LPT, H = TJ + 2, S = FT_W * H, NE = (S + FT_N - 1) / FT_N;
+  constexpr int W2 = FT_I + 4, S2 = W2 * (TJ + 4), NE2 = (S2 + FT_N - 1) / FT_N;
   __shared__ double sq[3][3][S];  // field, ring slot, tile
   __shared__ double sp[2][S];     // pressure planes k and k+1
   __shared__ double sd[CORR ? 3 : 1][CORR ? S2 : 1];  // dph planes (slot = plane % 3)
   const int i0 = (tile % ntx) * FT_I, j0 = (tile / ntx) * TJ;
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+  const int tx = threadIdx.x % FT_I, ty = threadIdx.x / FT_I;
   const long long P = g.P;
   // the tile elements this thread stages per plane: chunks 0..NE-2 are
   // full; in the last one threads past S load a valid element and do not
   // store it, so every global load is unconditional
-  long long off[NE];
-  const bool has_last = threadIdx.x + (NE - 1) * 256 < S;
+  int off[NE];
+  const bool has_last = threadIdx.x + (NE - 1) * FT_N < S;
 #pragma unroll
   for (int q = 0; q < NE; q++) {
-    const int e = threadIdx.x + q * 256;
+    const int e = threadIdx.x + q * FT_N;
     const int ee = e < S ? e : 0;
     int jj = j0 + ee / FT_W - 1, ii = i0 + ee % FT_W - 1;
     jj = ((jj % g.nzm) + g.nzm) % g.nzm;
     ii = ((ii % g.nthm) + g.nthm) % g.nthm;
-    off[q] = (long long)jj * g.nthm + ii;
+    off[q] = jj * g.nthm + ii;
   }
   // CORR: the dph tile elements (two-point halo) this thread stages, and
   // whether each of its velocity tile elements is an interior point whose
   // corrected pressure it writes
   int off2[CORR ? NE2 : 1];
   bool wpr[NE];
-  const bool has_last2 = threadIdx.x + (NE2 - 1) * 256 < S2;
+  const bool has_last2 = threadIdx.x + (NE2 - 1) * FT_N < S2;
   if constexpr (CORR) {
 #pragma unroll
     for (int q = 0; q < NE2; q++) {
-      const int e = threadIdx.x + q * 256;
+      const int e = threadIdx.x + q * FT_N;
       const int ee = e < S2 ? e : 0;
       int jj = j0 + ee / W2 - 2, ii = i0 + ee % W2 - 2;
       jj = ((jj % g.nzm) + g.nzm) % g.nzm;
@@ -640,7 +735,7 @@ DEVI void helm_fwd_body(
     }
 #pragma unroll
     for (int q = 0; q < NE; q++) {
-      const int e = threadIdx.x + q * 256;
+      const int e = threadIdx.x + q * FT_N;
       const int row = e / FT_W, col = e % FT_W;
       wpr[q] = (e < S) && row >= 1 && row <= TJ && col >= 1 && col <= FT_I &&
                j0 + row - 1 < g.nzm && i0 + col - 1 < g.nthm;
@@ -671,91 +766,129 @@ DEVI void helm_fwd_body(
     return corr_pr(g, p, v, dc[e2], dc[e2 - 1], dc[e2 + 1], dc[e2 - W2], dc[e2 + W2], dkm[e2],
                    dkp[e2], ci.be);
   };
+  // stage dph plane p (clamped to 1..nrm: beyond it no correction reads dph)
+  auto stage_dph = [&](int p) {
+    const long long od = (long long)(min(max(p, 1), g.nrm) - 1) * P;
+    double t[CORR ? NE2 : 1];
+#pragma unroll
+    for (int q = 0; q < NE2; q++) t[q] = dph[od + off2[q]];
+#pragma unroll
+    for (int q = 0; q < NE2; q++)
+      if (q < NE2 - 1 || has_last2) sd[(p + 3) % 3][threadIdx.x + q * FT_N] = t[q];
+  };
+  // stage plane p of the velocity (before the first iteration)
+  auto stage_q = [&](int p) {
+    const long long oq = (long long)(p - 1) * P;
+    double t[3][NE];
+#pragma unroll
+    for (int q = 0; q < NE; q++) {
+      t[0][q] = qt[oq + off[q]];
+      t[1][q] = qr[oq + off[q]];
+      t[2][q] = qz[oq + off[q]];
+    }
+#pragma unroll
+    for (int q = 0; q < NE; q++)
+      if (q < NE - 1 || has_last) {
+        const int e = threadIdx.x + q * FT_N;
+        if constexpr (CORR) corr_q(p, e, t[0][q], t[1][q], t[2][q]);
+        sq[0][p % 3][e] = t[0][q];
+        sq[1][p % 3][e] = t[1][q];
+        sq[2][p % 3][e] = t[2][q];
+      }
+  };
   // the RK history ru enters as ro*ru only: with ro = 0 (the first RK3
   // substep) it is not read at all
   const bool hist = CORR || a.ro != 0.0;
+  const int nrm = g.nrm;
   // per-line state
   bool valid[LPT];
   long long l[LPT];
   int base[LPT];
-  double fic[LPT], foc[LPT], h1[LPT], h2[LPT], h3[LPT], ct[LPT], cr[LPT], cz[LPT], pr_km[LPT];
+  double fic[LPT], foc[LPT], h1[LPT], h2[LPT], h3[LPT], pr_km[LPT];
   // !CORR: plane k-1 values carried from the previous iteration (qt centre,
   // qt theta+1, qr centre, qz centre, qz z+1), so that no thread reads the
   // ring slot of plane k-1 and the staging of plane k+2 into it needs no
   // barrier of its own
   double cm[LPT][5];
-  LUView Tt[LPT], Tz[LPT];
-  const LUView Tr = lu_view(lur, nt);
 #pragma unroll
   for (int u = 0; u < LPT; u++) {
-    const int row = ty + 4 * u;
+    const int row = ty + FT_J * u;
     const int i = i0 + tx, j = j0 + row;
     valid[u] = (i < g.nthm) && (j < g.nzm);
     l[u] = valid[u] ? (long long)j * g.nthm + i : 0;
     base[u] = (row + 1) * FT_W + tx + 1;
-    const int ic = (UNIFORM || !valid[u]) ? 1 : icyl[l[u]];
-    const int oc = (UNIFORM || !valid[u]) ? 1 : ocyl[l[u]];
-    fic[u] = (double)ic;
-    foc[u] = (double)oc;
-    const int v = UNIFORM ? 3 : ic + 2 * oc;
-    Tt[u] = lu_view(lut + (size_t)v * nt, nt);
-    Tz[u] = lu_view(luz + (size_t)v * nt, nt);
-    h1[u] = (valid[u] && hist) ? ld_nt(ru1 + l[u]) : 0.0;
-    h2[u] = 0.0;
-    h3[u] = (valid[u] && hist) ? ld_nt(ru3 + l[u]) : 0.0;
-    ct[u] = cr[u] = cz[u] = pr_km[u] = 0.0;
+    fic[u] = (UNIFORM || !valid[u]) ? 1.0 : (double)icyl[l[u]];
+    foc[u] = (UNIFORM || !valid[u]) ? 1.0 : (double)ocyl[l[u]];
+    const long long o = (long long)(k0 - 1) * P + l[u];
+    h1[u] = hist ? ld_nt(ru1 + o) : 0.0;
+    h2[u] = hist ? ld_nt(ru2 + o) : 0.0;
+    h3[u] = hist ? ld_nt(ru3 + o) : 0.0;
+    pr_km[u] = k0 > 1 ? pr[o - P] : 0.0;
 #pragma unroll
     for (int q = 0; q < 5; q++) cm[u][q] = 0.0;
   }
-  // planes 1 and 2 of the velocity, plane 1 of the pressure (CORR: planes 1
-  // and 2 of dph first, then the corrected values)
+  // planes k0-1 (if any), k0 and k0+1 of the velocity, k0 of the pressure
+  // and the pressure of k0-1 on the lines themselves.  CORR: with the dph
+  // planes that each of these corrections reads staged before it.
   if constexpr (CORR) {
-    const long long o2 = (g.nrm > 1) ? P : 0;
+    if (k0 > 1) {
+      stage_dph(k0 - 2);
+      stage_dph(k0 - 1);
+      stage_dph(k0);
+      __syncthreads();
+      stage_q(k0 - 1);
 #pragma unroll
-    for (int q = 0; q < NE2; q++) {
-      const double a1 = dph[off2[q]], a2 = dph[o2 + off2[q]];
-      if (q < NE2 - 1 || has_last2) {
-        const int e = threadIdx.x + q * 256;
-        sd[1][e] = a1;
-        sd[2][e] = a2;
-      }
+      for (int u = 0; u < LPT; u++) pr_km[u] = corr_p(k0 - 1, base[u], pr_km[u]);
+      __syncthreads();
+      stage_dph(k0 + 1);
+    } else {
+      stage_dph(1);
+      stage_dph(2);
     }
     __syncthreads();
+  } else if (k0 > 1) {
+    stage_q(k0 - 1);
   }
+  stage_q(k0);
+  stage_q(k0 + 1);
+  {
+    const long long op = (long long)(k0 - 1) * P;
 #pragma unroll
-  for (int q = 0; q < NE; q++) {
-    double v0 = qt[off[q]], v1 = qr[off[q]], v2 = qz[off[q]];
-    double w0 = qt[P + off[q]], w1 = qr[P + off[q]], w2 = qz[P + off[q]];
-    double v3 = pr[off[q]];
-    if (q < NE - 1 || has_last) {
-      if constexpr (CORR) {
-        const int e = threadIdx.x + q * 256;
-        corr_q(1, e, v0, v1, v2);
-        corr_q(2, e, w0, w1, w2);
-        v3 = corr_p(1, e, v3);
-        if (wpr[q]) st_nt(pr_out + off[q], v3);
+    for (int q = 0; q < NE; q++) {
+      double v = pr[op + off[q]];
+      const int e = threadIdx.x + q * FT_N;
+      if (q < NE - 1 || has_last) {
+        if constexpr (CORR) {
+          v = corr_p(k0, e, v);
+          if (wpr[q]) st_nt(pr_out + op + off[q], v);
+        }
+        sp[k0 & 1][e] = v;
       }
-      const int e = threadIdx.x + q * 256;
-      sq[0][1][e] = v0;
-      sq[1][1][e] = v1;
-      sq[2][1][e] = v2;
-      sq[0][2][e] = w0;
-      sq[1][2][e] = w1;
-      sq[2][2][e] = w2;
-      sp[1][e] = v3;
     }
   }
   __syncthreads();
-  const int nrm = g.nrm;
-  double yv;
+  if constexpr (!CORR) {
+    if (k0 > 1) {
+      const int sm = (k0 - 1) % 3;
+#pragma unroll
+      for (int u = 0; u < LPT; u++) {
+        cm[u][0] = sq[0][sm][base[u]];
+        cm[u][1] = sq[0][sm][base[u] + 1];
+        cm[u][2] = sq[1][sm][base[u]];
+        cm[u][3] = sq[2][sm][base[u]];
+        cm[u][4] = sq[2][sm][base[u] + FT_W];
+      }
+      __syncthreads();  // the first iteration overwrites that slot
+    }
+  }
 
-  for (int k = 1; k <= nrm; k++) {
+  for (int k = k0; k <= k1; k++) {
     // prefetch plane k+2 of the velocity, plane k+1 of the pressure and of
-    // the RK histories.  In the last iteration these re-read the last plane
-    // (their values are not used), so the loads carry no condition.
+    // the RK histories.  In the last iteration these re-read planes just
+    // read (their values are not used), so the loads carry no condition.
     double nq[3][NE], np[NE], n1[LPT], n2[LPT], n3[LPT], nd[CORR ? NE2 : 1];
-    const long long oq = (long long)(k + 2 <= g.nr ? k + 1 : g.nr - 1) * P;
-    const long long op = (long long)(k + 1 <= nrm ? k : nrm - 1) * P;
+    const long long oq = (long long)min(k + 1, k1) * P;
+    const long long op = (long long)min(k, k1 - 1) * P;
 #pragma unroll
     for (int q = 0; q < NE; q++) {
       nq[0][q] = qt[oq + off[q]];
@@ -765,7 +898,7 @@ DEVI void helm_fwd_body(
     }
     if constexpr (CORR) {
       // dph plane k+2 (clamped to nrm: beyond it no correction reads dph)
-      const long long od = (long long)(k + 2 <= nrm ? k + 1 : nrm - 1) * P;
+      const long long od = (long long)(min(min(k + 2, k1 + 1), nrm) - 1) * P;
 #pragma unroll
       for (int q = 0; q < NE2; q++) nd[q] = dph[od + off2[q]];
     }
@@ -780,9 +913,10 @@ DEVI void helm_fwd_body(
 #pragma unroll
       for (int u = 0; u < LPT; u++) n1[u] = n2[u] = n3[u] = 0.0;
     }
-    const int sm = (k + 2) % 3, sc = k % 3, sn = (k + 1) % 3;  // planes k-1, k, k+1
+        const int sm = (k + 2) % 3, sc = k % 3, sn = (k + 1) % 3;  // planes k-1, k, k+1
     const double *spk = sp[k & 1];
-    const HelmPlane hc = g.hp[k];
+    const HelmPlane hc = ldk_record(g.hp + k);
+    const RhsRow rw = ldk_record(rows + k);
 #pragma unroll
     for (int u = 0; u < LPT; u++) {
       if (!valid[u]) continue;
@@ -795,41 +929,37 @@ DEVI void helm_fwd_body(
       Z.m00 = cm[u][3]; Z.m01 = 0.0; Z.m10 = cm[u][4];
       const double pr_c = spk[base[u]], pr_im = spk[base[u] - 1], pr_jm = spk[base[u] - FT_W];
       const long long o = (long long)(k - 1) * P + l[u];
+      // the matrix rows of q_theta and q_z next to a free-slip wall
+      double am_t = rw.am_t, ap_t = rw.ap_t, am_z = rw.am_z, ap_z = rw.ap_z;
+      if constexpr (!UNIFORM) {
+        if (k == 1 && fic[u] == 0.0) ap_t = rw.x_t, ap_z = rw.x_z;
+        if (k == nrm && foc[u] == 0.0) am_t = rw.x_t, am_z = rw.x_z;
+      }
       // q_theta
       {
         const double dqv = explicit_qt_g(g, hc, T, R, Z, k);
         const double qm = (k > 1) ? T(-1, 0, 0) : 0.0, qp = (k < nrm) ? T(1, 0, 0) : 0.0;
-        const double r = rhs_qt<UNIFORM>(g, hc, a, k, qm, T(0, 0, 0), qp, pr_c, pr_im, dqv, h1[u], fic[u], foc[u]);
+        double r = rhs_qt<UNIFORM>(g, hc, a, k, qm, T(0, 0, 0), qp, pr_c, pr_im, dqv, h1[u], fic[u], foc[u]);
         st_nt(ru1 + o, dqv);
-        if (k == 1) {
-          ct[u] = (r + a.bc1) * Tt[u].sc(0);
-        } else {
-          lsolve_step(Tt[u], k - 2, r * Tt[u].sc(k - 1), ct[u], yv);
-          st_nt(yt + o - P, yv + Tt[u].uq(k - 2, qm, T(0, 0, 0), qp));
-        }
+        if (k == 1) r = r + a.bc1;
+        st_nt(yt + o, r * rw.sc_t + (am_t * qm + T(0, 0, 0) + ap_t * qp));
       }
-      // q_r (rows 2..nrm; row 1 is the wall with zero right-hand side)
+            // q_r (planes 2..nrm; the walls have no row)
       if (k >= 2) {
         const double dphv = explicit_qr_g(g, hc, T, R, Z, k);
         const double r = rhs_qr(hc, a, R(-1, 0, 0), R(0, 0, 0), R(1, 0, 0), pr_c, pr_km[u], dphv, h2[u]);
         st_nt(ru2 + o, dphv);
-        lsolve_step(Tr, k - 2, r * Tr.sc(k - 1), cr[u], yv);
-        st_nt(yr + o - P, yv + Tr.uq(k - 2, R(-1, 0, 0), R(0, 0, 0), R(1, 0, 0)));
+        st_nt(yr + o, r * rw.sc_r + (rw.am_r * R(-1, 0, 0) + R(0, 0, 0) + rw.ap_r * R(1, 0, 0)));
       }
-      // q_z
+            // q_z
       {
         const double qcv = explicit_qz_g(g, hc, T, R, Z, k);
         const double qm = (k > 1) ? Z(-1, 0, 0) : 0.0, qp = (k < nrm) ? Z(1, 0, 0) : 0.0;
         const double r = rhs_qz<UNIFORM>(g, hc, a, k, qm, Z(0, 0, 0), qp, pr_c, pr_jm, qcv, h3[u], fic[u], foc[u]);
         st_nt(ru3 + o, qcv);
-        if (k == 1) {
-          cz[u] = r * Tz[u].sc(0);
-        } else {
-          lsolve_step(Tz[u], k - 2, r * Tz[u].sc(k - 1), cz[u], yv);
-          st_nt(yz + o - P, yv + Tz[u].uq(k - 2, qm, Z(0, 0, 0), qp));
-        }
+        st_nt(yz + o, r * rw.sc_z + (am_z * qm + Z(0, 0, 0) + ap_z * qp));
       }
-      pr_km[u] = pr_c;
+            pr_km[u] = pr_c;
       if constexpr (!CORR) {
         cm[u][0] = T(0, 0, 0);
         cm[u][1] = T(0, 0, 1);
@@ -838,6 +968,7 @@ DEVI void helm_fwd_body(
         cm[u][4] = Z(0, 1, 0);
       }
     }
+    if (k == k1) break;
 #pragma unroll
     for (int u = 0; u < LPT; u++) {
       h1[u] = n1[u];
@@ -848,23 +979,20 @@ DEVI void helm_fwd_body(
       // dph slot (k+2)%3 held plane k-1, last read before the previous barrier
 #pragma unroll
       for (int q = 0; q < NE2; q++)
-        if (q < NE2 - 1 || has_last2) sd[(k + 2) % 3][threadIdx.x + q * 256] = nd[q];
+        if (q < NE2 - 1 || has_last2) sd[(k + 2) % 3][threadIdx.x + q * FT_N] = nd[q];
       // the ring slot of plane k-1 is read above, and the dph plane k+2 just
       // written is read by the staging below
       __syncthreads();
     }
-    // in the last iteration these fill slots no later plane reads
     const int s2 = (k + 2) % 3;
 #pragma unroll
     for (int q = 0; q < NE; q++) {
-      const int e = threadIdx.x + q * 256;
+      const int e = threadIdx.x + q * FT_N;
       if (q < NE - 1 || has_last) {
         if constexpr (CORR) {
           corr_q(k + 2, e, nq[0][q], nq[1][q], nq[2][q]);
-          if (k + 1 <= nrm) {
-            np[q] = corr_p(k + 1, e, np[q]);
-            if (wpr[q]) st_nt(pr_out + (long long)k * P + off[q], np[q]);
-          }
+          np[q] = corr_p(k + 1, e, np[q]);
+          if (wpr[q]) st_nt(pr_out + (long long)k * P + off[q], np[q]);
         }
         sq[0][s2][e] = nq[0][q];
         sq[1][s2][e] = nq[1][q];
@@ -874,55 +1002,47 @@ DEVI void helm_fwd_body(
     }
     __syncthreads();
   }
-  // after the last barrier the ring still holds planes nrm and nrm+1
-  const int s0 = nrm % 3, s1 = (nrm + 1) % 3;
-#pragma unroll
-  for (int u = 0; u < LPT; u++) {
-    if (!valid[u]) continue;
-    const int b = base[u];
-    yt[(long long)(nrm - 1) * P + l[u]] = ct[u] + Tt[u].ud(nrm - 1) * sq[0][s0][b];
-    yz[(long long)(nrm - 1) * P + l[u]] = cz[u] + Tz[u].ud(nrm - 1) * sq[2][s0][b];
-    double c2 = cr[u];
-    lsolve_step(Tr, g.nr - 2, 0.0, c2, yv);  // wall row nr
-    yr[(long long)(g.nr - 2) * P + l[u]] = yv + Tr.ud(g.nr - 2) * sq[1][s0][b] + Tr.du(g.nr - 2) * sq[1][s1][b];
-    yr[(long long)(g.nr - 1) * P + l[u]] = c2 + Tr.ud(g.nr - 1) * sq[1][s1][b];
-  }
 }
 
+// Planes k0..k1 of segment s of ns.
+DEVI int seg_first(int s, int ns, int nrm) { return 1 + (int)(((long long)s * nrm) / ns); }
+
 template <bool UNIFORM, int LPT, bool CORR>
-__global__ __launch_bounds__(256) void k_helm_fwd(
+__global__ __launch_bounds__(FT_N) void k_helm_rhs(
     GridDev g, ImpArgs a, const double *__restrict__ qt, const double *__restrict__ qr,
     const double *__restrict__ qz, const double *__restrict__ pr, double *__restrict__ ru1,
     double *__restrict__ ru2, double *__restrict__ ru3, double *__restrict__ yt,
     double *__restrict__ yr, double *__restrict__ yz, const unsigned char *__restrict__ icyl,
-    const unsigned char *__restrict__ ocyl, const double *__restrict__ lut,
-    const double *__restrict__ lur, const double *__restrict__ luz, int nt, int ntx, int ntz,
-    CorrIn ci, const double *__restrict__ dph, double *__restrict__ pr_out) {
-  helm_fwd_body<UNIFORM, LPT, CORR>(xcd_tile(blockIdx.x, ntx * ntz), g, a, qt, qr, qz, pr, ru1,
-                                    ru2, ru3, yt, yr, yz, icyl, ocyl, lut, lur, luz, nt, ntx, ci,
-                                    dph, pr_out);
+    const unsigned char *__restrict__ ocyl, const RhsRow *__restrict__ rows, int ntx, int ntz,
+    int nseg, CorrIn ci, const double *__restrict__ dph, double *__restrict__ pr_out) {
+  const int lin = xcd_tile(blockIdx.x, gridDim.x), seg = lin / (ntx * ntz);
+  helm_rhs_body<UNIFORM, LPT, CORR>(lin - seg * (ntx * ntz), seg_first(seg, nseg, g.nrm),
+                                    seg_first(seg + 1, nseg, g.nrm) - 1, g, a, qt, qr, qz, pr,
+                                    ru1, ru2, ru3, yt, yr, yz, icyl, ocyl, rows, ntx, ci, dph,
+                                    pr_out);
 }
 
-// Grouped: blockIdx.x = tile, blockIdx.y = instance of the shape group; the
-// XCD remap runs over the flattened (instance, tile) index.
+// Grouped: blockIdx.x = tile and segment, blockIdx.y = instance of the shape
+// group; the XCD remap runs over the flattened index.
 template <bool UNIFORM, int LPT, bool CORR>
-__global__ __launch_bounds__(256) void k_helm_fwd_g(const StepDesc *__restrict__ tab,
+__global__ __launch_bounds__(FT_N) void k_helm_rhs_g(const StepDesc *__restrict__ tab,
                                                     const BatchDyn *__restrict__ dyn, int ns,
-                                                    int ntx, int ntz) {
-  const int ntiles = ntx * ntz;
+                                                    int ntx, int ntz, int nseg) {
   const int lin = xcd_tile(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
-  const int inst = lin / ntiles, tile = lin - inst * ntiles;
+  const int inst = lin / (int)gridDim.x, rest = lin - inst * (int)gridDim.x;
+  const int seg = rest / (ntx * ntz), tile = rest - seg * (ntx * ntz);
   const StepDesc &d = tab[inst];
   if (inst_stopped(d)) return;
   ImpArgs a = d.a;
   a.vwall_in = glob(dyn)[inst].vwall[ns - 1];
   a.bc1 = glob(dyn)[inst].bc1[ns - 1];
   const CorrIn ci{d.dt, d.corr_al, d.beta};
-  helm_fwd_body<UNIFORM, LPT, CORR>(
-      tile, glob(d.g), a, glob(d.f[TC_QT]), glob(d.f[TC_QR]), glob(d.f[TC_QZ]), glob(d.pr_in),
-      glob(d.f[TC_RU1]), glob(d.f[TC_RU2]), glob(d.f[TC_RU3]), glob(d.f[TC_RHS]), glob(d.f[TC_DQ]),
-      glob(d.f[TC_QCAP]), glob(d.icyl), glob(d.ocyl), glob(d.lut), glob(d.lur), glob(d.luz),
-      d.lu_nt, ntx, ci, glob(d.f[TC_DPH]), glob(d.pr_out));
+  helm_rhs_body<UNIFORM, LPT, CORR>(
+      tile, seg_first(seg, nseg, d.g.nrm), seg_first(seg + 1, nseg, d.g.nrm) - 1, glob(d.g), a,
+      glob(d.f[TC_QT]), glob(d.f[TC_QR]), glob(d.f[TC_QZ]), glob(d.pr_in), glob(d.f[TC_RU1]),
+      glob(d.f[TC_RU2]), glob(d.f[TC_RU3]), glob(d.f[TC_RHS]), glob(d.f[TC_DQ]),
+      glob(d.f[TC_QCAP]), glob(d.icyl), glob(d.ocyl), glob(d.rows), ntx, ci, glob(d.f[TC_DPH]),
+      glob(d.pr_out));
 }
 
 static ImpArgs imp_args(const tc_ctx *c) {
@@ -939,103 +1059,184 @@ static ImpArgs imp_args(const tc_ctx *c) {
   return a;
 }
 
-static const double *lu_slot(const tc_ctx *c, int comp) {
-  // tables laid out [slot = ns-1][comp][variant 0..3][nt]
-  return c->lu + ((size_t)(c->ns - 1) * 3 + comp) * 4 * (size_t)c->lu_nt;
+// Layout of c->lu: [slot = ns-1] of tables [comp][variant 0..3][lu_nt], then
+// the records of the right-hand sides for k = 0..nrm (record 0 unused).
+size_t lu_slot_doubles(const tc_ctx *c) {
+  return (size_t)3 * 4 * c->lu_nt + (size_t)(c->nrm + 1) * (sizeof(RhsRow) / sizeof(double));
+}
+const double *lu_table(const tc_ctx *c, int ns, int comp) {
+  return c->lu + (size_t)(ns - 1) * lu_slot_doubles(c) + (size_t)comp * 4 * c->lu_nt;
+}
+const RhsRow *rhs_rows(const tc_ctx *c, int ns) {
+  return reinterpret_cast<const RhsRow *>(c->lu + (size_t)(ns - 1) * lu_slot_doubles(c) +
+                                          (size_t)3 * 4 * c->lu_nt);
 }
 
 static unsigned line_blocks(const tc_ctx *c) { return (unsigned)((c->P + 255) / 256); }
 
-static void launch_bwd(tc_ctx *c, int which, const char *name) {
+// Shape of the partitioned solve: waves per block and the row capacity R of
+// its kernel, by the line length alone (an instance's bits must not depend
+// on what it shares a launch with).  ns = 0: the serial form.  Measured us
+// with R = 8 / 25 / 50 / 100: 128x128x97 20 / 17 / 21 / 32, 256x256x193
+// 144 (R = 16) / 110 / 120 / 131, 256x256x385 - / 265 / 232 / 245,
+// 512x512x385 - / 1020 / 957 / 960.
+struct SolveShape {
+  int ns, rows;
+};
+static SolveShape solve_shape(const tc_ctx *c) {
+  const int n = c->nrm;
+  if (c->lu_pivots) return {0, 0};
+  const int R = n <= 72 ? 8 : (n <= 256 ? 25 : (n <= 400 ? 50 : 100));
+  const int ns = (n + R - 1) / R;
+  return ns <= (R > 32 ? 8 : 16) ? SolveShape{ns, R} : SolveShape{0, 0};
+}
+
+template <bool U, bool FOLD>
+static void launch_solve_u(const SolveShape s, dim3 grid, hipStream_t st, const tc_ctx *c,
+                           const SolveIO &io, int comp0) {
+  const dim3 block(64, (unsigned)s.ns);
+  const size_t lds = sizeof(double) * 4 * 64 * (size_t)s.ns;
+#define TC_SOLVE(R)                                                                          \
+  hipLaunchKernelGGL((k_helm_solve<R, U, FOLD>), grid, block, lds, st, c->gd, io, c->mask,           \
+                     c->mask + c->P, c->lu_nt, comp0)
+  switch (s.rows) {
+    case 8: TC_SOLVE(8); break;
+    case 25: TC_SOLVE(25); break;
+    case 50: TC_SOLVE(50); break;
+    default: TC_SOLVE(100); break;
+  }
+#undef TC_SOLVE
+}
+
+// FOLD: all three components; otherwise the one component comp0
+template <bool FOLD>
+static void launch_solve(tc_ctx *c, const SolveIO &io, int comp0) {
+  const SolveShape s = solve_shape(c);
+  const unsigned ncomp = FOLD ? 3 : 1;
+  if (s.ns == 0) {
+    hipLaunchKernelGGL(k_helm_solve_serial, dim3(line_blocks(c), ncomp), dim3(256), 0, c->stream,
+                       c->gd, io, c->mask, c->mask + c->P, c->lu_nt, comp0, FOLD);
+    return;
+  }
+  const dim3 grid((unsigned)((c->P + 63) / 64), ncomp);
+  if (c->masks_uniform_one)
+    launch_solve_u<true, FOLD>(s, grid, c->stream, c, io, comp0);
+  else
+    launch_solve_u<false, FOLD>(s, grid, c->stream, c, io, comp0);
+}
+
+static SolveIO solve_io(const tc_ctx *c) {
+  SolveIO io;
+  io.q[0] = c->f[TC_QT];
+  io.q[1] = c->f[TC_QR];
+  io.q[2] = c->f[TC_QZ];
+  io.y[0] = c->f[TC_RHS];
+  io.y[1] = c->f[TC_DQ];
+  io.y[2] = c->f[TC_QCAP];
+  for (int q = 0; q < 3; q++) io.lu[q] = lu_table(c, c->ns, q);
+  return io;
+}
+
+// Routine-level entries: right-hand side into the rhs field, then the solve.
+template <int WHICH>
+static void launch_implicit(tc_ctx *c, const char *name, int q, int expl, int ru) {
   timer_begin(c, name);
-  hipLaunchKernelGGL(k_helm_bwd<true>, dim3(line_blocks(c)), dim3(256), 0, c->stream, c->gd,
-                     c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->f[TC_RHS], c->f[TC_DQ],
-                     c->f[TC_QCAP], c->mask, c->mask + c->P, lu_slot(c, LU_QT), lu_slot(c, LU_QR),
-                     lu_slot(c, LU_QZ), c->lu_nt, which);
+  hipLaunchKernelGGL(k_implicit<WHICH>, point_grid(c, WHICH == 1 ? c->nrm - 1 : c->nrm),
+                     dim3(64, 4), 0, c->stream, c->gd, imp_args(c), c->f[q], c->f[TC_PR],
+                     c->f[expl], c->f[ru], c->f[TC_RHS], c->mask, c->mask + c->P,
+                     rhs_rows(c, c->ns));
   timer_end(c);
+  SolveIO io = solve_io(c);
+  io.y[WHICH] = c->f[TC_RHS];
+  launch_solve<false>(c, io, WHICH);
+}
+void launch_implicit_qt(tc_ctx *c) { launch_implicit<0>(c, "implicit_qt", TC_QT, TC_DQ, TC_RU1); }
+void launch_implicit_qr(tc_ctx *c) { launch_implicit<1>(c, "implicit_qr", TC_QR, TC_DPH, TC_RU2); }
+void launch_implicit_qz(tc_ctx *c) { launch_implicit<2>(c, "implicit_qz", TC_QZ, TC_QCAP, TC_RU3); }
+
+static long long helm_tiles(const tc_ctx *c, int lpt) {
+  return (long long)((c->nthm + FT_I - 1) / FT_I) * ((c->nzm + FT_J * lpt - 1) / (FT_J * lpt));
 }
 
-// Routine-level entries: right-hand side + forward substitution into the rhs
-// field, then the backward substitution.
-void launch_implicit_qt(tc_ctx *c) {
-  timer_begin(c, "implicit_qt");
-  hipLaunchKernelGGL(k_implicit_qt, dim3(line_blocks(c)), dim3(256), 0, c->stream, c->gd,
-                     imp_args(c), c->f[TC_QT], c->f[TC_PR], c->f[TC_DQ], c->f[TC_RU1],
-                     c->f[TC_RHS], c->mask, c->mask + c->P, lu_slot(c, LU_QT), c->lu_nt);
-  timer_end(c);
-  hipLaunchKernelGGL(k_helm_bwd<false>, dim3(line_blocks(c)), dim3(256), 0, c->stream, c->gd,
-                     c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->f[TC_RHS], c->f[TC_RHS],
-                     c->f[TC_RHS], c->mask, c->mask + c->P, lu_slot(c, LU_QT), lu_slot(c, LU_QR),
-                     lu_slot(c, LU_QZ), c->lu_nt, 1);
-}
-void launch_implicit_qr(tc_ctx *c) {
-  timer_begin(c, "implicit_qr");
-  hipLaunchKernelGGL(k_implicit_qr, dim3(line_blocks(c)), dim3(256), 0, c->stream, c->gd,
-                     imp_args(c), c->f[TC_QR], c->f[TC_PR], c->f[TC_DPH], c->f[TC_RU2],
-                     c->f[TC_RHS], lu_slot(c, LU_QR), c->lu_nt);
-  timer_end(c);
-  hipLaunchKernelGGL(k_helm_bwd<false>, dim3(line_blocks(c)), dim3(256), 0, c->stream, c->gd,
-                     c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->f[TC_RHS], c->f[TC_RHS],
-                     c->f[TC_RHS], c->mask, c->mask + c->P, lu_slot(c, LU_QT), lu_slot(c, LU_QR),
-                     lu_slot(c, LU_QZ), c->lu_nt, 2);
-}
-void launch_implicit_qz(tc_ctx *c) {
-  timer_begin(c, "implicit_qz");
-  hipLaunchKernelGGL(k_implicit_qz, dim3(line_blocks(c)), dim3(256), 0, c->stream, c->gd,
-                     imp_args(c), c->f[TC_QZ], c->f[TC_PR], c->f[TC_QCAP], c->f[TC_RU3],
-                     c->f[TC_RHS], c->mask, c->mask + c->P, lu_slot(c, LU_QZ), c->lu_nt);
-  timer_end(c);
-  hipLaunchKernelGGL(k_helm_bwd<false>, dim3(line_blocks(c)), dim3(256), 0, c->stream, c->gd,
-                     c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->f[TC_RHS], c->f[TC_RHS],
-                     c->f[TC_RHS], c->mask, c->mask + c->P, lu_slot(c, LU_QT), lu_slot(c, LU_QR),
-                     lu_slot(c, LU_QZ), c->lu_nt, 4);
+// r segments of the fused front over n instances of this shape.  A launch
+// takes (rounds of resident blocks) x (planes per segment and about three
+// that a segment stages before its first), and its blocks, which run apart,
+// end within about a quarter of a segment of each other; the segment count
+// with the least of that, of at least two planes each.  Measured, one
+// segment against the chosen count: 64x64x65 133 -> 15 us, 256x256x193
+// 400 -> 212 us, 512x512x385 (two lines per thread) 1775 -> 1674 us.
+static int helm_segments(const tc_ctx *c, int lpt, bool corr, int n) {
+  const long long tiles = n * helm_tiles(c, lpt), slots = c->helm_slots[corr];
+  int best = 1;
+  long long cost = 0;
+  for (int s = 1; s <= c->nrm / 2; s++) {
+    const long long len = (c->nrm + s - 1) / s, rounds = (tiles * s + slots - 1) / slots;
+    const long long t = 4 * rounds * (len + 3) + len;
+    if (s == 1 || t < cost) {
+      cost = t;
+      best = s;
+    }
+  }
+  return best;
 }
 
-// Fused path: y_theta -> rhs, y_r -> dq, y_z -> qcap (the explicit terms
-// stay in registers, so those fields serve as scratch).
+// Fused path: right-hand sides of q_theta -> rhs, q_r -> dq, q_z -> qcap (the
+// explicit terms stay in registers, so those fields serve as scratch).
 template <bool U, int LPT, bool CORR>
-static void launch_fwd(tc_ctx *c, const double *pr, const CorrIn &ci, double *pr_out) {
-  const int ntx = (c->nthm + FT_I - 1) / FT_I, ntz = (c->nzm + 4 * LPT - 1) / (4 * LPT);
-  hipLaunchKernelGGL((k_helm_fwd<U, LPT, CORR>), dim3((unsigned)(ntx * ntz)), dim3(256), 0,
+static void launch_rhs(tc_ctx *c, const double *pr, const CorrIn &ci, double *pr_out) {
+  const int ntx = (c->nthm + FT_I - 1) / FT_I, ntz = (c->nzm + FT_J * LPT - 1) / (FT_J * LPT);
+  const int nseg = helm_segments(c, LPT, CORR, 1);
+  hipLaunchKernelGGL((k_helm_rhs<U, LPT, CORR>), dim3((unsigned)(ntx * ntz * nseg)), dim3(FT_N), 0,
                      c->stream, c->gd, imp_args(c), c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], pr,
                      c->f[TC_RU1], c->f[TC_RU2], c->f[TC_RU3], c->f[TC_RHS], c->f[TC_DQ],
-                     c->f[TC_QCAP], c->mask, c->mask + c->P, lu_slot(c, LU_QT), lu_slot(c, LU_QR),
-                     lu_slot(c, LU_QZ), c->lu_nt, ntx, ntz, ci, c->f[TC_DPH], pr_out);
+                     c->f[TC_QCAP], c->mask, c->mask + c->P, rhs_rows(c, c->ns), ntx, ntz, nseg,
+                     ci, c->f[TC_DPH], pr_out);
 }
 
-// Lines per thread of the fused kernel: two where the two-line tiles alone
-// fill every resident slot of the device at least once, one otherwise.
-// Two lines per thread give each block twice the work per plane for less
-// than twice the time, but half the tiles: at 512x512x385 the 512 two-line
-// tiles fill the 512 slots once (2771 us per launch against 3445 for one
-// line), at 1024x1024x769 four times (22.4 ms against 26.0), while a lone
-// 256^2x193 grid (128 two-line tiles) runs faster with one line.
-int choose_helm_lpt(const tc_ctx *c) {
+// blocks of the fused front that one compute unit holds (asked once: every
+// device this library is built for is alike)
+template <int LPT, bool CORR>
+static int resident_blocks(int cus) {
+  static const int per_cu = [] {
+    int n = 0;
+    const hipError_t e =
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_helm_rhs<true, LPT, CORR>, FT_N, 0);
+    return e == hipSuccess && n > 0 ? n : 2;
+  }();
+  return per_cu * cus;
+}
+
+// Lines per thread (lpt, 0: chosen here) and the blocks of the fused front
+// resident at once.  Two lines per thread stage 1.29 elements per point
+// instead of 1.55, but halve the tiles; they are the default where their
+// tiles fill the device in segments of 32 planes.  One against two lines:
+// 64x64x65 15 / 17 us, 192x128x129 73 / 73, 375x240x151 362 / 336,
+// 512x512x385 1721 / 1674 (with the correction 2650 / 2581).
+void choose_helm_schedule(tc_ctx *c, int lpt) {
   int dev = 0, cus = 0;
   hipGetDevice(&dev);
   hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  if (cus <= 0) return 1;
-  int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_helm_fwd<true, 2, true>, 256, 0) !=
-          hipSuccess ||
-      per_cu <= 0)
-    return 1;
-  const long long tiles = (long long)((c->nthm + FT_I - 1) / FT_I) * ((c->nzm + 7) / 8);
-  return tiles >= (long long)per_cu * cus ? 2 : 1;
+  if (cus <= 0) cus = 256;
+  if (lpt == 0) lpt = helm_tiles(c, 2) * (c->nrm / 32) >= resident_blocks<2, true>(cus) ? 2 : 1;
+  c->helm_lpt = lpt;
+  c->helm_slots[0] = lpt == 2 ? resident_blocks<2, false>(cus) : resident_blocks<1, false>(cus);
+  c->helm_slots[1] = lpt == 2 ? resident_blocks<2, true>(cus) : resident_blocks<1, true>(cus);
 }
 
 void launch_helmholtz_fused(tc_ctx *c) {
   timer_begin(c, "helm_fwd");
   const CorrIn ci{};
   if (c->masks_uniform_one) {
-    if (c->helm_lpt == 2) launch_fwd<true, 2, false>(c, c->f[TC_PR], ci, nullptr);
-    else launch_fwd<true, 1, false>(c, c->f[TC_PR], ci, nullptr);
+    if (c->helm_lpt == 2) launch_rhs<true, 2, false>(c, c->f[TC_PR], ci, nullptr);
+    else launch_rhs<true, 1, false>(c, c->f[TC_PR], ci, nullptr);
   } else {
-    if (c->helm_lpt == 2) launch_fwd<false, 2, false>(c, c->f[TC_PR], ci, nullptr);
-    else launch_fwd<false, 1, false>(c, c->f[TC_PR], ci, nullptr);
+    if (c->helm_lpt == 2) launch_rhs<false, 2, false>(c, c->f[TC_PR], ci, nullptr);
+    else launch_rhs<false, 1, false>(c, c->f[TC_PR], ci, nullptr);
   }
   timer_end(c);
-  launch_bwd(c, 7, "helm_bwd");
+  timer_begin(c, "helm_bwd");
+  launch_solve<true>(c, solve_io(c), 0);
+  timer_end(c);
 }
 
 // The same with the previous substep's pressure correction (dph, al_prev)
@@ -1046,14 +1247,16 @@ void launch_helmholtz_fused_corr(tc_ctx *c, const double *pr_in, double *pr_out,
   timer_begin(c, "helm_fwd_corr");
   const CorrIn ci{c->dt, al_prev, c->beta};
   if (c->masks_uniform_one) {
-    if (c->helm_lpt == 2) launch_fwd<true, 2, true>(c, pr_in, ci, pr_out);
-    else launch_fwd<true, 1, true>(c, pr_in, ci, pr_out);
+    if (c->helm_lpt == 2) launch_rhs<true, 2, true>(c, pr_in, ci, pr_out);
+    else launch_rhs<true, 1, true>(c, pr_in, ci, pr_out);
   } else {
-    if (c->helm_lpt == 2) launch_fwd<false, 2, true>(c, pr_in, ci, pr_out);
-    else launch_fwd<false, 1, true>(c, pr_in, ci, pr_out);
+    if (c->helm_lpt == 2) launch_rhs<false, 2, true>(c, pr_in, ci, pr_out);
+    else launch_rhs<false, 1, true>(c, pr_in, ci, pr_out);
   }
   timer_end(c);
-  launch_bwd(c, 7, "helm_bwd");
+  timer_begin(c, "helm_bwd");
+  launch_solve<true>(c, solve_io(c), 0);
+  timer_end(c);
 }
 
 // ---------------------------------------------------------------------------
@@ -1926,27 +2129,52 @@ void launch_triad(tc_ctx *c, int a, int b, int cc, double s) {
 // ---------------------------------------------------------------------------
 
 template <bool U, int LPT>
-static void launch_fwd_g(tc_ctx *c, const StepDesc *tab, const BatchDyn *dyn, int ns, int n,
+static void launch_rhs_g(tc_ctx *c, const StepDesc *tab, const BatchDyn *dyn, int ns, int n,
                          hipStream_t st, bool corr) {
-  const int ntx = (c->nthm + FT_I - 1) / FT_I, ntz = (c->nzm + 4 * LPT - 1) / (4 * LPT);
-  const dim3 grid((unsigned)(ntx * ntz), (unsigned)n);
+  const int ntx = (c->nthm + FT_I - 1) / FT_I, ntz = (c->nzm + FT_J * LPT - 1) / (FT_J * LPT);
+  const int nseg = helm_segments(c, LPT, corr, n);
+  const dim3 grid((unsigned)(ntx * ntz * nseg), (unsigned)n);
   if (corr)
-    hipLaunchKernelGGL((k_helm_fwd_g<U, LPT, true>), grid, dim3(256), 0, st, tab, dyn, ns, ntx, ntz);
+    hipLaunchKernelGGL((k_helm_rhs_g<U, LPT, true>), grid, dim3(FT_N), 0, st, tab, dyn, ns, ntx, ntz,
+                       nseg);
   else
-    hipLaunchKernelGGL((k_helm_fwd_g<U, LPT, false>), grid, dim3(256), 0, st, tab, dyn, ns, ntx, ntz);
+    hipLaunchKernelGGL((k_helm_rhs_g<U, LPT, false>), grid, dim3(FT_N), 0, st, tab, dyn, ns, ntx,
+                       ntz, nseg);
+}
+
+template <bool U>
+static void launch_solve_g(const SolveShape s, dim3 grid, hipStream_t st, const StepDesc *tab) {
+  const dim3 block(64, (unsigned)s.ns);
+  const size_t lds = sizeof(double) * 4 * 64 * (size_t)s.ns;
+#define TC_SOLVE(R) hipLaunchKernelGGL((k_helm_solve_g<R, U>), grid, block, lds, st, tab)
+  switch (s.rows) {
+    case 8: TC_SOLVE(8); break;
+    case 25: TC_SOLVE(25); break;
+    case 50: TC_SOLVE(50); break;
+    default: TC_SOLVE(100); break;
+  }
+#undef TC_SOLVE
 }
 
 // corr: every instance's descriptor carries a deferred correction
 void launch_helmholtz_fused_g(tc_ctx *c, const StepDesc *tab, const BatchDyn *dyn, int ns, int n,
                               hipStream_t st, bool corr) {
   if (c->masks_uniform_one) {
-    if (c->helm_lpt == 2) launch_fwd_g<true, 2>(c, tab, dyn, ns, n, st, corr);
-    else launch_fwd_g<true, 1>(c, tab, dyn, ns, n, st, corr);
+    if (c->helm_lpt == 2) launch_rhs_g<true, 2>(c, tab, dyn, ns, n, st, corr);
+    else launch_rhs_g<true, 1>(c, tab, dyn, ns, n, st, corr);
   } else {
-    if (c->helm_lpt == 2) launch_fwd_g<false, 2>(c, tab, dyn, ns, n, st, corr);
-    else launch_fwd_g<false, 1>(c, tab, dyn, ns, n, st, corr);
+    if (c->helm_lpt == 2) launch_rhs_g<false, 2>(c, tab, dyn, ns, n, st, corr);
+    else launch_rhs_g<false, 1>(c, tab, dyn, ns, n, st, corr);
   }
-  hipLaunchKernelGGL(k_helm_bwd_g, dim3(line_blocks(c), (unsigned)n), dim3(256), 0, st, tab);
+  const SolveShape s = solve_shape(c);
+  if (s.ns == 0) {
+    hipLaunchKernelGGL(k_helm_solve_serial_g, dim3(line_blocks(c), 3, (unsigned)n), dim3(256), 0,
+                       st, tab);
+    return;
+  }
+  const dim3 grid((unsigned)((c->P + 63) / 64), 3, (unsigned)n);
+  if (c->masks_uniform_one) launch_solve_g<true>(s, grid, st, tab);
+  else launch_solve_g<false>(s, grid, st, tab);
 }
 
 void launch_correct_both_g(tc_ctx *c, const StepDesc *tab, int n, hipStream_t st) {

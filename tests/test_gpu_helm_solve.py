@@ -1,0 +1,60 @@
+"""The Helmholtz right-hand sides in r segments and the partitioned radial
+solves against the oracle, at the line lengths where their shapes change:
+one segment, a ragged last one, the ends of each row capacity (72, 256, 400,
+800 rows) and one past the longest, and for factors that exchange rows.
+Planes of 180 lines: no multiple of 64, and one partial theta tile.
+Tolerance: the 1e-10 relative L2 of the workload contract."""
+import numpy as np
+import pytest
+
+from helpers import compare_fields, load_both, random_state, rel_l2, small_params, start_pair
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("defer", ["0", "2"])
+@pytest.mark.parametrize("nrm", [3, 8, 9, 16, 72, 73, 256, 257, 400, 401, 800, 801])
+def test_step_at_row_capacities(tc, oracle, monkeypatch, nrm, defer):
+    monkeypatch.setenv("TC_DEFER_CORRECTION", defer)
+    p = small_params(tc, 20, 9, nrm, ntst=1000, dtmin=1e-4, dtmax=1e-4, sizepert=0.1,
+                     omegapert=0.5, virotext=-0.3)
+    dev, orc = start_pair(tc, oracle, p, 11, 1e-2)
+    for n in range(2):
+        assert dev.step(n)[0] == orc.step(n)[0] == 0
+    compare_fields(dev, orc, nrm, 1e-10)
+
+
+@pytest.mark.parametrize("nrm", [17, 100, 300, 500])
+def test_slip_walls_on_both_cylinders(tc, oracle, nrm):
+    """Masks that differ from line to line, on the outer wall too, through
+    the routine entries (which keep the masks they are given)."""
+    p = small_params(tc, 20, 9, nrm, ren=500.0)
+    _implicit(tc, oracle, p, 1e-4, nrm)
+
+
+@pytest.mark.parametrize("nrm,dt", [(9, 2.0), (33, 0.3)])
+def test_factors_with_row_exchanges(tc, oracle, nrm, dt):
+    """A free-slip outer wall at a dt whose last matrix row is larger off the
+    diagonal than on it: dgttrf exchanges the last two rows."""
+    p = small_params(tc, 20, 9, nrm, ren=50.0)
+    am = tc.grid_vector(p, "am1j")[nrm - 1]
+    assert am * 0.5 * dt / p["ren"] * 8.0 / 15.0 > 1.0
+    _implicit(tc, oracle, p, dt, nrm)
+
+
+def _implicit(tc, oracle, p, dt, nrm):
+    dev, orc = tc.Solver(p), oracle.Oracle(p)
+    rng = np.random.default_rng(nrm)
+    masks = [rng.integers(0, 2, (p["nzm"], p["nthm"])).astype(np.int32) for _ in range(2)]
+    load_both(dev, orc, random_state(p, 5))
+    for s in (dev, orc):
+        s.set_time(0.3, dt)
+        s.begin_step()
+        s.set_masks(*masks)
+        s.set_substep(1)
+    for a, b in (("ImplicitAndUpdateQT", "implicit_and_update_qt"), ("ImplicitAndUpdateQR", "implicit_and_update_qr"),
+                 ("ImplicitAndUpdateQZ", "implicit_and_update_qz")):
+        getattr(dev, a)()
+        orc.call(b)
+    for f, sl in (("qt", slice(0, nrm)), ("qr", slice(0, nrm + 1)), ("qz", slice(0, nrm))):
+        assert rel_l2(dev.get(f)[sl], orc.get(f)[sl]) < 1e-10, f
