@@ -533,12 +533,21 @@ int tc_create_tuned(const tc_params *p, const tc_tuning *tun, tc_ctx **out) {
   // grid vectors
   {
     const tc::Grid &g = c->g;
+    // rows 1..nrm-1 of the (0,0) Poisson line: a x(k-1) + b x(k) + c x(k+1)
+    std::vector<double> grd((size_t)c->nr + 1, 0.0), glo(grd), gup(grd);
+    for (int k = 1; k < c->nrm; k++) {
+      const double b = g.acph[k] - g.ak3[1] - g.ak1[1] * (g.usrm[k] * g.usrm[k]);
+      grd[k] = 1.0 / (k > 1 ? b + g.amph[k] * gup[k - 1] : b);
+      glo[k] = k > 1 ? -g.amph[k] * grd[k] : 0.0;
+      gup[k] = -g.apph[k] * grd[k];
+    }
+    if (c->nrm > 1) gup[c->nrm - 1] = 0.0;
     const std::vector<double> *vs[] = {&g.rc,   &g.rm,    &g.usrc,  &g.usrm,  &g.udx2rm,
                                        &g.udx2m, &g.udx2c, &g.rudx2c, &g.udx1vis1, &g.udx1vis2,
                                        &g.udx1qm, &g.pvol, &g.ap1j,  &g.am1j,  &g.ac1j,
                                        &g.ap2je, &g.am2je, &g.ac2je, &g.ap3j,  &g.am3j,
                                        &g.ac3j,  &g.apph,  &g.amph,  &g.acph,  &g.ak1, &g.ak3,
-                                       &g.udx2mm, &g.udx2cc};
+                                       &g.udx2mm, &g.udx2cc, &grd, &glo, &gup};
     const int nv = (int)(sizeof vs / sizeof vs[0]);
     size_t stride = (size_t)std::max(c->nr, std::max(c->nthm, c->nzm)) + 2;
     stride = (stride + 7) / 8 * 8;  // keeps the plane records 64-byte aligned
@@ -581,7 +590,8 @@ int tc_create_tuned(const tc_params *p, const tc_tuning *tun, tc_ctx **out) {
                             &c->gd.udx1vis2, &c->gd.udx1qm, &c->gd.pvol, &c->gd.ap1j,
                             &c->gd.am1j, &c->gd.ac1j, &c->gd.ap2je, &c->gd.am2je, &c->gd.ac2je,
                             &c->gd.ap3j, &c->gd.am3j, &c->gd.ac3j, &c->gd.apph, &c->gd.amph,
-                            &c->gd.acph, &c->gd.ak1, &c->gd.ak3, &c->gd.udx2mm, &c->gd.udx2cc};
+                            &c->gd.acph, &c->gd.ak1, &c->gd.ak3, &c->gd.udx2mm, &c->gd.udx2cc,
+                            &c->gd.grd, &c->gd.glo, &c->gd.gup};
     for (int q = 0; q < nv; q++) *dst[q] = c->gvbuf + q * stride;
     c->gd.hp = reinterpret_cast<const tc::HelmPlane *>(c->gvbuf + stride * nv);
     c->gd.dxt = g.dxt;

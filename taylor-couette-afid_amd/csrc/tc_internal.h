@@ -39,6 +39,8 @@ struct GridDev {
   const double *ap1j, *am1j, *ac1j, *ap2je, *am2je, *ac2je, *ap3j, *am3j, *ac3j;
   const double *apph, *amph, *acph, *ak1, *ak3;
   const double *udx2mm, *udx2cc;  // statistics and dissipation only
+  // Thomas factors of the (0,0) Poisson line: x = d grd + glo x down, x += gup x up
+  const double *grd, *glo, *gup;
   double dxt, dxz, dxtq, dxzq, ren, romeg;
   double ap1j_fs2, ac1j_fs1, ac1j_fs2, am1j_fs1, ap3j_fs2, ac3j_fs1, ac3j_fs2, am3j_fs1;
   int nthm, nzm, nrm, nr, nth2, sstr;  // sstr: spectral row stride >= nth2
@@ -166,6 +168,7 @@ __device__ __forceinline__ GridDev glob(const GridDev &s) {
   g.ap3j = glob(g.ap3j), g.am3j = glob(g.am3j), g.ac3j = glob(g.ac3j);
   g.apph = glob(g.apph), g.amph = glob(g.amph), g.acph = glob(g.acph);
   g.ak1 = glob(g.ak1), g.ak3 = glob(g.ak3), g.udx2mm = glob(g.udx2mm), g.udx2cc = glob(g.udx2cc);
+  g.grd = glob(g.grd), g.glo = glob(g.glo), g.gup = glob(g.gup);
   return g;
 }
 __device__ __forceinline__ bool inst_stopped(const StepDesc &d) {

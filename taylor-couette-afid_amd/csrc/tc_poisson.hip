@@ -484,7 +484,12 @@ __global__ __launch_bounds__(NT) void k_fft_z_g(const StepDesc *__restrict__ tab
 //
 // The singular (0,0) Neumann mode is solved on rows 1..nrm-1 with
 // phi(nrm) = 0.  Its partitions are nearly singular, so block 0 stages that
-// one line in LDS and solves it with a serial Thomas sweep instead.
+// one line in LDS and solves it with a serial Thomas sweep instead.  Its
+// factors depend on the grid alone and come from a table made once, so the
+// sweep is one multiply-add a row from LDS.  (Forming them in the sweep, a
+// division and four dependent global loads a row, made this one line the
+// launch's critical path on all but the largest grids: 64x64x65 18 us,
+// 256x256x193 61 us.)
 //   blockDim = (LB lines, PT partitions)
 //   LDS = LB*2PT*4 doubles (reduced systems) + 3*nrm doubles (gauge line)
 //         + 4*nrm doubles (the radial coefficients amph, apph, acph, usrm^2)
@@ -501,9 +506,9 @@ DEVI void poisson_body(const long long blk, const GridDev &g, double2 *__restric
   const long long m = blk * LB + lx;
   const int n = g.nrm;
   const int LS = 2 * PT * 4 + 4;                                // padded line stride
-  double2 *gline = (double2 *)(red + (size_t)LB * LS);            // gauge line, n values
-  double *gcp = (double *)(gline + n);                          // its multipliers
-  double *cam = gcp + n, *cap = cam + n, *cac = cap + n, *cus = cac + n;  // row k at [k-1]
+  // gauge line, n values (real: the (0,0) mode of a real field is), and its factors
+  double *gline = red + (size_t)LB * LS, *glo = gline + n, *gup = glo + n;
+  double *cam = gup + n, *cap = cam + n, *cac = cap + n, *cus = cac + n;  // row k at [k-1]
   const bool gblock = (blk == 0);
   const int lo = (int)(((long long)pp * n) / PT), S = (int)(((long long)(pp + 1) * n) / PT) - lo;
   double ar[PQ], cr[PQ];
@@ -522,8 +527,9 @@ DEVI void poisson_body(const long long blk, const GridDev &g, double2 *__restric
   }
   if (gblock)
     for (int k = tid; k < n; k += nthr) {
-      const double2 v = spec[(long long)k * M];
-      gline[k] = make_double2(v.x * inv_norm, v.y * inv_norm);
+      gline[k] = spec[(long long)k * M].x * (g.grd[k + 1] * inv_norm);
+      glo[k] = g.glo[k + 1];
+      gup[k] = g.gup[k + 1];
     }
   // this line's wavenumber terms and the line-independent radial
   // coefficients, staged once per block: all loads issued before any wait
@@ -692,29 +698,41 @@ DEVI void poisson_body(const long long blk, const GridDev &g, double2 *__restric
   }
   }
   if (gblock && tid == nthr - 1) {
-    // gauge line: Thomas on rows 1..nrm-1 (b = acph there), phi(nrm) = 0
+    // gauge line: Thomas on rows 1..nrm-1, phi(nrm) = 0 (glo(1) = gup(nrm-1)
+    // = 0).  Rows are read a chunk ahead of the dependent sweep.
+    constexpr int CH = 8;
     const int nn = n - 1;
-    double b = g.acph[1] - g.ak3[1] - g.ak1[1] * (g.usrm[1] * g.usrm[1]);
-    double rden = 1.0 / b;
-    double cp = g.apph[1] * rden;
-    double2 dp = make_double2(gline[0].x * rden, gline[0].y * rden);
-    gcp[0] = cp;
-    gline[0] = dp;
-    for (int k = 2; k <= nn; k++) {
-      const double a = g.amph[k];
-      b = g.acph[k] - g.ak3[1] - g.ak1[1] * (g.usrm[k] * g.usrm[k]);
-      rden = 1.0 / (b - a * cp);
-      dp = make_double2((gline[k - 1].x - a * dp.x) * rden, (gline[k - 1].y - a * dp.y) * rden);
-      gline[k - 1] = dp;
-      cp = g.apph[k] * rden;
-      gcp[k - 1] = cp;
+    double x = 0.0;
+    for (int k0 = 0; k0 < nn; k0 += CH) {
+      double v[CH], m[CH];
+#pragma unroll
+      for (int u = 0; u < CH; u++) {
+        v[u] = gline[min(k0 + u, nn - 1)];
+        m[u] = glo[min(k0 + u, nn - 1)];
+      }
+#pragma unroll
+      for (int u = 0; u < CH; u++)
+        if (k0 + u < nn) {
+          x = v[u] + m[u] * x;
+          gline[k0 + u] = x;
+        }
     }
-    double2 x = dp;
-    for (int k = nn - 1; k >= 1; k--) {
-      x = make_double2(gline[k - 1].x - gcp[k - 1] * x.x, gline[k - 1].y - gcp[k - 1] * x.y);
-      gline[k - 1] = x;
+    x = 0.0;
+    for (int k0 = nn - 1; k0 >= 0; k0 -= CH) {
+      double v[CH], m[CH];
+#pragma unroll
+      for (int u = 0; u < CH; u++) {
+        v[u] = gline[max(k0 - u, 0)];
+        m[u] = gup[max(k0 - u, 0)];
+      }
+#pragma unroll
+      for (int u = 0; u < CH; u++)
+        if (k0 - u >= 0) {
+          x = v[u] + m[u] * x;
+          gline[k0 - u] = x;
+        }
     }
-    gline[n - 1] = make_double2(0.0, 0.0);
+    gline[n - 1] = 0.0;
   }
   __syncthreads();
   if (valid) {
@@ -733,7 +751,7 @@ DEVI void poisson_body(const long long blk, const GridDev &g, double2 *__restric
     }
   }
   if (gblock)
-    for (int k = tid; k < n; k += nthr) spec[(long long)k * M] = gline[k];
+    for (int k = tid; k < n; k += nthr) spec[(long long)k * M] = make_double2(gline[k], 0.0);
 }
 
 template <int PQ>
@@ -758,7 +776,7 @@ __global__ __launch_bounds__(512) void k_poisson_tridiag_g(const StepDesc *__res
 // 594 (512); at 1024x1024x769, 26 rows, 3261 us against 4267 (128) and 3982
 // (512).
 // Dynamic LDS of k_poisson_tridiag: the padded reduced systems of lb lines
-// plus the gauge line (2n), its multipliers (n) and four coefficient tables.
+// plus the gauge line (n), its factors (2n) and four coefficient tables.
 size_t poisson_lds_doubles(int pt, int lb, int n) {
   return (size_t)lb * (2 * (size_t)pt * 4 + 4) + 7 * (size_t)n;
 }
