@@ -645,8 +645,7 @@ int tc_create_tuned(const tc_params *p, const tc_tuning *tun, tc_ctx **out) {
     HTRY(hipStreamSynchronize(c->stream));
   }
   // reductions
-  // per-block partials of the reductions: one block of 256 per (j, i) column group
-  c->red_cap = 40 * (size_t)((c->P + 255) / 256);
+  c->red_cap = tc::reduction_doubles(c);  // per-block partials
   TRY(dev_alloc(c, (void **)&c->red, sizeof(double) * c->red_cap));
   TRY(dev_alloc(c, (void **)&c->red_out, sizeof(double) * 16));
   HTRY(hipHostMalloc((void **)&c->red_host, sizeof(double) * 16, hipHostMallocDefault));

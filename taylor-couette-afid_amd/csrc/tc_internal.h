@@ -211,8 +211,8 @@ struct tc_ctx {
   // reductions
   double *red = nullptr;        // device partials
   size_t red_cap = 0;           // their capacity in doubles
-  double *red_out = nullptr;    // device results (16)
-  double *red_host = nullptr;   // pinned copy of red_out
+  double *red_out = nullptr;    // device results (16) of the grouped launches
+  double *red_host = nullptr;   // pinned host results (16), written by the kernels
   int red_blocks = 0;
   // scalars of module param
   double time = 0, dt = 0, beta = 0, al = 0, ga = 0, ro = 0, vinner_t = 0, dvinner_t = 0;
@@ -269,7 +269,8 @@ void launch_correct_velocity(tc_ctx *c, double aldt);
 void launch_correct_pressure(tc_ctx *c);
 void launch_correct_both(tc_ctx *c);
 void launch_zero_wall_qr(tc_ctx *c);
-// reductions: results land in c->red_out and are copied to c->red_host
+// reductions: results land in c->red_host
+size_t reduction_doubles(const tc_ctx *c);
 void launch_max_cfl(tc_ctx *c);
 void launch_max_div(tc_ctx *c);
 void launch_torque(tc_ctx *c);

@@ -5,6 +5,7 @@
 // r-plane k (1-based, k = 1..nr) at offset (k-1)*P, P = nzm*nthm.  The
 // reference's periodic halos (InitVariables.F90:26-35, halo_common.f90:67-108)
 // become index wrap-around, so no halo update is ever launched.
+#include <algorithm>
 #include <map>
 #include <mutex>
 
@@ -1476,6 +1477,8 @@ void launch_zero_wall_qr(tc_ctx *c) {
 // ---------------------------------------------------------------------------
 
 constexpr int RED_THREADS = 256;
+constexpr int RED_TARGET = 1024;    // blocks of a column reduction that fill the device
+constexpr int CDIAG_TARGET = 1536;  // blocks of the fused last correction
 
 template <int NV>
 DEVI void block_reduce(double (&v)[NV], const int *ops /*0 sum, 1 max*/, double *out) {
@@ -1505,14 +1508,19 @@ DEVI void block_reduce(double (&v)[NV], const int *ops /*0 sum, 1 max*/, double 
 
 // Point reductions march along r: thread = (j, i) column, k = 1..nrm, so the
 // qr(k+1) plane of one step is the qr(k) plane of the next.
+// Block blk of nb * nseg owns 256 columns over segment blk / nb of r.
 struct Col {
   long long l;
   long long lip, ljp;  // in-plane offsets of (j, i+1) and (j+1, i)
+  int k0, k1;          // planes of the segment
   bool ok;
 };
-DEVI Col column(const GridDev &g, long long blk) {
+DEVI Col column(const GridDev &g, int blk, int nseg) {
   Col c;
-  c.l = blk * blockDim.x + threadIdx.x;
+  const int nb = (int)((g.P + RED_THREADS - 1) / RED_THREADS), seg = blk / nb;
+  c.k0 = seg_first(seg, nseg, g.nrm);
+  c.k1 = seg_first(seg + 1, nseg, g.nrm) - 1;
+  c.l = (long long)(blk - seg * nb) * RED_THREADS + threadIdx.x;
   c.ok = c.l < g.P;
   const long long l = c.ok ? c.l : 0;
   const int j = (int)(l / g.nthm), i = (int)(l - (long long)j * g.nthm);
@@ -1523,25 +1531,27 @@ DEVI Col column(const GridDev &g, long long blk) {
 
 // CalcMaxCFL.F90:30-43 (WHICH 0) and CheckDivergence.F90:28-40 (WHICH 1)
 template <int WHICH>
-DEVI void pointmax_body(const int blk, const GridDev &g, const double *__restrict__ qt,
+DEVI void pointmax_body(const int blk, const int nseg, const GridDev &g, const double *__restrict__ qt,
                         const double *__restrict__ qr, const double *__restrict__ qz,
                         double *__restrict__ part) {
 #pragma clang fp contract(off)
   double m[1] = {0.0};
-  const Col c = column(g, blk);
+  const Col c = column(g, blk, nseg);
   if (c.ok) {
-    double r_c = qr[c.l];
-    for (int kc = 1; kc <= g.nrm; kc++) {
+    double r_c = qr[(long long)(c.k0 - 1) * g.P + c.l];
+#pragma unroll 2
+    for (int kc = c.k0; kc <= c.k1; kc++) {
       const long long b = (long long)(kc - 1) * g.P;
       const double t_c = qt[b + c.l], t_ip = qt[b + c.lip];
       const double r_kp = qr[b + g.P + c.l];
       const double z_c = qz[b + c.l], z_jp = qz[b + c.ljp];
       double val;
       if (WHICH == 0)
-        val = (fabs((t_ip + t_c) * 0.5 * g.dxt * g.usrm[kc]) + fabs((r_kp + r_c) * 0.5 * g.udx2rm[kc]) +
-               fabs((z_jp + z_c) * 0.5 * g.dxz));
+        val = (fabs((t_ip + t_c) * 0.5 * g.dxt * ldk(g.usrm + kc)) +
+               fabs((r_kp + r_c) * 0.5 * ldk(g.udx2rm + kc)) + fabs((z_jp + z_c) * 0.5 * g.dxz));
       else
-        val = fabs(((t_ip - t_c) * g.dxt + (r_kp - r_c) * g.udx2m[kc]) * g.usrm[kc] + (z_jp - z_c) * g.dxz);
+        val = fabs(((t_ip - t_c) * g.dxt + (r_kp - r_c) * ldk(g.udx2m + kc)) * ldk(g.usrm + kc) +
+                   (z_jp - z_c) * g.dxz);
       m[0] = fmax(m[0], val);
       r_c = r_kp;
     }
@@ -1554,15 +1564,16 @@ template <int WHICH>
 __global__ __launch_bounds__(RED_THREADS) void k_pointmax(GridDev g, const double *__restrict__ qt,
                                                          const double *__restrict__ qr,
                                                          const double *__restrict__ qz,
-                                                         double *__restrict__ part) {
-  pointmax_body<WHICH>(blockIdx.x, g, qt, qr, qz, part);
+                                                         double *__restrict__ part, int nseg) {
+  pointmax_body<WHICH>(blockIdx.x, nseg, g, qt, qr, qz, part);
 }
 
 // Grouped CalcMaxCFL partials: blockIdx.y = instance.
-__global__ __launch_bounds__(RED_THREADS) void k_pointmax_cfl_g(const StepDesc *__restrict__ tab) {
+__global__ __launch_bounds__(RED_THREADS) void k_pointmax_cfl_g(const StepDesc *__restrict__ tab,
+                                                               int nseg) {
   const StepDesc &d = tab[blockIdx.y];
   if (inst_stopped(d)) return;
-  pointmax_body<0>(blockIdx.x, glob(d.g), glob(d.f[TC_QT]), glob(d.f[TC_QR]), glob(d.f[TC_QZ]),
+  pointmax_body<0>(blockIdx.x, nseg, glob(d.g), glob(d.f[TC_QT]), glob(d.f[TC_QR]), glob(d.f[TC_QZ]),
                    glob(d.red));
 }
 
@@ -1591,12 +1602,14 @@ __global__ __launch_bounds__(RED_THREADS) void k_torque(GridDev g, const double 
 __global__ __launch_bounds__(RED_THREADS) void k_velstats(GridDev g, const double *__restrict__ qt,
                                                          const double *__restrict__ qr,
                                                          const double *__restrict__ qz,
-                                                         double pi, double *__restrict__ part) {
+                                                         double pi, double *__restrict__ part,
+                                                         int nseg) {
   double v[6] = {-100.0, -100.0, -100.0, 0.0, 0.0, 0.0};
-  const Col c = column(g, blockIdx.x);
+  const Col c = column(g, blockIdx.x, nseg);
   if (c.ok) {
-    double r_c = qr[c.l];
-    for (int kc = 1; kc <= g.nrm; kc++) {
+    double r_c = qr[(long long)(c.k0 - 1) * g.P + c.l];
+#pragma unroll 2
+    for (int kc = c.k0; kc <= c.k1; kc++) {
       const long long b = (long long)(kc - 1) * g.P;
       const double a = qt[b + c.l], cz = qz[b + c.l];
       const double r_kp = qr[b + g.P + c.l];
@@ -1604,11 +1617,11 @@ __global__ __launch_bounds__(RED_THREADS) void k_velstats(GridDev g, const doubl
       v[1] = fmax(v[1], fabs(r_c));
       v[2] = fmax(v[2], fabs(cz));
       const double t = a + qt[b + c.lip];
-      v[3] += t * t * g.pvol[kc] * pi * 0.25;
-      const double u = r_c * g.usrc[kc] + r_kp * g.usrc[kc + 1];
-      v[4] += u * u * g.pvol[kc] * pi * 0.25;
+      v[3] += t * t * ldk(g.pvol + kc) * pi * 0.25;
+      const double u = r_c * ldk(g.usrc + kc) + r_kp * ldk(g.usrc + kc + 1);
+      v[4] += u * u * ldk(g.pvol + kc) * pi * 0.25;
       const double w = cz + qz[b + c.ljp];
-      v[5] += w * w * g.pvol[kc] * pi * 0.25;
+      v[5] += w * w * ldk(g.pvol + kc) * pi * 0.25;
       r_c = r_kp;
     }
   }
@@ -1693,25 +1706,40 @@ __global__ void k_diag_store_g(const StepDesc *__restrict__ tab, const BatchDyn 
 
 static unsigned red_blocks(const tc_ctx *c) { return (unsigned)((c->P + RED_THREADS - 1) / RED_THREADS); }
 
-static void finish_reduction(tc_ctx *c, int nv, unsigned opmask) {
-  hipLaunchKernelGGL(k_combine, dim3((unsigned)nv), dim3(256), 0, c->stream, c->red, (int)red_blocks(c),
-                     nv, opmask, c->red_out);
-  hipMemcpyAsync(c->red_host, c->red_out, sizeof(double) * (size_t)nv, hipMemcpyDeviceToHost,
-                 c->stream);
+// r segments of a column reduction: about four blocks per CU in all, at
+// least four planes each.  (One segment: 64x64x65 runs 16 blocks that march
+// 65 planes each, 14-18 us a pass over 6 MB.)
+static int red_segments(const tc_ctx *c) {
+  const int nb = (int)red_blocks(c);
+  return std::max(1, std::min(RED_TARGET / nb, c->nrm / 4));
+}
+
+size_t reduction_doubles(const tc_ctx *c) {
+  const size_t cols = (size_t)((c->nthm / 2 + 63) / 64) * ((c->nzm + 3) / 4);
+  return 10 * std::max({(size_t)red_blocks(c), cols, (size_t)RED_TARGET, (size_t)CDIAG_TARGET + cols});
+}
+
+// The results go to pinned host memory (coherent), which the host reads
+// after the stream has drained: no copy is queued behind the kernel.
+static void finish_reduction(tc_ctx *c, unsigned nb, int nv, unsigned opmask) {
+  hipLaunchKernelGGL(k_combine, dim3((unsigned)nv), dim3(256), 0, c->stream, c->red, (int)nb, nv,
+                     opmask, c->red_host);
 }
 
 void launch_max_cfl(tc_ctx *c) {
   timer_begin(c, "max_cfl");
-  hipLaunchKernelGGL(k_pointmax<0>, dim3(red_blocks(c)), dim3(RED_THREADS), 0, c->stream, c->gd,
-                     c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->red);
-  finish_reduction(c, 1, 1u);
+  const int ns = red_segments(c);
+  hipLaunchKernelGGL(k_pointmax<0>, dim3(red_blocks(c) * ns), dim3(RED_THREADS), 0, c->stream, c->gd,
+                     c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->red, ns);
+  finish_reduction(c, red_blocks(c) * ns, 1, 1u);
   timer_end(c);
 }
 void launch_max_div(tc_ctx *c) {
   timer_begin(c, "max_div");
-  hipLaunchKernelGGL(k_pointmax<1>, dim3(red_blocks(c)), dim3(RED_THREADS), 0, c->stream, c->gd,
-                     c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->red);
-  finish_reduction(c, 1, 1u);
+  const int ns = red_segments(c);
+  hipLaunchKernelGGL(k_pointmax<1>, dim3(red_blocks(c) * ns), dim3(RED_THREADS), 0, c->stream, c->gd,
+                     c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->red, ns);
+  finish_reduction(c, red_blocks(c) * ns, 1, 1u);
   timer_end(c);
 }
 // ---------------------------------------------------------------------------
@@ -1764,9 +1792,11 @@ int check_divergence_noalloc(tc_ctx *c, double *qmax_dev) {
   double *part = nullptr;
   int rc = scratch_on(c->device, &part);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_pointmax<1>, dim3(nb), dim3(RED_THREADS), 0, c->stream, c->gd, c->f[TC_QT],
-                     c->f[TC_QR], c->f[TC_QZ], part);
-  hipLaunchKernelGGL(k_combine, dim3(1u), dim3(256), 0, c->stream, part, (int)nb, 1, 1u, qmax_dev);
+  const int ns = red_segments(c);  // nb * ns stays within the larger of nb and RED_TARGET
+  hipLaunchKernelGGL(k_pointmax<1>, dim3(nb * ns), dim3(RED_THREADS), 0, c->stream, c->gd,
+                     c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], part, ns);
+  hipLaunchKernelGGL(k_combine, dim3(1u), dim3(256), 0, c->stream, part, (int)(nb * ns), 1, 1u,
+                     qmax_dev);
   return check_launch();
 }
 
@@ -1776,12 +1806,13 @@ void launch_torque(tc_ctx *c) {
   hipLaunchKernelGGL(k_torque, dim3(red_blocks(c)), dim3(RED_THREADS), 0, c->stream, c->gd,
                      c->f[TC_QT], c->mask, c->mask + c->P, c->p.virotint, c->p.virotext, del,
                      deln, c->red);
-  finish_reduction(c, 2, 0u);
+  finish_reduction(c, red_blocks(c), 2, 0u);
 }
 void launch_velocity_stats(tc_ctx *c) {
-  hipLaunchKernelGGL(k_velstats, dim3(red_blocks(c)), dim3(RED_THREADS), 0, c->stream, c->gd,
-                     c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->g.pi, c->red);
-  finish_reduction(c, 6, 7u);
+  const int ns = red_segments(c);
+  hipLaunchKernelGGL(k_velstats, dim3(red_blocks(c) * ns), dim3(RED_THREADS), 0, c->stream, c->gd,
+                     c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->g.pi, c->red, ns);
+  finish_reduction(c, red_blocks(c) * ns, 6, 7u);
 }
 
 // One pass over the velocity for the logging step of main.F90:180-186:
@@ -1789,7 +1820,7 @@ void launch_velocity_stats(tc_ctx *c) {
 // CalcVelocityStats (CalcVelocityStats.F90:35-44) and CalcTorque
 // (CalcTorque.F90:38-43).  v = cfl, |div|, vmax1..3, rms sums 1..3,
 // torque sums inner/outer.
-DEVI void diagnostics_body(const int blk, const GridDev &g, const double *__restrict__ qt,
+DEVI void diagnostics_body(const int blk, const int nseg, const GridDev &g, const double *__restrict__ qt,
                            const double *__restrict__ qr, const double *__restrict__ qz,
                            const unsigned char *__restrict__ icyl,
                            const unsigned char *__restrict__ ocyl, double virotint,
@@ -1799,28 +1830,29 @@ DEVI void diagnostics_body(const int blk, const GridDev &g, const double *__rest
   // correction pass (correct_diag_body) and of the CFL pass bit for bit
 #pragma clang fp contract(off)
   double v[10] = {0.0, 0.0, -100.0, -100.0, -100.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  const Col c = column(g, blk);
+  const Col c = column(g, blk, nseg);
   if (c.ok) {
-    double r_c = qr[c.l], t_prev = 0.0;
-    for (int kc = 1; kc <= g.nrm; kc++) {
+    const long long b0 = (long long)(c.k0 - 1) * g.P;
+    double r_c = qr[b0 + c.l], t_prev = c.k0 > 1 ? qt[b0 - g.P + c.l] : 0.0;
+    for (int kc = c.k0; kc <= c.k1; kc++) {
       const long long b = (long long)(kc - 1) * g.P;
       const double t_c = qt[b + c.l], t_ip = qt[b + c.lip];
       const double r_kp = qr[b + g.P + c.l];
       const double z_c = qz[b + c.l], z_jp = qz[b + c.ljp];
-      const double cfl = (fabs((t_ip + t_c) * 0.5 * g.dxt * g.usrm[kc]) +
-                          fabs((r_kp + r_c) * 0.5 * g.udx2rm[kc]) + fabs((z_jp + z_c) * 0.5 * g.dxz));
-      const double dv = ((t_ip - t_c) * g.dxt + (r_kp - r_c) * g.udx2m[kc]) * g.usrm[kc] + (z_jp - z_c) * g.dxz;
+      const double cfl = (fabs((t_ip + t_c) * 0.5 * g.dxt * ldk(g.usrm + kc)) +
+                          fabs((r_kp + r_c) * 0.5 * ldk(g.udx2rm + kc)) + fabs((z_jp + z_c) * 0.5 * g.dxz));
+      const double dv = ((t_ip - t_c) * g.dxt + (r_kp - r_c) * ldk(g.udx2m + kc)) * ldk(g.usrm + kc) + (z_jp - z_c) * g.dxz;
       v[0] = fmax(v[0], cfl);
       v[1] = fmax(v[1], fabs(dv));
       v[2] = fmax(v[2], fabs(t_c));
       v[3] = fmax(v[3], fabs(r_c));
       v[4] = fmax(v[4], fabs(z_c));
       const double t = t_c + t_ip;
-      v[5] += t * t * g.pvol[kc] * pi * 0.25;
-      const double u = r_c * g.usrc[kc] + r_kp * g.usrc[kc + 1];
-      v[6] += u * u * g.pvol[kc] * pi * 0.25;
+      v[5] += t * t * ldk(g.pvol + kc) * pi * 0.25;
+      const double u = r_c * ldk(g.usrc + kc) + r_kp * ldk(g.usrc + kc + 1);
+      v[6] += u * u * ldk(g.pvol + kc) * pi * 0.25;
       const double w = z_c + z_jp;
-      v[7] += w * w * g.pvol[kc] * pi * 0.25;
+      v[7] += w * w * ldk(g.pvol + kc) * pi * 0.25;
       if (kc == 2) {
         const double grtlow = ((t_c * g.usrm[2] + t_prev * g.usrm[1]) * 0.5 - virotint * g.usrc[1]) * del;
         v[8] += grtlow * (double)icyl[c.l];
@@ -1841,18 +1873,19 @@ __global__ __launch_bounds__(RED_THREADS) void k_diagnostics(
     GridDev g, const double *__restrict__ qt, const double *__restrict__ qr,
     const double *__restrict__ qz, const unsigned char *__restrict__ icyl,
     const unsigned char *__restrict__ ocyl, double virotint, double virotext, double del,
-    double deln, double pi, double *__restrict__ part) {
-  diagnostics_body(blockIdx.x, g, qt, qr, qz, icyl, ocyl, virotint, virotext, del, deln, pi, part);
+    double deln, double pi, double *__restrict__ part, int nseg) {
+  diagnostics_body(blockIdx.x, nseg, g, qt, qr, qz, icyl, ocyl, virotint, virotext, del, deln, pi, part);
 }
 
 // Grouped logging pass: blockIdx.y = instance; instances not logging this
 // step leave at once.
 __global__ __launch_bounds__(RED_THREADS) void k_diagnostics_g(const StepDesc *__restrict__ tab,
-                                                              const BatchDyn *__restrict__ dyn) {
+                                                              const BatchDyn *__restrict__ dyn,
+                                                              int nseg) {
   if (!dyn[blockIdx.y].log) return;
   const StepDesc &d = tab[blockIdx.y];
   if (inst_stopped(d)) return;
-  diagnostics_body(blockIdx.x, glob(d.g), glob(d.f[TC_QT]), glob(d.f[TC_QR]), glob(d.f[TC_QZ]),
+  diagnostics_body(blockIdx.x, nseg, glob(d.g), glob(d.f[TC_QT]), glob(d.f[TC_QR]), glob(d.f[TC_QZ]),
                    glob(d.icyl), glob(d.ocyl), d.virotint, d.virotext, d.del, d.deln, d.pi,
                    glob(d.red));
 }
@@ -1861,10 +1894,11 @@ void launch_diagnostics(tc_ctx *c) {
   const double del = -1.0 / (c->g.rc[2] - c->g.rc[1]);
   const double deln = -1.0 / (c->g.rc[c->nr] - c->g.rc[c->nrm]);
   timer_begin(c, "diagnostics");
-  hipLaunchKernelGGL(k_diagnostics, dim3(red_blocks(c)), dim3(RED_THREADS), 0, c->stream, c->gd,
+  const int ns = red_segments(c);
+  hipLaunchKernelGGL(k_diagnostics, dim3(red_blocks(c) * ns), dim3(RED_THREADS), 0, c->stream, c->gd,
                      c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->mask, c->mask + c->P,
-                     c->p.virotint, c->p.virotext, del, deln, c->g.pi, c->red);
-  finish_reduction(c, 10, 0x1Fu);
+                     c->p.virotint, c->p.virotext, del, deln, c->g.pi, c->red, ns);
+  finish_reduction(c, red_blocks(c) * ns, 10, 0x1Fu);
   timer_end(c);
 }
 
@@ -1985,21 +2019,21 @@ DEVI void correct_diag_body(const int bx, const int by, const int seg, const int
         for (int e = 0; e < 2; e++) {
           const double t_c = tt[e], t_ip = tip[e], r_c = rr[e], r_kp = rp[e], z_c = zz[e],
                        z_jp = zp[e];
-          const double cfl = (fabs((t_ip + t_c) * 0.5 * g.dxt * g.usrm[kc]) +
-                              fabs((r_kp + r_c) * 0.5 * g.udx2rm[kc]) + fabs((z_jp + z_c) * 0.5 * g.dxz));
+          const double cfl = (fabs((t_ip + t_c) * 0.5 * g.dxt * ldk(g.usrm + kc)) +
+                              fabs((r_kp + r_c) * 0.5 * ldk(g.udx2rm + kc)) + fabs((z_jp + z_c) * 0.5 * g.dxz));
           const double dv =
-              ((t_ip - t_c) * g.dxt + (r_kp - r_c) * g.udx2m[kc]) * g.usrm[kc] + (z_jp - z_c) * g.dxz;
+              ((t_ip - t_c) * g.dxt + (r_kp - r_c) * ldk(g.udx2m + kc)) * ldk(g.usrm + kc) + (z_jp - z_c) * g.dxz;
           v[0] = fmax(v[0], cfl);
           v[1] = fmax(v[1], fabs(dv));
           v[2] = fmax(v[2], fabs(t_c));
           v[3] = fmax(v[3], fabs(r_c));
           v[4] = fmax(v[4], fabs(z_c));
           const double tsum = t_c + t_ip;
-          v[5] += tsum * tsum * g.pvol[kc] * pi * 0.25;
-          const double u = r_c * g.usrc[kc] + r_kp * g.usrc[kc + 1];
-          v[6] += u * u * g.pvol[kc] * pi * 0.25;
+          v[5] += tsum * tsum * ldk(g.pvol + kc) * pi * 0.25;
+          const double u = r_c * ldk(g.usrc + kc) + r_kp * ldk(g.usrc + kc + 1);
+          v[6] += u * u * ldk(g.pvol + kc) * pi * 0.25;
           const double w = z_c + z_jp;
-          v[7] += w * w * g.pvol[kc] * pi * 0.25;
+          v[7] += w * w * ldk(g.pvol + kc) * pi * 0.25;
           if (kc == 2) {
             const double grtlow = ((t_c * g.usrm[2] + tpv[e] * g.usrm[1]) * 0.5 - virotint * g.usrc[1]) * del;
             v[8] += grtlow * (double)icyl[l + e];
@@ -2042,17 +2076,23 @@ __global__ __launch_bounds__(256) void k_correct_diag(
 
 // Segments of r per column: enough blocks for about six per CU (at
 // 512x512x385 three segments of 129 planes ran 1.46-1.51 ms against 1.81 ms
-// for two and 1.56-1.61 ms for four to twelve), each segment at least 16
-// planes, and the partials within the reduction buffer (TC_CDIAG_SEG
-// overrides).
+// for two and 1.56-1.61 ms for four to twelve) of at least 24 planes
+// (256x256x193: 178 us with 8 segments, 195 with 12), or down to four planes
+// while there are fewer than two blocks per CU (64x64x65: 19 us with 16
+// segments, 24 with 8, 36 with 4), and the partials within the reduction
+// buffer (TC_CDIAG_SEG overrides).
 int correct_diag_segments(const tc_ctx *c) {
   const long long cols = (long long)((c->nthm / 2 + 63) / 64) * ((c->nzm + 3) / 4);
   static const int env = [] {
     const char *e = std::getenv("TC_CDIAG_SEG");
     return e ? std::atoi(e) : 0;
   }();
-  long long s = env > 0 ? env : (1536 + cols - 1) / cols;
-  s = std::min<long long>(s, std::max(1, c->nrm / 16));
+  long long s = env > 0 ? env : (CDIAG_TARGET + cols - 1) / cols;
+  if (env <= 0) {
+    s = std::min<long long>(s, std::max(1, c->nrm / 24));
+    if (s * cols < 512) s = std::max<long long>(s, std::min<long long>(512 / cols, c->nrm / 4));
+  }
+  s = std::min<long long>(s, c->nrm);
   s = std::min<long long>(s, (long long)c->red_cap / (10 * cols));
   return (int)std::max<long long>(s, 1);
 }
@@ -2075,8 +2115,7 @@ void launch_correct_diag(tc_ctx *c) {
   std::swap(c->f[TC_QR], c->f[TC_DQ]);
   std::swap(c->f[TC_QZ], c->f[TC_QCAP]);
   hipLaunchKernelGGL(k_combine, dim3(10u), dim3(256), 0, c->stream, c->red, (int)grid.x, 10,
-                     0x1Fu, c->red_out);
-  hipMemcpyAsync(c->red_host, c->red_out, sizeof(double) * 10, hipMemcpyDeviceToHost, c->stream);
+                     0x1Fu, c->red_host);
   timer_end(c);
 }
 
@@ -2191,8 +2230,9 @@ void launch_correct_both_g(tc_ctx *c, const StepDesc *tab, int n, hipStream_t st
 
 void launch_cfl_check_g(tc_ctx *c, const StepDesc *tab, const BatchDyn *dyn, BatchRes *res, int n,
                         hipStream_t st) {
-  const unsigned nb = red_blocks(c);
-  hipLaunchKernelGGL(k_pointmax_cfl_g, dim3(nb, (unsigned)n), dim3(RED_THREADS), 0, st, tab);
+  const int ns = red_segments(c);
+  const unsigned nb = red_blocks(c) * ns;
+  hipLaunchKernelGGL(k_pointmax_cfl_g, dim3(nb, (unsigned)n), dim3(RED_THREADS), 0, st, tab, ns);
   hipLaunchKernelGGL(k_combine_g, dim3(1, (unsigned)n), dim3(256), 0, st, tab,
                      (const BatchDyn *)nullptr, (int)nb, 1, 1u);
   hipLaunchKernelGGL(k_cfl_check_g, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, st, tab, dyn, res,
@@ -2201,8 +2241,9 @@ void launch_cfl_check_g(tc_ctx *c, const StepDesc *tab, const BatchDyn *dyn, Bat
 
 void launch_diagnostics_g(tc_ctx *c, const StepDesc *tab, const BatchDyn *dyn, BatchRes *res, int n,
                           hipStream_t st) {
-  const unsigned nb = red_blocks(c);
-  hipLaunchKernelGGL(k_diagnostics_g, dim3(nb, (unsigned)n), dim3(RED_THREADS), 0, st, tab, dyn);
+  const int ns = red_segments(c);
+  const unsigned nb = red_blocks(c) * ns;
+  hipLaunchKernelGGL(k_diagnostics_g, dim3(nb, (unsigned)n), dim3(RED_THREADS), 0, st, tab, dyn, ns);
   hipLaunchKernelGGL(k_combine_g, dim3(10, (unsigned)n), dim3(256), 0, st, tab, dyn, (int)nb, 10,
                      0x1Fu);
   hipLaunchKernelGGL(k_diag_store_g, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, st, tab, dyn,

@@ -245,8 +245,7 @@ void launch_stats(tc_ctx *c, bool stats, bool diss) {
                        c->stat_part, ren);
   if (diss) {
     hipLaunchKernelGGL(k_sum_fixed, dim3(1), dim3(256), 0, c->stream, c->stat_part,
-                       (long long)c->nrm * c->nzm, c->red_out);
-    hipMemcpyAsync(c->red_host, c->red_out, sizeof(double), hipMemcpyDeviceToHost, c->stream);
+                       (long long)c->nrm * c->nzm, c->red_host);
   }
   timer_end(c);
 }
