@@ -397,13 +397,12 @@ DEVI double rlane(double v, int i) {
   return r.d;
 }
 
-// comp: 0 q_theta, 1 q_r (rows 2..nrm; both walls are set to zero), 2 q_z
+// comp: 0 q_theta, 1 q_r (rows 2..nrm; both walls are set to zero), 2 q_z.
+// lu: the line's table, the same for all lines of the block with UNIFORM.
 template <int R, bool UNIFORM, bool FOLD>
-DEVI void helm_solve_body(const long long lgrp, const int comp, const GridDev &g,
-                          double *__restrict__ q, const double *__restrict__ y,
-                          const unsigned char *__restrict__ icyl,
-                          const unsigned char *__restrict__ ocyl, const double *__restrict__ lu,
-                          int nt, double *ex) {
+DEVI void helm_solve_lines(const long long lgrp, const int comp, const GridDev &g,
+                           double *__restrict__ q, const double *__restrict__ y,
+                           const double *__restrict__ lu, double *ex) {
   const int lane = threadIdx.x, NS = blockDim.y;
   const int p = __builtin_amdgcn_readfirstlane(threadIdx.y);
   const long long P = g.P, l = lgrp * 64 + lane;
@@ -411,25 +410,36 @@ DEVI void helm_solve_body(const long long lgrp, const int comp, const GridDev &g
   const long long lc = ok ? l : P - 1;
   const int first = comp == 1 ? 1 : 0, n = g.nrm - first, last = first + n - 1;
   const int lo = first + p * n / NS, S = first + (p + 1) * n / NS - lo;
-  double v[R];
-  {
-    const double *yp = y + (long long)lo * P + lc;
-#pragma unroll
-    for (int i = 0; i < R; i++) v[i] = ld_nt(yp + (long long)min(i, S - 1) * P);
-  }
-  const int var = comp == 1 ? 0 : (UNIFORM ? 3 : icyl[lc] + 2 * ocyl[lc]);
-  const LUView T = lu_view(lu + (size_t)var * nt);
+  const LUView T = lu_view(lu);
   // -dl_(r-1), rd_r and -du_r rd_r of row lo + i (UNIFORM: of rows lo + lane
-  // and, past 64 rows, lo + 64 + lane)
+  // and, past 64 rows, lo + 64 + lane, loaded before the rows so that their
+  // latency is not behind them).  Past the segment's S rows they are those
+  // of rows that pass a value on unchanged in both sweeps (right-hand side
+  // zero), so the sweeps carry no conditions.
   constexpr int NK = (R + 63) / 64;
   double kdl[NK], kdu[NK], krd[NK];
   if constexpr (UNIFORM) {
 #pragma unroll
     for (int u = 0; u < NK; u++) {
       const int r = lo + min(lane + 64 * u, S - 1);
-      kdl[u] = r > first ? -T.dl(r - 1) : 0.0;
+      kdl[u] = T.dl(max(r - 1, 0));
+      kdu[u] = T.du(r);
       krd[u] = T.rd(r);
-      kdu[u] = r < last ? -T.du(r) * krd[u] : 0.0;
+    }
+  }
+  double v[R];
+  {
+    const double *yp = y + (long long)lo * P + lc;
+#pragma unroll
+    for (int i = 0; i < R; i++) v[i] = ld_nt(yp + (long long)min(i, S - 1) * P);
+  }
+  if constexpr (UNIFORM) {
+#pragma unroll
+    for (int u = 0; u < NK; u++) {
+      const int i = lane + 64 * u, r = lo + i;
+      kdl[u] = i < S ? (r > first ? -kdl[u] : 0.0) : 1.0;
+      kdu[u] = i < S ? (r < last ? -kdu[u] * krd[u] : 0.0) : 1.0;
+      krd[u] = i < S ? krd[u] : 0.0;
     }
   }
   auto dl = [&](int i) {
@@ -447,53 +457,75 @@ DEVI void helm_solve_body(const long long lgrp, const int comp, const GridDev &g
   double *exc = ex, *exw = ex + NS * 64;  // outgoing values and factors
   double c = 0.0, w = 1.0;
 #pragma unroll
-  for (int i = 0; i < R; i++)
-    if (i < S) {
-      const double d = dl(i);
-      c = v[i] + d * c;
-      v[i] = c;
-      w = w * d;
-    }
+  for (int i = 0; i < R; i++) {
+    if (!UNIFORM && i >= S) continue;
+    const double d = dl(i);
+    c = (i < S ? v[i] : 0.0) + d * c;
+    v[i] = c;
+    w = w * d;
+  }
   exc[p * 64 + lane] = c;
   exw[p * 64 + lane] = w;
   __syncthreads();
   w = 0.0;
   for (int s = 0; s < p; s++) w = exc[s * 64 + lane] + exw[s * 64 + lane] * w;
 #pragma unroll
-  for (int i = 0; i < R; i++)
-    if (i < S) {
-      w = w * dl(i);
-      v[i] = v[i] + w;
-    }
+  for (int i = 0; i < R; i++) {
+    if (!UNIFORM && i >= S) continue;
+    w = w * dl(i);
+    v[i] = v[i] + w;
+  }
   exc += 2 * NS * 64;
   exw += 2 * NS * 64;
   c = 0.0;
   w = 1.0;
 #pragma unroll
-  for (int i = R - 1; i >= 0; i--)
-    if (i < S) {
-      const double u = ud(i);
-      c = v[i] * rd(i) + u * c;
-      v[i] = c;
-      w = w * u;
-    }
+  for (int i = R - 1; i >= 0; i--) {
+    if (!UNIFORM && i >= S) continue;
+    const double u = ud(i);
+    c = v[i] * rd(i) + u * c;
+    v[i] = c;
+    w = w * u;
+  }
   exc[p * 64 + lane] = c;
   exw[p * 64 + lane] = w;
   __syncthreads();
   w = 0.0;
   for (int s = NS - 1; s > p; s--) w = exc[s * 64 + lane] + exw[s * 64 + lane] * w;
-  if (!ok) return;
   double *qp = q + (long long)lo * P + l;
 #pragma unroll
-  for (int i = R - 1; i >= 0; i--)
-    if (i < S) {
-      w = w * ud(i);
+  for (int i = R - 1; i >= 0; i--) {
+    if (!UNIFORM && i >= S) continue;
+    w = w * ud(i);
+    if (i < S && ok) {
       double *o = qp + (long long)i * P;
       st_nt(o, FOLD ? v[i] + w : *o + (v[i] + w));
     }
-  if (comp == 1) {  // ImplicitAndUpdateQR.F90:70-71
+  }
+  if (comp == 1 && ok) {  // ImplicitAndUpdateQR.F90:70-71
     if (p == 0) q[l] = 0.0;
     if (p == NS - 1) q[(long long)(g.nr - 1) * P + l] = 0.0;
+  }
+}
+
+// The table of a block's lines: one for all of them where their wall masks
+// agree (always with no-slip walls, and for the lines of a wave along a
+// groove), else one for each lane.
+template <int R, bool UNIFORM, bool FOLD>
+DEVI void helm_solve_body(const long long lgrp, const int comp, const GridDev &g,
+                          double *__restrict__ q, const double *__restrict__ y,
+                          const unsigned char *__restrict__ icyl,
+                          const unsigned char *__restrict__ ocyl, const double *__restrict__ lu,
+                          int nt, double *ex) {
+  if (UNIFORM || comp == 1) {
+    helm_solve_lines<R, true, FOLD>(lgrp, comp, g, q, y, lu + (size_t)(comp == 1 ? 0 : 3) * nt, ex);
+  } else {
+    const long long l = lgrp * 64 + threadIdx.x, lc = l < g.P ? l : g.P - 1;
+    const int var = icyl[lc] + 2 * ocyl[lc], v0 = __builtin_amdgcn_readfirstlane(var);
+    if (__all(var == v0))  // the same lines in every wave of the block
+      helm_solve_lines<R, true, FOLD>(lgrp, comp, g, q, y, lu + (size_t)v0 * nt, ex);
+    else
+      helm_solve_lines<R, false, FOLD>(lgrp, comp, g, q, y, lu + (size_t)var * nt, ex);
   }
 }
 
@@ -1076,18 +1108,19 @@ const RhsRow *rhs_rows(const tc_ctx *c, int ns) {
 static unsigned line_blocks(const tc_ctx *c) { return (unsigned)((c->P + 255) / 256); }
 
 // Shape of the partitioned solve: waves per block and the row capacity R of
-// its kernel, by the line length alone (an instance's bits must not depend
-// on what it shares a launch with).  ns = 0: the serial form.  Measured us
-// with R = 8 / 25 / 50 / 100: 128x128x97 20 / 17 / 21 / 32, 256x256x193
-// 144 (R = 16) / 110 / 120 / 131, 256x256x385 - / 265 / 232 / 245,
-// 512x512x385 - / 1020 / 957 / 960.
+// its kernel, by the grid's shape alone (an instance's bits must not depend
+// on what it shares a launch with).  ns = 0: the serial form.  Few rows a
+// wave shorten the chain where there are few lines, many keep more loads in
+// flight where there are many: measured us with R = 25 / 50 / 100,
+// 128x128x97 18 / 21 / 32, 256x256x193 110 / 118 / 131, 256x256x385 257 /
+// 239 / 254, 512x512x385 970 / 953 / 887.
 struct SolveShape {
   int ns, rows;
 };
 static SolveShape solve_shape(const tc_ctx *c) {
   const int n = c->nrm;
   if (c->lu_pivots) return {0, 0};
-  const int R = n <= 72 ? 8 : (n <= 256 ? 25 : (n <= 400 ? 50 : 100));
+  const int R = n <= 72 ? 8 : (n <= 256 ? 25 : (n <= 400 && c->P < (1 << 17) ? 50 : 100));
   const int ns = (n + R - 1) / R;
   return ns <= (R > 32 ? 8 : 16) ? SolveShape{ns, R} : SolveShape{0, 0};
 }
