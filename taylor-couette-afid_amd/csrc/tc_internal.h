@@ -284,6 +284,7 @@ void launch_stats(tc_ctx *c, bool stats, bool diss);
 void launch_dump(tc_ctx *c, int kind, int k);
 int regrid_field(tc_ctx *c, int field, const double *old, int ntho, int nzo, int nro, int istro,
                  double stro);
+void launch_transpose(tc_ctx *c, bool to_device, double *f, double *d, int i0, int ni);
 void launch_copy(tc_ctx *c, int dst, int src);
 void launch_triad(tc_ctx *c, int a, int b, int cc, double s);
 

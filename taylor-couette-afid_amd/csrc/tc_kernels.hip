@@ -2173,6 +2173,49 @@ void launch_copy(tc_ctx *c, int dst, int src) {
   timer_end(c);
 }
 
+// Fortran order (1:nr,1:nzm,1:nthm) to and from the device's [r][z][theta],
+// for the theta columns i0 .. i0+ni-1, whose nr*nzm values each are
+// contiguous in f.  A 32 x 32 (r x theta) tile of one z goes through LDS, so
+// both sides move 256-byte runs; bound by HBM (16 bytes a value), behind the
+// host copy that feeds it.
+constexpr int TP = 32;
+template <bool TO_DEVICE>
+__global__ __launch_bounds__(256) void k_transpose(double *__restrict__ f, double *__restrict__ d,
+                                                   int nr, int nzm, int nthm, int i0, int ni) {
+  __shared__ double t[TP][TP + 1];
+  const int x = threadIdx.x % TP, y = threadIdx.x / TP, j = blockIdx.z;
+  const int ib = blockIdx.x * TP, kb = blockIdx.y * TP;
+  auto at_f = [&](int k, int i) { return ((long long)i * nzm + j) * nr + k; };
+  auto at_d = [&](int k, int i) { return ((long long)k * nzm + j) * nthm + i0 + i; };
+#pragma unroll
+  for (int q = 0; q < TP; q += 256 / TP) {
+    if (TO_DEVICE) {
+      if (kb + x < nr && ib + y + q < ni) t[y + q][x] = f[at_f(kb + x, ib + y + q)];
+    } else {
+      if (ib + x < ni && kb + y + q < nr) t[y + q][x] = d[at_d(kb + y + q, ib + x)];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < TP; q += 256 / TP) {
+    if (TO_DEVICE) {
+      if (ib + x < ni && kb + y + q < nr) d[at_d(kb + y + q, ib + x)] = t[x][y + q];
+    } else {
+      if (kb + x < nr && ib + y + q < ni) f[at_f(kb + x, ib + y + q)] = t[x][y + q];
+    }
+  }
+}
+
+void launch_transpose(tc_ctx *c, bool to_device, double *f, double *d, int i0, int ni) {
+  const dim3 grid((unsigned)((ni + TP - 1) / TP), (unsigned)((c->nr + TP - 1) / TP), (unsigned)c->nzm);
+  if (to_device)
+    hipLaunchKernelGGL(k_transpose<true>, grid, dim3(256), 0, c->stream, f, d, c->nr, c->nzm,
+                       c->nthm, i0, ni);
+  else
+    hipLaunchKernelGGL(k_transpose<false>, grid, dim3(256), 0, c->stream, f, d, c->nr, c->nzm,
+                       c->nthm, i0, ni);
+}
+
 // STREAM triad a = b + s*c over whole fields, two doubles per thread.
 __global__ __launch_bounds__(256) void k_triad(double2 *__restrict__ a, const double2 *__restrict__ b,
                                                const double2 *__restrict__ cc, double s, long long n2,
