@@ -171,6 +171,35 @@ __device__ __forceinline__ GridDev glob(const GridDev &s) {
   g.grd = glob(g.grd), g.glo = glob(g.glo), g.gup = glob(g.gup);
   return g;
 }
+// Workgroups are dispatched round-robin over the XCDs; hand each XCD a
+// contiguous run of tiles so neighbouring tiles share one L2.
+__device__ __forceinline__ int xcd_tile(int b, int nb) {
+  constexpr int NX = 8;
+  const int q = nb / NX, r = nb - q * NX;
+  const int x = b % NX, local = b / NX;
+  return x * q + (x < r ? x : r) + local;
+}
+
+// A load from a table that no kernel writes while it is read.  In the
+// constant address space a load at a wave-uniform address is a scalar load
+// whatever else the kernel stores; through a plain pointer it is one only
+// where the compiler can rule out every store, and else a vector load whose
+// wait also drains the loads in flight.
+__device__ __forceinline__ double ldk(const double *p) {
+  typedef __attribute__((address_space(4))) const double CT;
+  return *(CT *)(unsigned long long)p;
+}
+template <class T>
+__device__ __forceinline__ T ldk_record(const T *p) {
+  constexpr int N = sizeof(T) / sizeof(double);
+  struct {
+    double v[N];
+  } a;
+#pragma unroll
+  for (int q = 0; q < N; q++) a.v[q] = ldk(reinterpret_cast<const double *>(p) + q);
+  return __builtin_bit_cast(T, a);
+}
+
 __device__ __forceinline__ bool inst_stopped(const StepDesc &d) {
   if (!d.res) return false;
   const BatchRes *r = glob(d.res);
@@ -271,6 +300,8 @@ void launch_correct_both(tc_ctx *c);
 void launch_zero_wall_qr(tc_ctx *c);
 // reductions: results land in c->red_host
 size_t reduction_doubles(const tc_ctx *c);
+// value q < nv of the nb partials in c->red, summed or (bit q of opmask) maximised
+void combine_partials(tc_ctx *c, unsigned nb, int nv, unsigned opmask);
 void launch_max_cfl(tc_ctx *c);
 void launch_max_div(tc_ctx *c);
 void launch_torque(tc_ctx *c);

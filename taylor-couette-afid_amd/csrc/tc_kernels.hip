@@ -21,35 +21,6 @@ DEVI long long IX(const GridDev &g, int k, int j, int i) {
 DEVI int wrap_p(int i, int n) { return (i + 1 == n) ? 0 : i + 1; }
 DEVI int wrap_m(int i, int n) { return (i == 0) ? n - 1 : i - 1; }
 
-// Workgroups are dispatched round-robin over the XCDs; hand each XCD a
-// contiguous run of tiles so neighbouring tiles share one L2.
-DEVI int xcd_tile(int b, int nb) {
-  constexpr int NX = 8;
-  const int q = nb / NX, r = nb - q * NX;
-  const int x = b % NX, local = b / NX;
-  return x * q + (x < r ? x : r) + local;
-}
-
-// A load from a table that no kernel writes while it is read.  In the
-// constant address space a load at a wave-uniform address is a scalar load
-// whatever else the kernel stores; through a plain pointer it is one only
-// where the compiler can rule out every store, and else a vector load whose
-// wait also drains the loads in flight.
-DEVI double ldk(const double *p) {
-  typedef __attribute__((address_space(4))) const double CT;
-  return *(CT *)(unsigned long long)p;
-}
-template <class T>
-DEVI T ldk_record(const T *p) {
-  constexpr int N = sizeof(T) / sizeof(double);
-  struct {
-    double v[N];
-  } a;
-#pragma unroll
-  for (int q = 0; q < N; q++) a.v[q] = ldk(reinterpret_cast<const double *>(p) + q);
-  return __builtin_bit_cast(T, a);
-}
-
 // Non-temporal access for arrays streamed once per kernel (no other block
 // re-reads them soon): a streaming copy runs 5.8% faster with both.
 DEVI double ld_nt(const double *p) { return __builtin_nontemporal_load(p); }
@@ -1754,7 +1725,7 @@ size_t reduction_doubles(const tc_ctx *c) {
 
 // The results go to pinned host memory (coherent), which the host reads
 // after the stream has drained: no copy is queued behind the kernel.
-static void finish_reduction(tc_ctx *c, unsigned nb, int nv, unsigned opmask) {
+void combine_partials(tc_ctx *c, unsigned nb, int nv, unsigned opmask) {
   hipLaunchKernelGGL(k_combine, dim3((unsigned)nv), dim3(256), 0, c->stream, c->red, (int)nb, nv,
                      opmask, c->red_host);
 }
@@ -1764,7 +1735,7 @@ void launch_max_cfl(tc_ctx *c) {
   const int ns = red_segments(c);
   hipLaunchKernelGGL(k_pointmax<0>, dim3(red_blocks(c) * ns), dim3(RED_THREADS), 0, c->stream, c->gd,
                      c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->red, ns);
-  finish_reduction(c, red_blocks(c) * ns, 1, 1u);
+  combine_partials(c, red_blocks(c) * ns, 1, 1u);
   timer_end(c);
 }
 void launch_max_div(tc_ctx *c) {
@@ -1772,7 +1743,7 @@ void launch_max_div(tc_ctx *c) {
   const int ns = red_segments(c);
   hipLaunchKernelGGL(k_pointmax<1>, dim3(red_blocks(c) * ns), dim3(RED_THREADS), 0, c->stream, c->gd,
                      c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->red, ns);
-  finish_reduction(c, red_blocks(c) * ns, 1, 1u);
+  combine_partials(c, red_blocks(c) * ns, 1, 1u);
   timer_end(c);
 }
 // ---------------------------------------------------------------------------
@@ -1839,13 +1810,13 @@ void launch_torque(tc_ctx *c) {
   hipLaunchKernelGGL(k_torque, dim3(red_blocks(c)), dim3(RED_THREADS), 0, c->stream, c->gd,
                      c->f[TC_QT], c->mask, c->mask + c->P, c->p.virotint, c->p.virotext, del,
                      deln, c->red);
-  finish_reduction(c, red_blocks(c), 2, 0u);
+  combine_partials(c, red_blocks(c), 2, 0u);
 }
 void launch_velocity_stats(tc_ctx *c) {
   const int ns = red_segments(c);
   hipLaunchKernelGGL(k_velstats, dim3(red_blocks(c) * ns), dim3(RED_THREADS), 0, c->stream, c->gd,
                      c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->g.pi, c->red, ns);
-  finish_reduction(c, red_blocks(c) * ns, 6, 7u);
+  combine_partials(c, red_blocks(c) * ns, 6, 7u);
 }
 
 // One pass over the velocity for the logging step of main.F90:180-186:
@@ -1931,7 +1902,7 @@ void launch_diagnostics(tc_ctx *c) {
   hipLaunchKernelGGL(k_diagnostics, dim3(red_blocks(c) * ns), dim3(RED_THREADS), 0, c->stream, c->gd,
                      c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->mask, c->mask + c->P,
                      c->p.virotint, c->p.virotext, del, deln, c->g.pi, c->red, ns);
-  finish_reduction(c, red_blocks(c) * ns, 10, 0x1Fu);
+  combine_partials(c, red_blocks(c) * ns, 10, 0x1Fu);
   timer_end(c);
 }
 

@@ -421,15 +421,6 @@ __global__ __launch_bounds__(256) void k_fft_theta_inv_g(const StepDesc *__restr
                      (long long)d.g.nrm * d.g.nzm, d.g.nth2, d.g.sstr);
 }
 
-// Workgroups are dispatched round-robin over the XCDs; hand each XCD a
-// contiguous run of tiles so tiles sharing cache lines share one L2.
-DEVI int xcd_tile(int b, int nb) {
-  constexpr int NX = 8;
-  const int q = nb / NX, r = nb - q * NX;
-  const int x = b % NX, local = b / NX;
-  return x * q + (x < r ? x : r) + local;
-}
-
 // c2c along z for a tile of pl.lines ktheta columns of one r-plane.  The LDS
 // tile keeps the global row-major order [z][column]; lane = column fastest,
 // so global and LDS accesses are both contiguous across lanes.  Spectral rows

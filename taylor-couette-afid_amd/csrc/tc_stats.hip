@@ -2,12 +2,11 @@
 // vorticity of CalcVorticity (StatRoutines.F90:12-71, CalcVorticity.F90:11-88)
 // and CalcDissipation (CalcDissipation.F90:11-153).
 //
-// One 256-thread block owns one (r-plane k, z-row j) theta line: its
-// threads stride along theta, each sums its points, a fixed butterfly
-// reduces each wave, the four wave sums are added in order, and the block
-// adds the result to the (k, j) accumulators it alone owns.  So the
-// accumulators need no atomics and the sums are the same run to run.  The
-// vorticity is evaluated at the point and never stored.
+// One wave owns one (r-plane k, z-row j) theta line: its lanes stride along
+// theta, each sums its points, a fixed tree over the wave reduces the sums,
+// and the wave adds the result to the (k, j) accumulators it alone owns.  So
+// the accumulators need no atomics and the sums are the same run to run.
+// The vorticity is evaluated at the point and never stored.
 //
 // Accumulators: TC_NSTATS arrays of (nrm, nzm) in Fortran order (k fastest),
 // in WriteStats order (StatRoutines.F90:97-152), so a download is the
@@ -27,15 +26,45 @@ struct Fields {
 constexpr int NS = TC_NSTATS;  // accumulators
 constexpr int NV = NS + 1;     // + the pvol-weighted dissipation of nute
 
-// One 256-thread block per (k, j) theta line: lanes stride along theta by
-// 256, each wave reduces with a fixed butterfly, and the four wave sums are
-// added in wave order.
+// Sums of NQ <= 16 values over a wave, value (lane & 15) left in each lane:
+// every step halves the values a lane holds by exchanging the other half
+// with its partner, 15 exchanges instead of 4 NQ, and two more complete it.
+template <int NQ>
+DEVI double wave_sums(const double *s, int lane) {
+  double v[16];
+#pragma unroll
+  for (int q = 0; q < 16; q++) v[q] = q < NQ ? s[q] : 0.0;
+#pragma unroll
+  for (int w = 8; w >= 1; w >>= 1) {
+    const bool up = lane & w;
+#pragma unroll
+    for (int q = 0; q < w; q++) {
+      const double keep = up ? v[q + w] : v[q], send = up ? v[q] : v[q + w];
+      v[q] = keep + __shfl_xor(send, w, 64);
+    }
+  }
+  v[0] += __shfl_xor(v[0], 16, 64);
+  return v[0] + __shfl_xor(v[0], 32, 64);
+}
+
+// One wave per (k, j) line, four consecutive j per block.  z is cut into one
+// band per XCD, and a band's blocks run along z first, then over the planes,
+// so that the rows j-1, j, j+1, the planes k-1, k, k+1 and the accumulator
+// lines (consecutive in k) that neighbouring lines share meet in one L2.  A
+// block per line, whose four waves each reduced all sums for 64 points,
+// spent its time in the reductions: 256x256x193 472 us for the statistics.
+constexpr int NBAND = 8;
+static int band_blocks(int nzm) { return (nzm + 4 * NBAND - 1) / (4 * NBAND); }
 template <bool STATS, bool DISS>
 __global__ __launch_bounds__(256) void k_stats(GridDev g, Fields f, double *__restrict__ acc,
                                                double *__restrict__ part, double ren) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int j = blockIdx.x;
-  const int k = blockIdx.y + 1;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nj = gridDim.x / (NBAND * g.nrm);  // blocks along z in a band
+  const int id = xcd_tile(blockIdx.x, gridDim.x), band = id / (nj * g.nrm);
+  const int rest = id - band * (nj * g.nrm), k = rest / nj + 1;
+  const int j = (band * nj + rest % nj) * 4 + wave;
+  if (j >= g.nzm) return;
   const int nthm = g.nthm, nzm = g.nzm, nrm = g.nrm;
   const long long P = g.P;
   const int kp = k + 1;                       // qr face above the cell
@@ -43,11 +72,11 @@ __global__ __launch_bounds__(256) void k_stats(GridDev g, Fields f, double *__re
   const int kmm = k > 1 ? k - 1 : 1;          // kmv(k)
   const int jp = j + 1 == nzm ? 0 : j + 1, jm = j == 0 ? nzm - 1 : j - 1;
   const double dxt = g.dxt, dxz = g.dxz, pi = M_PI;
-  const double usrc_k = g.usrc[k], usrc_kp = g.usrc[kp], usrc_kpp = g.usrc[kpp];
-  const double usrc_kmm = g.usrc[kmm];
-  const double usrm_k = g.usrm[k], usrm_kpp = g.usrm[kpp], usrm_kmm = g.usrm[kmm];
-  const double rm_k = g.rm[k], rm_kpp = g.rm[kpp], rm_kmm = g.rm[kmm];
-  const double udx2mm = g.udx2mm[k], udx2cc = g.udx2cc[k], pvol = g.pvol[k];
+  const double usrc_k = ldk(g.usrc + k), usrc_kp = ldk(g.usrc + kp), usrc_kpp = ldk(g.usrc + kpp);
+  const double usrc_kmm = ldk(g.usrc + kmm);
+  const double usrm_k = ldk(g.usrm + k), usrm_kpp = ldk(g.usrm + kpp), usrm_kmm = ldk(g.usrm + kmm);
+  const double rm_k = ldk(g.rm + k), rm_kpp = ldk(g.rm + kpp), rm_kmm = ldk(g.rm + kmm);
+  const double udx2mm = ldk(g.udx2mm + k), udx2cc = ldk(g.udx2cc + k), pvol = ldk(g.pvol + k);
   const double usnthm = 1.0 / nthm;
   auto at = [&](const double *a, int kk, int jj, int ii) {
     return a[(long long)(kk - 1) * P + (long long)jj * nthm + ii];
@@ -57,7 +86,7 @@ __global__ __launch_bounds__(256) void k_stats(GridDev g, Fields f, double *__re
 #pragma unroll
   for (int q = 0; q < NV; q++) s[q] = 0.0;
 
-  for (int i = threadIdx.x; i < nthm; i += 256) {
+  for (int i = lane; i < nthm; i += 64) {
     const int ip = i + 1 == nthm ? 0 : i + 1, im = i == 0 ? nthm - 1 : i - 1;
     if (STATS) {
       // CalcVorticity.F90:41-79
@@ -118,44 +147,39 @@ __global__ __launch_bounds__(256) void k_stats(GridDev g, Fields f, double *__re
       s[NS] += d * pvol * pi;
     }
   }
-  // fixed butterfly over each wave, then the four waves in order
-  __shared__ double sh[4][NV];
-#pragma unroll
-  for (int q = 0; q < NV; q++) {
-    double v = s[q];
-#pragma unroll
-    for (int w = 32; w >= 1; w >>= 1) v += __shfl_xor(v, w, 64);
-    if (lane == 0) sh[wave][q] = v;
-  }
-  __syncthreads();
-  // thread q adds accumulator q of this (k, j)
   const long long kj = (long long)(k - 1) + (long long)nrm * j;
   const long long M = (long long)nrm * nzm;
-  const int q = threadIdx.x;
-  if (q < NV) {
-    const double v = ((sh[0][q] + sh[1][q]) + sh[2][q]) + sh[3][q];
-    if (q < NS) {
-      const bool mine = (q == TC_ST_DISSTE) ? DISS : STATS;
-      if (mine) acc[q * M + kj] += v;
-    } else if (DISS) {
-      part[kj] = v;
-    }
+  if (STATS) {
+    // accumulators 0..15 and 16, all but the last one (DISSTE)
+    static_assert(TC_ST_DISSTE == 17 && NS == 18, "order of the accumulators");
+    const double v = wave_sums<16>(s, lane);
+    double w = s[16];
+#pragma unroll
+    for (int x = 1; x <= 32; x <<= 1) w += __shfl_xor(w, x, 64);
+    if (lane < 17) acc[lane * M + kj] += lane < 16 ? v : w;
+  }
+  if (DISS) {
+    const double v = wave_sums<2>(s + TC_ST_DISSTE, lane);
+    if (lane == 0) acc[TC_ST_DISSTE * M + kj] += v;
+    if (lane == 1) part[kj] = v;
   }
 }
 
-// Sum of the n per-line dissipation partials in a fixed order (one block).
+// Sums of contiguous runs of the n per-line dissipation partials, each in a
+// fixed order, one per block; the blocks' sums are added by k_combine.
 __global__ __launch_bounds__(256) void k_sum_fixed(const double *__restrict__ part, long long n,
                                                    double *__restrict__ out) {
   __shared__ double sh[256];
+  const long long b0 = blockIdx.x * n / gridDim.x, b1 = (blockIdx.x + 1) * n / gridDim.x;
   double v = 0.0;
-  for (long long b = threadIdx.x; b < n; b += 256) v += part[b];
+  for (long long b = b0 + threadIdx.x; b < b1; b += 256) v += part[b];
   sh[threadIdx.x] = v;
   __syncthreads();
   for (int w = 128; w >= 1; w >>= 1) {
     if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[0] = sh[0];
+  if (threadIdx.x == 0) out[blockIdx.x] = sh[0];
 }
 
 // DumpRCuts.F90:28-36 at r-plane k: vt, vr (mean of the two faces), vz;
@@ -231,7 +255,7 @@ void launch_dump(tc_ctx *c, int kind, int k) {
 // vorticity); diss: CalcDissipation, whose volume sum lands in c->red_out[0].
 void launch_stats(tc_ctx *c, bool stats, bool diss) {
   timer_begin(c, "stats");
-  const dim3 grid((unsigned)c->nzm, (unsigned)c->nrm);
+  const dim3 grid((unsigned)(NBAND * band_blocks(c->nzm)) * (unsigned)c->nrm);
   Fields f{c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->f[TC_PR]};
   const double ren = c->p.ren;
   if (stats && diss)
@@ -244,8 +268,10 @@ void launch_stats(tc_ctx *c, bool stats, bool diss) {
     hipLaunchKernelGGL((k_stats<false, true>), grid, dim3(256), 0, c->stream, c->gd, f, c->stats,
                        c->stat_part, ren);
   if (diss) {
-    hipLaunchKernelGGL(k_sum_fixed, dim3(1), dim3(256), 0, c->stream, c->stat_part,
-                       (long long)c->nrm * c->nzm, c->red_host);
+    constexpr int NB = 64;
+    hipLaunchKernelGGL(k_sum_fixed, dim3(NB), dim3(256), 0, c->stream, c->stat_part,
+                       (long long)c->nrm * c->nzm, c->red);
+    combine_partials(c, NB, 1, 0u);
   }
   timer_end(c);
 }
