@@ -83,9 +83,10 @@ int tc_create(const tc_params *p, tc_ctx **out);
  * fields take the TC_* environment override, else the default. */
 typedef struct tc_tuning {
   int helm_lpt;   /* radial lines per thread of the fused Helmholtz kernel: 1, 2 (0: by occupancy) */
-  int fft_t_lds;  /* LDS bytes of a theta-FFT block (default 32768) */
-  int fft_z_lds;  /* LDS bytes of a z-FFT block (default 65536) */
-  int fft_z_nt;   /* threads of a z-FFT block: 256 or 512 (default) */
+  int fft_t_lds;  /* LDS bytes of a theta-FFT block (default 16384 up to NTM = 384, else 32768) */
+  int fft_z_lds;  /* LDS bytes of a z-FFT block (default: 16 columns within 32768 up to
+                     NZM = 256, else 65536) */
+  int fft_z_nt;   /* threads of a z-FFT block: 256 (default up to NZM = 256) or 512 */
   int fft_pad;    /* LDS padding of the FFT tiles: one slot per 8 points (1, default),
                      per 4 (2) or per 16 (3); -1 off */
   int poisson_pq; /* rows per thread of the radial Poisson solve: 13 (default) or 26 */

@@ -332,9 +332,8 @@ void set_substep(tc_ctx *c, int ns) {
 
 
 // Effective tuning: explicit nonzero fields first, then the TC_* environment
-// overrides, then the defaults (which come from sweeps at 512x512x385).
-// nrm: the radial size, for the defaults that depend on it
-tc_tuning resolve_tuning(const tc_tuning *in, int nrm) {
+// overrides, then the defaults for a grid of nthm x nzm x nrm.
+tc_tuning resolve_tuning(const tc_tuning *in, int nthm, int nzm, int nrm) {
   tc_tuning t{};
   if (in) t = *in;
   auto env = [](const char *name, int dflt) {
@@ -342,9 +341,18 @@ tc_tuning resolve_tuning(const tc_tuning *in, int nrm) {
     return v ? std::atoi(v) : dflt;
   };
   if (t.helm_lpt == 0) t.helm_lpt = std::max(0, std::min(2, env("TC_HELM_LPT", 0)));
-  if (t.fft_t_lds == 0) t.fft_t_lds = env("TC_FFT_T_LDS", 32768);
-  if (t.fft_z_lds == 0) t.fft_z_lds = env("TC_FFT_Z_LDS", 65536);
-  if (t.fft_z_nt == 0) t.fft_z_nt = env("TC_FFT_Z_NT", 512) == 256 ? 256 : 512;
+  // FFT blocks: short lines need few per block, or the grid is too coarse to
+  // fill the device and the last column tile mostly empty (64x64x65: 65
+  // blocks of 32 theta lines or 64 columns).  theta, us with 16 / 32 KiB
+  // (divergence fused): n = 64 11.4 / 14.7, 192 34.2 / 35.1, 375 123 / 124;
+  // inverse 375 72 / 76; 512 keeps its four lines in 32 KiB.  z, us with the
+  // default here / 64 KiB and 512 threads: n = 64 7.7 / 9.0, 128 (192 columns)
+  // 18.1 / 24.5, 240 62 / 67, 256 51 / 54; 512 keeps eight columns in 64 KiB
+  // and 512 threads.
+  if (t.fft_t_lds == 0) t.fft_t_lds = env("TC_FFT_T_LDS", nthm <= 384 ? 16384 : 32768);
+  if (t.fft_z_lds == 0)
+    t.fft_z_lds = env("TC_FFT_Z_LDS", nzm <= 256 ? std::min(32768, 16 * 16 * nzm) : 65536);
+  if (t.fft_z_nt == 0) t.fft_z_nt = env("TC_FFT_Z_NT", nzm <= 256 ? 256 : 512) == 256 ? 256 : 512;
   if (t.fft_pad == 0) {
     const int v = env("TC_FFT_PAD", 1);
     t.fft_pad = (v == 0) ? -1 : std::max(1, std::min(3, v));
@@ -483,7 +491,7 @@ int tc_create_tuned(const tc_params *p, const tc_tuning *tun, tc_ctx **out) {
   if (!c) return fail("out of host memory");
   c->p = *p;
   std::string e = tc::build_grid(*p, c->g);
-  const tc_tuning t = resolve_tuning(tun, p->nrm);
+  const tc_tuning t = resolve_tuning(tun, p->nthm, p->nzm, p->nrm);
   if (e.empty()) e = apply_plans(c, t);
   if (!e.empty()) {
     delete c;
@@ -675,7 +683,7 @@ int tc_create_tuned(const tc_params *p, const tc_tuning *tun, tc_ctx **out) {
 int tc_set_tuning(tc_ctx *c, const tc_tuning *t) {
   CTXCHK(c);
   HIPCHK(hipStreamSynchronize(c->stream));
-  const tc_tuning r = resolve_tuning(t, c->nrm);
+  const tc_tuning r = resolve_tuning(t, c->nthm, c->nzm, c->nrm);
   const std::string e = apply_plans(c, r);
   if (!e.empty()) return fail(e);
   tc::choose_helm_schedule(c, r.helm_lpt);
