@@ -92,7 +92,7 @@ typedef struct tc_tuning {
   int poisson_pq; /* rows per thread of the radial Poisson solve: 13 (default) or 26 */
   int defer;      /* RK3 with even nthm: apply the pressure correction of substeps 1 and 2
                      inside the next substep's Helmholtz kernel: 2 always, -1 never,
-                     1 from 8 Mi grid points up (default; TC_DEFER_CORRECTION 2/0/1).
+                     1 from 1 Mi grid points up (default; TC_DEFER_CORRECTION 2/0/1).
                      Changes results at the rounding level only. */
 } tc_tuning;
 

@@ -409,13 +409,14 @@ void torque_from_sums(const tc_ctx *c, double slow, double sup, double *inner, d
 }  // namespace
 
 namespace tc {
-// tc_tuning::defer: 1 defers from 8 Mi grid points up, where the saved
-// passes pay; below that a lone grid lives in the caches and the
-// correction's extra instructions cost more than they save (a batch of many
-// small instances is another matter).  2: always; -1: never.  The spare
-// pressure array is allocated where the deferral applies.
+// tc_tuning::defer: 1 defers from 1 Mi grid points up, where the two
+// correction passes saved are more than the correction adds to the Helmholtz
+// launches (step in us, never / always: 64x64x65 222 / 224, 96x96x97 362 /
+// 360, 128x128x97 480 / 463, 192x128x129 799 / 738, 256x256x193 2484 /
+// 2330).  2: always; -1: never.  The spare pressure array is allocated where
+// the deferral applies.
 int set_deferral(tc_ctx *c, int mode) {
-  c->defer_corr = mode == 2 || (mode == 1 && (long long)c->nthm * c->nzm * c->nrm >= (8LL << 20));
+  c->defer_corr = mode == 2 || (mode == 1 && (long long)c->nthm * c->nzm * c->nrm >= (1LL << 20));
   if (c->defer_corr && c->p.nsst == 3 && c->nthm % 2 == 0 && !c->pr_alt) {
     int rc = dev_alloc(c, (void **)&c->pr_alt, sizeof(double) * (size_t)c->N);
     if (rc) return rc;

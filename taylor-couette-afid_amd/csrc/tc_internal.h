@@ -250,7 +250,7 @@ struct tc_ctx {
   // fused RK3 step: the pressure correction of substeps 1 and 2 is applied
   // by the next substep's Helmholtz kernel instead of its own pass; pr_alt
   // receives the corrected pressure of substep 1 (TC_DEFER_CORRECTION at
-  // tc_create: 1 from 8 Mi grid points up, 2 always, 0 never)
+  // tc_create: 1 from 1 Mi grid points up, 2 always, 0 never)
   bool defer_corr = true;
   double corr_al = 0.0;
   double *pr_alt = nullptr;

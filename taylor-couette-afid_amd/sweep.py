@@ -159,7 +159,7 @@ def footprint_bytes(p, tuning=None):
     """Device bytes of one instance: eleven fields of nr planes (twelve where
     the RK3 step defers its pressure correction: even nthm and the tuning's
     ``defer`` 2, or 1 (the default, unless TC_DEFER_CORRECTION says 2 or 0)
-    with at least 8 Mi grid points), the spectrum, and the small
+    with at least 1 Mi grid points), the spectrum, and the small
     per-instance tables."""
     nthm, nzm, nrm = p["nthm"], p["nzm"], p["nrm"]
     sstr = ((nthm // 2 + 1) + 7) // 8 * 8
@@ -167,7 +167,7 @@ def footprint_bytes(p, tuning=None):
     if mode == 0:
         mode = {"0": -1, "2": 2}.get(os.environ.get("TC_DEFER_CORRECTION", "1"), 1)
     defer = (nthm % 2 == 0 and p.get("nsst", 3) == 3
-             and (mode == 2 or (mode == 1 and nthm * nzm * nrm >= 8 << 20)))
+             and (mode == 2 or (mode == 1 and nthm * nzm * nrm >= 1 << 20)))
     nf = 12 if defer else 11
     return 8 * nf * (nrm + 1) * nzm * nthm + 16 * nrm * nzm * sstr + (8 << 20)
 
