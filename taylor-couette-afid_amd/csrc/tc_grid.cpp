@@ -258,6 +258,13 @@ std::string build_grid(const tc_params &p, Grid &g) {
   return std::string();
 }
 
+int slip_displacement(const tc_params &p, const Grid &g, double time) {
+  const double perdist = 2 * g.pi / p.lamb;
+  const double wint = p.virotint / p.rint;
+  double anglemoved = std::fmod(wint * time, perdist);
+  return (int)std::floor(anglemoved * g.dxt);
+}
+
 void slip_bcs(const tc_params &p, const Grid &g, double time, std::vector<int> &icyl,
               std::vector<int> &ocyl) {
   // SlipBCs.F90:31-90; masks are 1 everywhere unless MINSTR*·MULTMIN != 0
@@ -268,10 +275,7 @@ void slip_bcs(const tc_params &p, const Grid &g, double time, std::vector<int> &
   const int ntot = ntott + ntotz;
   if (ntot == 0) return;
   const int acute = 1;
-  const double perdist = 2 * g.pi / p.lamb;
-  const double wint = p.virotint / p.rint;
-  double anglemoved = std::fmod(wint * time, perdist);
-  const int points_moved = (int)std::floor(anglemoved * g.dxt);
+  const int points_moved = slip_displacement(p, g, time);
   std::vector<int> thdispl((size_t)nthm + 1);
   for (int i = 1; i <= nthm; i++) {
     thdispl[i] = (i + points_moved) % nthm;

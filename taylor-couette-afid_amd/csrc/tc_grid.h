@@ -29,6 +29,8 @@ struct Grid {
 std::string build_grid(const tc_params &p, Grid &g);
 
 // SlipBCs.F90:31-90 at time t: masks (nzm,nthm) column-major.
+// theta points the inner wall's pattern has moved by: all that slip_bcs takes from the time
+int slip_displacement(const tc_params &p, const Grid &g, double time);
 void slip_bcs(const tc_params &p, const Grid &g, double time, std::vector<int> &icyl,
               std::vector<int> &ocyl);
 

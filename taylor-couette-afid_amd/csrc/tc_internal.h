@@ -225,6 +225,8 @@ struct tc_ctx {
   unsigned char *mask = nullptr;  // device [2][nzm*nthm] (icyl, ocyl), [j][i]
   std::vector<int> icyl, ocyl;    // host copies, (nzm,nthm) column-major
   bool masks_uniform_one = true;
+  bool slip_valid = false;  // the masks are SlipBCs' for a displacement of slip_moved points
+  int slip_moved = 0;
   // Helmholtz LU tables
   double *lu = nullptr;        // device
   double *lu_host = nullptr;   // pinned staging

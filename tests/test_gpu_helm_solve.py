@@ -58,3 +58,19 @@ def _implicit(tc, oracle, p, dt, nrm):
         orc.call(b)
     for f, sl in (("qt", slice(0, nrm)), ("qr", slice(0, nrm + 1)), ("qz", slice(0, nrm))):
         assert rel_l2(dev.get(f)[sl], orc.get(f)[sl]) < 1e-10, f
+
+
+def test_masks_set_between_steps_are_replaced(tc):
+    """A step forms SlipBCs' masks again after others were set, also where
+    the pattern has not moved since the last step."""
+    p = small_params(tc, 48, 40, 17, minstrz=3, multmin=1)
+    s = tc.Solver(p)
+    s.set_time(0.0, 1e-3)
+    s.begin_step()
+    want = s.masks()
+    ones = np.ones_like(want[0])
+    assert want[0].min() == 0
+    s.set_masks(ones, ones)
+    s.begin_step()
+    got = s.masks()
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
