@@ -444,8 +444,8 @@ _KERNEL_TIMER = {"k_correct_both2": "correct_both", "k_helm_rhs": "helm_fwd",
 def _timer_of(kernel):
     """Kernel timer name (the kernel_bytes key) of a device kernel name."""
     base = kernel.split("<")[0]
-    if base == "k_helm_rhs" and kernel.replace(" ", "").endswith(",true>"):
-        return "helm_fwd_corr"  # k_helm_rhs<UNIFORM, LPT, CORR = true>
+    if base == "k_helm_rhs" and kernel.replace(" ", "").endswith(",true,true>"):
+        return "helm_fwd_corr"  # k_helm_rhs<UNIFORM, LPT, CORR = true, PAIR>
     if base in _KERNEL_TIMER:
         return _KERNEL_TIMER[base]
     return base[2:] if base.startswith("k_") else base

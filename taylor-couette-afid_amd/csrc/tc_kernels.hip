@@ -25,14 +25,14 @@ DEVI int wrap_m(int i, int n) { return (i == 0) ? n - 1 : i - 1; }
 // re-reads them soon): a streaming copy runs 5.8% faster with both.
 DEVI double ld_nt(const double *p) { return __builtin_nontemporal_load(p); }
 DEVI void st_nt(double *p, double v) { __builtin_nontemporal_store(v, p); }
+typedef double d2v __attribute__((ext_vector_type(2)));
 DEVI double2 ld2_nt(const double *p) {
-  const double2 *q = reinterpret_cast<const double2 *>(p);
-  return make_double2(__builtin_nontemporal_load(&q->x), __builtin_nontemporal_load(&q->y));
+  const d2v v = __builtin_nontemporal_load(reinterpret_cast<const d2v *>(p));
+  return make_double2(v.x, v.y);
 }
 DEVI void st2_nt(double *p, double u, double v) {
-  double2 *q = reinterpret_cast<double2 *>(p);
-  __builtin_nontemporal_store(u, &q->x);
-  __builtin_nontemporal_store(v, &q->y);
+  const d2v w = {u, v};
+  __builtin_nontemporal_store(w, reinterpret_cast<d2v *>(p));
 }
 
 // ---------------------------------------------------------------------------
@@ -668,42 +668,34 @@ struct CorrIn {
 // read plane k-1 only at (dj, di) = (0, 0), (0, +1) and (+1, 0): m00, m01
 // and m10 hold those (the centre, theta+1 and z+1 values of the previous
 // iteration's plane k).
-template <bool CARRY>
+template <bool CARRY, int W = FT_W>
 struct LAcc {
   const double *m, *c, *p;  // planes k-1, k, k+1 of one field
-  int base;                 // (row+1)*FT_W + tx+1
+  int base;                 // of the point in a tile of rows W apart
   double m00, m01, m10;
   DEVI double operator()(int dk, int dj, int di) const {
     if constexpr (CARRY) {
       if (dk < 0) return dj != 0 ? m10 : (di != 0 ? m01 : m00);
     }
     const double *s = dk < 0 ? m : (dk > 0 ? p : c);
-    return s[base + dj * FT_W + di];
+    return s[base + dj * W + di];
   }
 };
 
 // A block of 256 threads owns a 64 (theta) x 4*LPT (z) tile of radial lines
 // from plane k0 to plane k1, LPT lines per thread (rows ty and ty+4).
 // UNIFORM: every wall mask is 1 (no-slip everywhere, the SlipBCs default).
-// CORR: qt, qr, qz hold the previous substep's velocity before its pressure
-// correction and pr its pressure before the correction; the correction
-// (dph of that substep) is applied to each plane as it is staged, from a
-// ring of dph planes with a two-point theta/z halo, so the corrected fields
-// are the ones the per-substep path would have stored, bit for bit.
-template <bool UNIFORM, int LPT, bool CORR>
+template <bool UNIFORM, int LPT>
 DEVI void helm_rhs_body(
     const int tile, const int k0, const int k1, const GridDev &g, const ImpArgs &a,
     const double *__restrict__ qt, const double *__restrict__ qr, const double *__restrict__ qz,
     const double *__restrict__ pr, double *__restrict__ ru1, double *__restrict__ ru2,
     double *__restrict__ ru3, double *__restrict__ yt, double *__restrict__ yr,
     double *__restrict__ yz, const unsigned char *__restrict__ icyl,
-    const unsigned char *__restrict__ ocyl, const RhsRow *__restrict__ rows, int ntx,
-    const CorrIn &ci, const double *__restrict__ dph, double *__restrict__ pr_out) {
+    const unsigned char *__restrict__ ocyl, const RhsRow *__restrict__ rows, int ntx) {
   constexpr int TJ = FT_J * LPT, H = TJ + 2, S = FT_W * H, NE = (S + FT_N - 1) / FT_N;
-  constexpr int W2 = FT_I + 4, S2 = W2 * (TJ + 4), NE2 = (S2 + FT_N - 1) / FT_N;
   __shared__ double sq[3][3][S];  // field, ring slot, tile
   __shared__ double sp[2][S];     // pressure planes k and k+1
-  __shared__ double sd[CORR ? 3 : 1][CORR ? S2 : 1];  // dph planes (slot = plane % 3)
   const int i0 = (tile % ntx) * FT_I, j0 = (tile / ntx) * TJ;
   const int tx = threadIdx.x % FT_I, ty = threadIdx.x / FT_I;
   const long long P = g.P;
@@ -721,65 +713,6 @@ DEVI void helm_rhs_body(
     ii = ((ii % g.nthm) + g.nthm) % g.nthm;
     off[q] = jj * g.nthm + ii;
   }
-  // CORR: the dph tile elements (two-point halo) this thread stages, and
-  // whether each of its velocity tile elements is an interior point whose
-  // corrected pressure it writes
-  int off2[CORR ? NE2 : 1];
-  bool wpr[NE];
-  const bool has_last2 = threadIdx.x + (NE2 - 1) * FT_N < S2;
-  if constexpr (CORR) {
-#pragma unroll
-    for (int q = 0; q < NE2; q++) {
-      const int e = threadIdx.x + q * FT_N;
-      const int ee = e < S2 ? e : 0;
-      int jj = j0 + ee / W2 - 2, ii = i0 + ee % W2 - 2;
-      jj = ((jj % g.nzm) + g.nzm) % g.nzm;
-      ii = ((ii % g.nthm) + g.nthm) % g.nthm;
-      off2[q] = jj * g.nthm + ii;
-    }
-#pragma unroll
-    for (int q = 0; q < NE; q++) {
-      const int e = threadIdx.x + q * FT_N;
-      const int row = e / FT_W, col = e % FT_W;
-      wpr[q] = (e < S) && row >= 1 && row <= TJ && col >= 1 && col <= FT_I &&
-               j0 + row - 1 < g.nzm && i0 + col - 1 < g.nthm;
-    }
-  }
-  // the corrected velocity of plane p at tile element e (correct_pair's
-  // arithmetic; q_r is zero on both walls)
-  auto corr_q = [&](int p, int e, double &vt, double &vr, double &vz) {
-    const int row = e / FT_W, col = e - row * FT_W;
-    const int e2 = (row + 1) * W2 + col + 1;
-    const double *dc = sd[CORR ? p % 3 : 0];
-    if (p <= g.nrm) {
-      vt = corr_qt(g, p, vt, dc[e2], dc[e2 - 1], ci.dt, ci.al);
-      vz = corr_qz(g, vz, dc[e2], dc[e2 - W2], ci.dt, ci.al);
-    }
-    if (p == 1 || p >= g.nr)
-      vr = 0.0;
-    else
-      vr = corr_qr(g, p, vr, dc[e2], sd[CORR ? (p - 1) % 3 : 0][e2], ci.dt, ci.al);
-  };
-  // the corrected pressure of plane p <= nrm at tile element e
-  auto corr_p = [&](int p, int e, double v) {
-    const int row = e / FT_W, col = e - row * FT_W;
-    const int e2 = (row + 1) * W2 + col + 1;
-    const double *dc = sd[CORR ? p % 3 : 0];
-    const double *dkp = sd[CORR ? (p < g.nrm ? p + 1 : p) % 3 : 0];
-    const double *dkm = sd[CORR ? (p > 1 ? p - 1 : p) % 3 : 0];
-    return corr_pr(g, p, v, dc[e2], dc[e2 - 1], dc[e2 + 1], dc[e2 - W2], dc[e2 + W2], dkm[e2],
-                   dkp[e2], ci.be);
-  };
-  // stage dph plane p (clamped to 1..nrm: beyond it no correction reads dph)
-  auto stage_dph = [&](int p) {
-    const long long od = (long long)(min(max(p, 1), g.nrm) - 1) * P;
-    double t[CORR ? NE2 : 1];
-#pragma unroll
-    for (int q = 0; q < NE2; q++) t[q] = dph[od + off2[q]];
-#pragma unroll
-    for (int q = 0; q < NE2; q++)
-      if (q < NE2 - 1 || has_last2) sd[(p + 3) % 3][threadIdx.x + q * FT_N] = t[q];
-  };
   // stage plane p of the velocity (before the first iteration)
   auto stage_q = [&](int p) {
     const long long oq = (long long)(p - 1) * P;
@@ -794,7 +727,6 @@ DEVI void helm_rhs_body(
     for (int q = 0; q < NE; q++)
       if (q < NE - 1 || has_last) {
         const int e = threadIdx.x + q * FT_N;
-        if constexpr (CORR) corr_q(p, e, t[0][q], t[1][q], t[2][q]);
         sq[0][p % 3][e] = t[0][q];
         sq[1][p % 3][e] = t[1][q];
         sq[2][p % 3][e] = t[2][q];
@@ -802,14 +734,14 @@ DEVI void helm_rhs_body(
   };
   // the RK history ru enters as ro*ru only: with ro = 0 (the first RK3
   // substep) it is not read at all
-  const bool hist = CORR || a.ro != 0.0;
+  const bool hist = a.ro != 0.0;
   const int nrm = g.nrm;
   // per-line state
   bool valid[LPT];
   long long l[LPT];
   int base[LPT];
   double fic[LPT], foc[LPT], h1[LPT], h2[LPT], h3[LPT], pr_km[LPT];
-  // !CORR: plane k-1 values carried from the previous iteration (qt centre,
+  // plane k-1 values carried from the previous iteration (qt centre,
   // qt theta+1, qr centre, qz centre, qz z+1), so that no thread reads the
   // ring slot of plane k-1 and the staging of plane k+2 into it needs no
   // barrier of its own
@@ -832,65 +764,36 @@ DEVI void helm_rhs_body(
     for (int q = 0; q < 5; q++) cm[u][q] = 0.0;
   }
   // planes k0-1 (if any), k0 and k0+1 of the velocity, k0 of the pressure
-  // and the pressure of k0-1 on the lines themselves.  CORR: with the dph
-  // planes that each of these corrections reads staged before it.
-  if constexpr (CORR) {
-    if (k0 > 1) {
-      stage_dph(k0 - 2);
-      stage_dph(k0 - 1);
-      stage_dph(k0);
-      __syncthreads();
-      stage_q(k0 - 1);
-#pragma unroll
-      for (int u = 0; u < LPT; u++) pr_km[u] = corr_p(k0 - 1, base[u], pr_km[u]);
-      __syncthreads();
-      stage_dph(k0 + 1);
-    } else {
-      stage_dph(1);
-      stage_dph(2);
-    }
-    __syncthreads();
-  } else if (k0 > 1) {
-    stage_q(k0 - 1);
-  }
+  if (k0 > 1) stage_q(k0 - 1);
   stage_q(k0);
   stage_q(k0 + 1);
   {
     const long long op = (long long)(k0 - 1) * P;
 #pragma unroll
     for (int q = 0; q < NE; q++) {
-      double v = pr[op + off[q]];
-      const int e = threadIdx.x + q * FT_N;
-      if (q < NE - 1 || has_last) {
-        if constexpr (CORR) {
-          v = corr_p(k0, e, v);
-          if (wpr[q]) st_nt(pr_out + op + off[q], v);
-        }
-        sp[k0 & 1][e] = v;
-      }
+      const double v = pr[op + off[q]];
+      if (q < NE - 1 || has_last) sp[k0 & 1][threadIdx.x + q * FT_N] = v;
     }
   }
   __syncthreads();
-  if constexpr (!CORR) {
-    if (k0 > 1) {
-      const int sm = (k0 - 1) % 3;
+  if (k0 > 1) {
+    const int sm = (k0 - 1) % 3;
 #pragma unroll
-      for (int u = 0; u < LPT; u++) {
-        cm[u][0] = sq[0][sm][base[u]];
-        cm[u][1] = sq[0][sm][base[u] + 1];
-        cm[u][2] = sq[1][sm][base[u]];
-        cm[u][3] = sq[2][sm][base[u]];
-        cm[u][4] = sq[2][sm][base[u] + FT_W];
-      }
-      __syncthreads();  // the first iteration overwrites that slot
+    for (int u = 0; u < LPT; u++) {
+      cm[u][0] = sq[0][sm][base[u]];
+      cm[u][1] = sq[0][sm][base[u] + 1];
+      cm[u][2] = sq[1][sm][base[u]];
+      cm[u][3] = sq[2][sm][base[u]];
+      cm[u][4] = sq[2][sm][base[u] + FT_W];
     }
+    __syncthreads();  // the first iteration overwrites that slot
   }
 
   for (int k = k0; k <= k1; k++) {
     // prefetch plane k+2 of the velocity, plane k+1 of the pressure and of
     // the RK histories.  In the last iteration these re-read planes just
     // read (their values are not used), so the loads carry no condition.
-    double nq[3][NE], np[NE], n1[LPT], n2[LPT], n3[LPT], nd[CORR ? NE2 : 1];
+    double nq[3][NE], np[NE], n1[LPT], n2[LPT], n3[LPT];
     const long long oq = (long long)min(k + 1, k1) * P;
     const long long op = (long long)min(k, k1 - 1) * P;
 #pragma unroll
@@ -899,12 +802,6 @@ DEVI void helm_rhs_body(
       nq[1][q] = qr[oq + off[q]];
       nq[2][q] = qz[oq + off[q]];
       np[q] = pr[op + off[q]];
-    }
-    if constexpr (CORR) {
-      // dph plane k+2 (clamped to nrm: beyond it no correction reads dph)
-      const long long od = (long long)(min(min(k + 2, k1 + 1), nrm) - 1) * P;
-#pragma unroll
-      for (int q = 0; q < NE2; q++) nd[q] = dph[od + off2[q]];
     }
     if (hist) {
 #pragma unroll
@@ -924,7 +821,7 @@ DEVI void helm_rhs_body(
 #pragma unroll
     for (int u = 0; u < LPT; u++) {
       if (!valid[u]) continue;
-      LAcc<!CORR> T, R, Z;
+      LAcc<true> T, R, Z;
       T.m = sq[0][sm]; T.c = sq[0][sc]; T.p = sq[0][sn]; T.base = base[u];
       R.m = sq[1][sm]; R.c = sq[1][sc]; R.p = sq[1][sn]; R.base = base[u];
       Z.m = sq[2][sm]; Z.c = sq[2][sc]; Z.p = sq[2][sn]; Z.base = base[u];
@@ -964,13 +861,11 @@ DEVI void helm_rhs_body(
         st_nt(yz + o, r * rw.sc_z + (am_z * qm + Z(0, 0, 0) + ap_z * qp));
       }
             pr_km[u] = pr_c;
-      if constexpr (!CORR) {
-        cm[u][0] = T(0, 0, 0);
-        cm[u][1] = T(0, 0, 1);
-        cm[u][2] = R(0, 0, 0);
-        cm[u][3] = Z(0, 0, 0);
-        cm[u][4] = Z(0, 1, 0);
-      }
+      cm[u][0] = T(0, 0, 0);
+      cm[u][1] = T(0, 0, 1);
+      cm[u][2] = R(0, 0, 0);
+      cm[u][3] = Z(0, 0, 0);
+      cm[u][4] = Z(0, 1, 0);
     }
     if (k == k1) break;
 #pragma unroll
@@ -979,25 +874,11 @@ DEVI void helm_rhs_body(
       h2[u] = n2[u];
       h3[u] = n3[u];
     }
-    if constexpr (CORR) {
-      // dph slot (k+2)%3 held plane k-1, last read before the previous barrier
-#pragma unroll
-      for (int q = 0; q < NE2; q++)
-        if (q < NE2 - 1 || has_last2) sd[(k + 2) % 3][threadIdx.x + q * FT_N] = nd[q];
-      // the ring slot of plane k-1 is read above, and the dph plane k+2 just
-      // written is read by the staging below
-      __syncthreads();
-    }
     const int s2 = (k + 2) % 3;
 #pragma unroll
     for (int q = 0; q < NE; q++) {
       const int e = threadIdx.x + q * FT_N;
       if (q < NE - 1 || has_last) {
-        if constexpr (CORR) {
-          corr_q(k + 2, e, nq[0][q], nq[1][q], nq[2][q]);
-          np[q] = corr_p(k + 1, e, np[q]);
-          if (wpr[q]) st_nt(pr_out + (long long)k * P + off[q], np[q]);
-        }
         sq[0][s2][e] = nq[0][q];
         sq[1][s2][e] = nq[1][q];
         sq[2][s2][e] = nq[2][q];
@@ -1008,11 +889,336 @@ DEVI void helm_rhs_body(
   }
 }
 
+// Even theta sizes: a thread owns two theta-adjacent lines, so that planes,
+// histories and results move as 16-byte pairs (the address unit takes a
+// 64-lane load or store 16 cycles whatever its width) and the two points
+// share the LDS reads and the sums that their stencils have in common.  A
+// block of 32*TJ threads owns a 64 (theta) x TJ (z) tile from plane k0 to k1.
+// CORR: qt, qr, qz hold the previous substep's velocity before its pressure
+// correction and pr its pressure before the correction; the correction (dph
+// of that substep) is applied to each plane as it is staged, from a ring of
+// dph planes with one more row of halo on either side, so the corrected
+// fields are the ones the per-substep path would have stored, bit for bit.
+// Against one line or two z-rows of lines per thread, with the correction:
+// 256x256x193 343 -> 318 us, 512x512x385 2576 -> 2491 us, 1024x1024x769 20.5
+// -> 17.95 ms (HBM bound at the larger sizes: 4.9 of the 5.7 TB/s that
+// fifteen streamed arrays reach).  The kernels ask for two waves per SIMD,
+// which the masked form leaves by a few registers when it is not asked to:
+// grooved walls, corrected, 192x128x129 125 us at one wave, 88 at two,
+// 256x256x193 447 and 335.
+// (The outermost column of the tile on either side is staged only to keep
+// pairs aligned; nothing reads it.)
+constexpr int PT_W = FT_I + 4, PT_P = PT_W / 2;  // tile row: i0-2 .. i0+65
+template <bool UNIFORM, int TJ, bool CORR>
+DEVI void helm_rhs_pair_body(
+    const int tile, const int k0, const int k1, const GridDev &g, const ImpArgs &a,
+    const double *__restrict__ qt, const double *__restrict__ qr, const double *__restrict__ qz,
+    const double *__restrict__ pr, double *__restrict__ ru1, double *__restrict__ ru2,
+    double *__restrict__ ru3, double *__restrict__ yt, double *__restrict__ yr,
+    double *__restrict__ yz, const unsigned char *__restrict__ icyl,
+    const unsigned char *__restrict__ ocyl, const RhsRow *__restrict__ rows, int ntx,
+    const CorrIn &ci, const double *__restrict__ dph, double *__restrict__ pr_out) {
+  constexpr int NT = 32 * TJ, S = PT_P * (TJ + 2), NE = (S + NT - 1) / NT;      // pairs
+  constexpr int S2 = PT_P * (TJ + 4), NE2 = (S2 + NT - 1) / NT;
+  __shared__ __align__(16) double sq[3][3][2 * S];  // field, ring slot, tile
+  __shared__ __align__(16) double sp[2][2 * S];     // pressure planes k and k+1
+  __shared__ __align__(16) double sd[CORR ? 3 : 1][CORR ? 2 * S2 : 2];  // dph planes (slot = plane % 3)
+  const int i0 = (tile % ntx) * FT_I, j0 = (tile / ntx) * TJ;
+  const int tx = threadIdx.x % 32, ty = threadIdx.x / 32;
+  const long long P = g.P;
+  auto ld2 = [](const double *p) { return *reinterpret_cast<const double2 *>(p); };
+  auto put2 = [](double *p, double2 v) { *reinterpret_cast<double2 *>(p) = v; };
+  // the pairs of the tile that this thread stages per plane: in the last
+  // chunk threads past S load a valid pair and do not store it, so every
+  // global load is unconditional
+  auto wrapped = [&](int row, int pair) {
+    int jj = j0 + row, ii = i0 - 2 + 2 * pair;
+    jj = ((jj % g.nzm) + g.nzm) % g.nzm;
+    ii = ((ii % g.nthm) + g.nthm) % g.nthm;
+    return jj * g.nthm + ii;
+  };
+  int off[NE], off2[CORR ? NE2 : 1];
+  bool wpr[NE];
+  const bool has_last = threadIdx.x + (NE - 1) * NT < S;
+  const bool has_last2 = threadIdx.x + (NE2 - 1) * NT < S2;
+#pragma unroll
+  for (int q = 0; q < NE; q++) {
+    const int e = threadIdx.x + q * NT, ee = e < S ? e : 0;
+    const int row = ee / PT_P, pair = ee % PT_P;
+    off[q] = wrapped(row - 1, pair);
+    // an interior pair, whose corrected pressure this thread writes
+    wpr[q] = CORR && e < S && row >= 1 && row <= TJ && pair >= 1 && pair <= 32 &&
+             j0 + row - 1 < g.nzm && i0 - 2 + 2 * pair < g.nthm;
+  }
+  if constexpr (CORR) {
+#pragma unroll
+    for (int q = 0; q < NE2; q++) {
+      const int e = threadIdx.x + q * NT, ee = e < S2 ? e : 0;
+      off2[q] = wrapped(ee / PT_P - 2, ee % PT_P);
+    }
+  }
+  // the corrected velocity of plane p at the tile pair e (correct_pair's
+  // arithmetic; q_r is zero on both walls)
+  auto corr_q = [&](int p, int e, double2 &vt, double2 &vr, double2 &vz) {
+    const int e2 = 2 * (e + PT_P);  // the same point in a dph plane
+    const double *dc = sd[CORR ? p % 3 : 0];
+    const double2 d = ld2(dc + e2);
+    if (p <= g.nrm) {
+      const double2 djm = ld2(dc + e2 - PT_W);
+      vt.x = corr_qt(g, p, vt.x, d.x, dc[e2 - 1], ci.dt, ci.al);
+      vt.y = corr_qt(g, p, vt.y, d.y, d.x, ci.dt, ci.al);
+      vz.x = corr_qz(g, vz.x, d.x, djm.x, ci.dt, ci.al);
+      vz.y = corr_qz(g, vz.y, d.y, djm.y, ci.dt, ci.al);
+    }
+    if (p == 1 || p >= g.nr) {
+      vr = make_double2(0.0, 0.0);
+    } else {
+      const double2 dkm = ld2(sd[CORR ? (p - 1) % 3 : 0] + e2);
+      vr.x = corr_qr(g, p, vr.x, d.x, dkm.x, ci.dt, ci.al);
+      vr.y = corr_qr(g, p, vr.y, d.y, dkm.y, ci.dt, ci.al);
+    }
+  };
+  // the corrected pressure of plane p <= nrm at the tile pair e
+  auto corr_p = [&](int p, int e, double2 v) {
+    const int e2 = 2 * (e + PT_P);
+    const double *dc = sd[CORR ? p % 3 : 0];
+    const double2 dkp = ld2(sd[CORR ? (p < g.nrm ? p + 1 : p) % 3 : 0] + e2);
+    const double2 dkm = ld2(sd[CORR ? (p > 1 ? p - 1 : p) % 3 : 0] + e2);
+    const double2 d = ld2(dc + e2), djm = ld2(dc + e2 - PT_W), djp = ld2(dc + e2 + PT_W);
+    return make_double2(
+        corr_pr(g, p, v.x, d.x, dc[e2 - 1], d.y, djm.x, djp.x, dkm.x, dkp.x, ci.be),
+        corr_pr(g, p, v.y, d.y, d.x, dc[e2 + 2], djm.y, djp.y, dkm.y, dkp.y, ci.be));
+  };
+  // stage dph plane p (clamped to 1..nrm: beyond it no correction reads dph)
+  auto stage_dph = [&](int p) {
+    const long long od = (long long)(min(max(p, 1), g.nrm) - 1) * P;
+    double2 t[CORR ? NE2 : 1];
+#pragma unroll
+    for (int q = 0; q < NE2; q++) t[q] = ld2(dph + od + off2[q]);
+#pragma unroll
+    for (int q = 0; q < NE2; q++)
+      if (q < NE2 - 1 || has_last2) put2(sd[(p + 3) % 3] + 2 * (threadIdx.x + q * NT), t[q]);
+  };
+  // stage plane p of the velocity (before the first iteration)
+  auto stage_q = [&](int p) {
+    const long long oq = (long long)(p - 1) * P;
+    double2 t[3][NE];
+#pragma unroll
+    for (int q = 0; q < NE; q++) {
+      t[0][q] = ld2(qt + oq + off[q]);
+      t[1][q] = ld2(qr + oq + off[q]);
+      t[2][q] = ld2(qz + oq + off[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < NE; q++)
+      if (q < NE - 1 || has_last) {
+        const int e = threadIdx.x + q * NT;
+        if constexpr (CORR) corr_q(p, e, t[0][q], t[1][q], t[2][q]);
+#pragma unroll
+        for (int f = 0; f < 3; f++) put2(sq[f][p % 3] + 2 * e, t[f][q]);
+      }
+  };
+  // the RK history ru enters as ro*ru only: with ro = 0 (the first RK3
+  // substep) it is not read at all
+  const bool hist = CORR || a.ro != 0.0;
+  const int nrm = g.nrm;
+  const int i = i0 + 2 * tx, j = j0 + ty;
+  const bool valid = i < g.nthm && j < g.nzm;
+  const long long l = valid ? (long long)j * g.nthm + i : 0;
+  const int base = (ty + 1) * PT_W + 2 * tx + 2;
+  // wall masks: bits 0, 1 the inner wall's at the two points, 2, 3 the outer's
+  int wall = 15;
+  if (!UNIFORM && valid) wall = icyl[l] + 2 * icyl[l + 1] + 4 * ocyl[l] + 8 * ocyl[l + 1];
+  const double2 zero = make_double2(0.0, 0.0);
+  double2 h1, h2, h3, pkm;
+  {
+    const long long o = (long long)(k0 - 1) * P + l;
+    h1 = hist ? ld2_nt(ru1 + o) : zero;
+    h2 = hist ? ld2_nt(ru2 + o) : zero;
+    h3 = hist ? ld2_nt(ru3 + o) : zero;
+    pkm = k0 > 1 ? ld2(pr + o - P) : zero;
+  }
+  // !CORR: plane k-1 values carried from the previous iteration (qt at
+  // theta, +1, +2; qr and qz at theta, +1; qz of row z+1), so that no thread
+  // reads the ring slot of plane k-1 and the staging of plane k+2 into it
+  // needs no barrier of its own
+  double cm[9] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  auto carry = [&](const double *t, const double *r, const double *z) {
+    cm[0] = t[base], cm[1] = t[base + 1], cm[2] = t[base + 2];
+    cm[3] = r[base], cm[4] = r[base + 1];
+    cm[5] = z[base], cm[6] = z[base + 1];
+    cm[7] = z[base + PT_W], cm[8] = z[base + PT_W + 1];
+  };
+  // planes k0-1 (if any), k0 and k0+1 of the velocity, k0 of the pressure
+  // and the pressure of k0-1 on the lines themselves.  CORR: with the dph
+  // planes that each of these corrections reads staged before it.
+  if constexpr (CORR) {
+    if (k0 > 1) {
+      stage_dph(k0 - 2);
+      stage_dph(k0 - 1);
+      stage_dph(k0);
+      __syncthreads();
+      stage_q(k0 - 1);
+      pkm = corr_p(k0 - 1, base / 2, pkm);
+      __syncthreads();
+      stage_dph(k0 + 1);
+    } else {
+      stage_dph(1);
+      stage_dph(2);
+    }
+    __syncthreads();
+  } else if (k0 > 1) {
+    stage_q(k0 - 1);
+  }
+  stage_q(k0);
+  stage_q(k0 + 1);
+  {
+    const long long op = (long long)(k0 - 1) * P;
+#pragma unroll
+    for (int q = 0; q < NE; q++) {
+      double2 v = ld2(pr + op + off[q]);
+      const int e = threadIdx.x + q * NT;
+      if (q < NE - 1 || has_last) {
+        if constexpr (CORR) {
+          v = corr_p(k0, e, v);
+          if (wpr[q]) st2_nt(pr_out + op + off[q], v.x, v.y);
+        }
+        put2(sp[k0 & 1] + 2 * e, v);
+      }
+    }
+  }
+  __syncthreads();
+  if constexpr (!CORR) {
+    if (k0 > 1) {
+      const int sm = (k0 - 1) % 3;
+      carry(sq[0][sm], sq[1][sm], sq[2][sm]);
+      __syncthreads();  // the first iteration overwrites that slot
+    }
+  }
+
+  for (int k = k0; k <= k1; k++) {
+    // prefetch plane k+2 of the velocity, plane k+1 of the pressure and of
+    // the RK histories.  In the last iteration these re-read planes just
+    // read (their values are not used), so the loads carry no condition.
+    double2 nq[3][NE], np[NE], n1 = zero, n2 = zero, n3 = zero, nd[CORR ? NE2 : 1];
+    const long long oq = (long long)min(k + 1, k1) * P;
+    const long long op = (long long)min(k, k1 - 1) * P;
+#pragma unroll
+    for (int q = 0; q < NE; q++) {
+      nq[0][q] = ld2(qt + oq + off[q]);
+      nq[1][q] = ld2(qr + oq + off[q]);
+      nq[2][q] = ld2(qz + oq + off[q]);
+      np[q] = ld2(pr + op + off[q]);
+    }
+    if constexpr (CORR) {
+      const long long od = (long long)(min(min(k + 2, k1 + 1), nrm) - 1) * P;
+#pragma unroll
+      for (int q = 0; q < NE2; q++) nd[q] = ld2(dph + od + off2[q]);
+    }
+    if (hist) {
+      n1 = ld2_nt(ru1 + op + l);
+      n2 = ld2_nt(ru2 + op + l);
+      n3 = ld2_nt(ru3 + op + l);
+    }
+    const int sm = (k + 2) % 3, sc = k % 3, sn = (k + 1) % 3;  // planes k-1, k, k+1
+    const HelmPlane hc = ldk_record(g.hp + k);
+    const RhsRow rw = ldk_record(rows + k);
+    if (valid) {
+      const double *spk = sp[k & 1];
+      const long long o = (long long)(k - 1) * P + l;
+      double e1[2], e2[2], e3[2], g1[2], g2[2], g3[2];
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const int b = base + u;
+        LAcc<!CORR, PT_W> T, R, Z;
+        T.m = sq[0][sm]; T.c = sq[0][sc]; T.p = sq[0][sn]; T.base = b;
+        R.m = sq[1][sm]; R.c = sq[1][sc]; R.p = sq[1][sn]; R.base = b;
+        Z.m = sq[2][sm]; Z.c = sq[2][sc]; Z.p = sq[2][sn]; Z.base = b;
+        T.m00 = cm[u]; T.m01 = cm[u + 1]; T.m10 = 0.0;
+        R.m00 = cm[3 + u]; R.m01 = R.m10 = 0.0;
+        Z.m00 = cm[5 + u]; Z.m01 = 0.0; Z.m10 = cm[7 + u];
+        const double fic = (double)(wall >> u & 1), foc = (double)(wall >> u >> 2 & 1);
+        const double pr_c = spk[b], pr_im = spk[b - 1], pr_jm = spk[b - PT_W];
+        // the matrix rows of q_theta and q_z next to a free-slip wall
+        double am_t = rw.am_t, ap_t = rw.ap_t, am_z = rw.am_z, ap_z = rw.ap_z;
+        if constexpr (!UNIFORM) {
+          if (k == 1 && !(wall >> u & 1)) ap_t = rw.x_t, ap_z = rw.x_z;
+          if (k == nrm && !(wall >> u & 4)) am_t = rw.x_t, am_z = rw.x_z;
+        }
+        // q_theta
+        e1[u] = explicit_qt_g(g, hc, T, R, Z, k);
+        const double tm = (k > 1) ? T(-1, 0, 0) : 0.0, tp = (k < nrm) ? T(1, 0, 0) : 0.0;
+        double r = rhs_qt<UNIFORM>(g, hc, a, k, tm, T(0, 0, 0), tp, pr_c, pr_im, e1[u],
+                                   u ? h1.y : h1.x, fic, foc);
+        if (k == 1) r = r + a.bc1;
+        g1[u] = r * rw.sc_t + (am_t * tm + T(0, 0, 0) + ap_t * tp);
+        // q_r (planes 2..nrm; the walls have no row)
+        if (k >= 2) {
+          e2[u] = explicit_qr_g(g, hc, T, R, Z, k);
+          r = rhs_qr(hc, a, R(-1, 0, 0), R(0, 0, 0), R(1, 0, 0), pr_c, u ? pkm.y : pkm.x, e2[u],
+                     u ? h2.y : h2.x);
+          g2[u] = r * rw.sc_r + (rw.am_r * R(-1, 0, 0) + R(0, 0, 0) + rw.ap_r * R(1, 0, 0));
+        }
+        // q_z
+        e3[u] = explicit_qz_g(g, hc, T, R, Z, k);
+        const double zm = (k > 1) ? Z(-1, 0, 0) : 0.0, zp = (k < nrm) ? Z(1, 0, 0) : 0.0;
+        r = rhs_qz<UNIFORM>(g, hc, a, k, zm, Z(0, 0, 0), zp, pr_c, pr_jm, e3[u], u ? h3.y : h3.x,
+                            fic, foc);
+        g3[u] = r * rw.sc_z + (am_z * zm + Z(0, 0, 0) + ap_z * zp);
+        if (u)
+          pkm.y = pr_c;
+        else
+          pkm.x = pr_c;
+      }
+      st2_nt(ru1 + o, e1[0], e1[1]);
+      st2_nt(yt + o, g1[0], g1[1]);
+      if (k >= 2) {
+        st2_nt(ru2 + o, e2[0], e2[1]);
+        st2_nt(yr + o, g2[0], g2[1]);
+      }
+      st2_nt(ru3 + o, e3[0], e3[1]);
+      st2_nt(yz + o, g3[0], g3[1]);
+      if constexpr (!CORR) carry(sq[0][sc], sq[1][sc], sq[2][sc]);
+    }
+    if (k == k1) break;
+    h1 = n1;
+    h2 = n2;
+    h3 = n3;
+    if constexpr (CORR) {
+      // dph slot (k+2)%3 held plane k-1, last read before the previous barrier
+#pragma unroll
+      for (int q = 0; q < NE2; q++)
+        if (q < NE2 - 1 || has_last2) put2(sd[(k + 2) % 3] + 2 * (threadIdx.x + q * NT), nd[q]);
+      // the ring slot of plane k-1 is read above, and the dph plane k+2 just
+      // written is read by the staging below
+      __syncthreads();
+    }
+    const int s2 = (k + 2) % 3;
+#pragma unroll
+    for (int q = 0; q < NE; q++) {
+      const int e = threadIdx.x + q * NT;
+      if (q < NE - 1 || has_last) {
+        if constexpr (CORR) {
+          corr_q(k + 2, e, nq[0][q], nq[1][q], nq[2][q]);
+          np[q] = corr_p(k + 1, e, np[q]);
+          if (wpr[q]) st2_nt(pr_out + (long long)k * P + off[q], np[q].x, np[q].y);
+        }
+#pragma unroll
+        for (int f = 0; f < 3; f++) put2(sq[f][s2] + 2 * e, nq[f][q]);
+        put2(sp[(k + 1) & 1] + 2 * e, np[q]);
+      }
+    }
+    __syncthreads();
+  }
+}
+
 // Planes k0..k1 of segment s of ns.
 DEVI int seg_first(int s, int ns, int nrm) { return 1 + (int)(((long long)s * nrm) / ns); }
 
-template <bool UNIFORM, int LPT, bool CORR>
-__global__ __launch_bounds__(FT_N) void k_helm_rhs(
+// PAIR: the pair form (even nthm), tiles of 4*LPT rows; otherwise LPT lines
+// per thread.
+template <bool UNIFORM, int LPT, bool CORR, bool PAIR>
+__global__ __launch_bounds__(PAIR ? 128 * LPT : FT_N, 2) void k_helm_rhs(
     GridDev g, ImpArgs a, const double *__restrict__ qt, const double *__restrict__ qr,
     const double *__restrict__ qz, const double *__restrict__ pr, double *__restrict__ ru1,
     double *__restrict__ ru2, double *__restrict__ ru3, double *__restrict__ yt,
@@ -1020,18 +1226,22 @@ __global__ __launch_bounds__(FT_N) void k_helm_rhs(
     const unsigned char *__restrict__ ocyl, const RhsRow *__restrict__ rows, int ntx, int ntz,
     int nseg, CorrIn ci, const double *__restrict__ dph, double *__restrict__ pr_out) {
   const int lin = xcd_tile(blockIdx.x, gridDim.x), seg = lin / (ntx * ntz);
-  helm_rhs_body<UNIFORM, LPT, CORR>(lin - seg * (ntx * ntz), seg_first(seg, nseg, g.nrm),
-                                    seg_first(seg + 1, nseg, g.nrm) - 1, g, a, qt, qr, qz, pr,
-                                    ru1, ru2, ru3, yt, yr, yz, icyl, ocyl, rows, ntx, ci, dph,
-                                    pr_out);
+  const int tile = lin - seg * (ntx * ntz);
+  const int k0 = seg_first(seg, nseg, g.nrm), k1 = seg_first(seg + 1, nseg, g.nrm) - 1;
+  if constexpr (PAIR)
+    helm_rhs_pair_body<UNIFORM, 4 * LPT, CORR>(tile, k0, k1, g, a, qt, qr, qz, pr, ru1, ru2, ru3,
+                                               yt, yr, yz, icyl, ocyl, rows, ntx, ci, dph, pr_out);
+  else
+    helm_rhs_body<UNIFORM, LPT>(tile, k0, k1, g, a, qt, qr, qz, pr, ru1, ru2, ru3, yt, yr, yz, icyl,
+                                ocyl, rows, ntx);
 }
 
 // Grouped: blockIdx.x = tile and segment, blockIdx.y = instance of the shape
 // group; the XCD remap runs over the flattened index.
-template <bool UNIFORM, int LPT, bool CORR>
-__global__ __launch_bounds__(FT_N) void k_helm_rhs_g(const StepDesc *__restrict__ tab,
-                                                    const BatchDyn *__restrict__ dyn, int ns,
-                                                    int ntx, int ntz, int nseg) {
+template <bool UNIFORM, int LPT, bool CORR, bool PAIR>
+__global__ __launch_bounds__(PAIR ? 128 * LPT : FT_N, 2) void k_helm_rhs_g(
+    const StepDesc *__restrict__ tab, const BatchDyn *__restrict__ dyn, int ns, int ntx, int ntz,
+    int nseg) {
   const int lin = xcd_tile(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
   const int inst = lin / (int)gridDim.x, rest = lin - inst * (int)gridDim.x;
   const int seg = rest / (ntx * ntz), tile = rest - seg * (ntx * ntz);
@@ -1040,13 +1250,18 @@ __global__ __launch_bounds__(FT_N) void k_helm_rhs_g(const StepDesc *__restrict_
   ImpArgs a = d.a;
   a.vwall_in = glob(dyn)[inst].vwall[ns - 1];
   a.bc1 = glob(dyn)[inst].bc1[ns - 1];
-  const CorrIn ci{d.dt, d.corr_al, d.beta};
-  helm_rhs_body<UNIFORM, LPT, CORR>(
-      tile, seg_first(seg, nseg, d.g.nrm), seg_first(seg + 1, nseg, d.g.nrm) - 1, glob(d.g), a,
-      glob(d.f[TC_QT]), glob(d.f[TC_QR]), glob(d.f[TC_QZ]), glob(d.pr_in), glob(d.f[TC_RU1]),
-      glob(d.f[TC_RU2]), glob(d.f[TC_RU3]), glob(d.f[TC_RHS]), glob(d.f[TC_DQ]),
-      glob(d.f[TC_QCAP]), glob(d.icyl), glob(d.ocyl), glob(d.rows), ntx, ci, glob(d.f[TC_DPH]),
-      glob(d.pr_out));
+  const int k0 = seg_first(seg, nseg, d.g.nrm), k1 = seg_first(seg + 1, nseg, d.g.nrm) - 1;
+  if constexpr (PAIR)
+    helm_rhs_pair_body<UNIFORM, 4 * LPT, CORR>(
+        tile, k0, k1, glob(d.g), a, glob(d.f[TC_QT]), glob(d.f[TC_QR]), glob(d.f[TC_QZ]),
+        glob(d.pr_in), glob(d.f[TC_RU1]), glob(d.f[TC_RU2]), glob(d.f[TC_RU3]), glob(d.f[TC_RHS]),
+        glob(d.f[TC_DQ]), glob(d.f[TC_QCAP]), glob(d.icyl), glob(d.ocyl), glob(d.rows), ntx,
+        CorrIn{d.dt, d.corr_al, d.beta}, glob(d.f[TC_DPH]), glob(d.pr_out));
+  else
+    helm_rhs_body<UNIFORM, LPT>(
+        tile, k0, k1, glob(d.g), a, glob(d.f[TC_QT]), glob(d.f[TC_QR]), glob(d.f[TC_QZ]),
+        glob(d.pr_in), glob(d.f[TC_RU1]), glob(d.f[TC_RU2]), glob(d.f[TC_RU3]), glob(d.f[TC_RHS]),
+        glob(d.f[TC_DQ]), glob(d.f[TC_QCAP]), glob(d.icyl), glob(d.ocyl), glob(d.rows), ntx);
 }
 
 static ImpArgs imp_args(const tc_ctx *c) {
@@ -1159,6 +1374,7 @@ void launch_implicit_qt(tc_ctx *c) { launch_implicit<0>(c, "implicit_qt", TC_QT,
 void launch_implicit_qr(tc_ctx *c) { launch_implicit<1>(c, "implicit_qr", TC_QR, TC_DPH, TC_RU2); }
 void launch_implicit_qz(tc_ctx *c) { launch_implicit<2>(c, "implicit_qz", TC_QZ, TC_QCAP, TC_RU3); }
 
+static unsigned helm_threads(const tc_ctx *c, int lpt) { return c->nthm % 2 == 0 ? 128 * lpt : FT_N; }
 static long long helm_tiles(const tc_ctx *c, int lpt) {
   return (long long)((c->nthm + FT_I - 1) / FT_I) * ((c->nzm + FT_J * lpt - 1) / (FT_J * lpt));
 }
@@ -1167,9 +1383,9 @@ static long long helm_tiles(const tc_ctx *c, int lpt) {
 // takes (rounds of resident blocks) x (planes per segment and about three
 // that a segment stages before its first), and its blocks, which run apart,
 // end within about a quarter of a segment of each other; the segment count
-// with the least of that, of at least two planes each.  Measured, one
-// segment against the chosen count: 64x64x65 133 -> 15 us, 256x256x193
-// 400 -> 212 us, 512x512x385 (two lines per thread) 1775 -> 1674 us.
+// with the least of that, of at least two planes each.  Measured with one
+// line per thread, one segment against the chosen count: 64x64x65 133 -> 15
+// us, 256x256x193 400 -> 212 us, 512x512x385 1775 -> 1674 us.
 static int helm_segments(const tc_ctx *c, int lpt, bool corr, int n) {
   const long long tiles = n * helm_tiles(c, lpt), slots = c->helm_slots[corr];
   int best = 1;
@@ -1191,7 +1407,8 @@ template <bool U, int LPT, bool CORR>
 static void launch_rhs(tc_ctx *c, const double *pr, const CorrIn &ci, double *pr_out) {
   const int ntx = (c->nthm + FT_I - 1) / FT_I, ntz = (c->nzm + FT_J * LPT - 1) / (FT_J * LPT);
   const int nseg = helm_segments(c, LPT, CORR, 1);
-  hipLaunchKernelGGL((k_helm_rhs<U, LPT, CORR>), dim3((unsigned)(ntx * ntz * nseg)), dim3(FT_N), 0,
+  auto *kernel = c->nthm % 2 == 0 ? k_helm_rhs<U, LPT, CORR, true> : k_helm_rhs<U, LPT, false, false>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(ntx * ntz * nseg)), dim3(helm_threads(c, LPT)), 0,
                      c->stream, c->gd, imp_args(c), c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], pr,
                      c->f[TC_RU1], c->f[TC_RU2], c->f[TC_RU3], c->f[TC_RHS], c->f[TC_DQ],
                      c->f[TC_QCAP], c->mask, c->mask + c->P, rhs_rows(c, c->ns), ntx, ntz, nseg,
@@ -1200,32 +1417,40 @@ static void launch_rhs(tc_ctx *c, const double *pr, const CorrIn &ci, double *pr
 
 // blocks of the fused front that one compute unit holds (asked once: every
 // device this library is built for is alike)
-template <int LPT, bool CORR>
+template <int LPT, bool CORR, bool PAIR>
 static int resident_blocks(int cus) {
   static const int per_cu = [] {
     int n = 0;
-    const hipError_t e =
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_helm_rhs<true, LPT, CORR>, FT_N, 0);
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        &n, k_helm_rhs<true, LPT, CORR, PAIR>, PAIR ? 128 * LPT : FT_N, 0);
     return e == hipSuccess && n > 0 ? n : 2;
   }();
   return per_cu * cus;
 }
 
-// Lines per thread (lpt, 0: chosen here) and the blocks of the fused front
-// resident at once.  Two lines per thread stage 1.29 elements per point
-// instead of 1.55, but halve the tiles; they are the default where their
-// tiles fill the device in segments of 32 planes.  One against two lines:
-// 64x64x65 15 / 17 us, 192x128x129 73 / 73, 375x240x151 362 / 336,
-// 512x512x385 1721 / 1674 (with the correction 2650 / 2581).
+// Schedule of the fused front (lpt 0: chosen here) and its blocks resident
+// at once.  Even nthm, the pair form: tiles of 4*lpt rows; eight rows stage
+// 1.29 elements per point instead of 1.55 and are the faster at every size
+// (us, four / eight, with the correction from the second on: 64x64x65 17.1 /
+// 16.9, 128x128x97 52.9 / 49.7, 192x128x129 90 / 82, 256x256x193 358 / 313,
+// 512x512x385 2688 / 2558).  Odd nthm: lpt lines per thread, two where their
+// tiles fill the device in segments of 32 planes (375x240x151 362 / 336).
 void choose_helm_schedule(tc_ctx *c, int lpt) {
   int dev = 0, cus = 0;
   hipGetDevice(&dev);
   hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   if (cus <= 0) cus = 256;
-  if (lpt == 0) lpt = helm_tiles(c, 2) * (c->nrm / 32) >= resident_blocks<2, true>(cus) ? 2 : 1;
+  const bool pair = c->nthm % 2 == 0;
+  if (lpt == 0)
+    lpt = pair || helm_tiles(c, 2) * (c->nrm / 32) >= resident_blocks<2, false, false>(cus) ? 2 : 1;
   c->helm_lpt = lpt;
-  c->helm_slots[0] = lpt == 2 ? resident_blocks<2, false>(cus) : resident_blocks<1, false>(cus);
-  c->helm_slots[1] = lpt == 2 ? resident_blocks<2, true>(cus) : resident_blocks<1, true>(cus);
+  if (pair) {
+    c->helm_slots[0] = lpt == 2 ? resident_blocks<2, false, true>(cus) : resident_blocks<1, false, true>(cus);
+    c->helm_slots[1] = lpt == 2 ? resident_blocks<2, true, true>(cus) : resident_blocks<1, true, true>(cus);
+  } else {
+    c->helm_slots[0] = c->helm_slots[1] =
+        lpt == 2 ? resident_blocks<2, false, false>(cus) : resident_blocks<1, false, false>(cus);
+  }
 }
 
 void launch_helmholtz_fused(tc_ctx *c) {
@@ -2220,12 +2445,11 @@ static void launch_rhs_g(tc_ctx *c, const StepDesc *tab, const BatchDyn *dyn, in
   const int ntx = (c->nthm + FT_I - 1) / FT_I, ntz = (c->nzm + FT_J * LPT - 1) / (FT_J * LPT);
   const int nseg = helm_segments(c, LPT, corr, n);
   const dim3 grid((unsigned)(ntx * ntz * nseg), (unsigned)n);
-  if (corr)
-    hipLaunchKernelGGL((k_helm_rhs_g<U, LPT, true>), grid, dim3(FT_N), 0, st, tab, dyn, ns, ntx, ntz,
-                       nseg);
-  else
-    hipLaunchKernelGGL((k_helm_rhs_g<U, LPT, false>), grid, dim3(FT_N), 0, st, tab, dyn, ns, ntx,
-                       ntz, nseg);
+  // (a corrected launch has an even nthm, defers_correction)
+  auto *kernel = corr ? k_helm_rhs_g<U, LPT, true, true>
+                      : (c->nthm % 2 == 0 ? k_helm_rhs_g<U, LPT, false, true>
+                                          : k_helm_rhs_g<U, LPT, false, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(helm_threads(c, LPT)), 0, st, tab, dyn, ns, ntx, ntz, nseg);
 }
 
 template <bool U>
