@@ -204,10 +204,10 @@ void launch_explicit_qz(tc_ctx *c) {
 // Helmholtz solves.  The LU factors (dgttrf with partial pivoting of the
 // row-normalised matrices of SolveImpEqnUpdate_*) do not depend on the line
 // (j, i) except through the wall masks, so they come from a per-substep
-// table with one entry per mask combination.  One radial line per lane;
-// lanes run along theta so every plane access is coalesced.  The forward
-// substitution is streamed while the right-hand side is produced; its output
-// y is written to a scratch field and read back by the backward substitution.
+// table with one entry per mask combination.  Lanes run along theta so every
+// plane access is coalesced.  The right-hand sides are formed point by point
+// in one kernel and written to a scratch field; a second kernel reads them
+// back and solves, each line's rows in registers.
 // ---------------------------------------------------------------------------
 
 struct LUView {
