@@ -156,6 +156,13 @@ DEVI double explicit_qz_g(const GridDev &g, const HelmPlane &c, const A &T, cons
   return -(h31 + h32 + h33) + dqz1 + dqz2;
 }
 
+template <int WHICH, class A>
+DEVI double explicit_g(const GridDev &g, const HelmPlane &c, const A &T, const A &R, const A &Z, int kc) {
+  if constexpr (WHICH == 0) return explicit_qt_g(g, c, T, R, Z, kc);
+  else if constexpr (WHICH == 1) return explicit_qr_g(g, c, T, R, Z, kc);
+  else return explicit_qz_g(g, c, T, R, Z, kc);
+}
+
 template <int WHICH>
 __global__ __launch_bounds__(256) void k_explicit(GridDev g, const double *__restrict__ qt,
                                                   const double *__restrict__ qr,
@@ -167,38 +174,74 @@ __global__ __launch_bounds__(256) void k_explicit(GridDev g, const double *__res
   const int kc = blockIdx.z + (WHICH == 1 ? 2 : 1);
   const GAcc T = gacc(g, qt, kc, j, i), R = gacc(g, qr, kc, j, i), Z = gacc(g, qz, kc, j, i);
   const HelmPlane c = g.hp[kc];
-  double v;
-  if (WHICH == 0)
-    v = explicit_qt_g(g, c, T, R, Z, kc);
-  else if (WHICH == 1)
-    v = explicit_qr_g(g, c, T, R, Z, kc);
-  else
-    v = explicit_qz_g(g, c, T, R, Z, kc);
-  out[IX(g, kc, j, i)] = v;
+  out[IX(g, kc, j, i)] = explicit_g<WHICH>(g, c, T, R, Z, kc);
+}
+
+// Point U (0, 1) of a theta pair (i, i+1), i even: the pair itself is one
+// 16-byte load, which the two points share, as they do the outer neighbours.
+template <int U>
+struct PairAcc {
+  const double *__restrict__ a;
+  long long base, P;  // IX(k, j, i)
+  int jm, jp, im, ip;  // offsets of rows j-1, j+1, of points i-1, i+2
+  DEVI double operator()(int dk, int dj, int di) const {
+    const double *p = a + (base + dk * P + (dj < 0 ? jm : (dj > 0 ? jp : 0)));
+    const int e = U + di;
+    if (e < 0) return p[im];
+    if (e > 1) return p[ip];
+    const double2 v = *reinterpret_cast<const double2 *>(p);
+    return e ? v.y : v.x;
+  }
+};
+
+// Even nthm: a theta pair per thread, pairs of a plane in one row so that no
+// lane idles at the end of a theta line.  The 17 loads of 8 bytes a point,
+// 16 cycles of the address unit each, bounded the one-point form:
+// 256x256x193, q_theta / q_r / q_z 132 / 130 / 131 us, in pairs 92 / 109 / 98
+// (4.4 / 3.7 / 4.1 TB/s).  Contiguous planes per XCD gave nothing (92 / 112 /
+// 101 us).  Odd nthm, whose rows are not 16-byte aligned, keeps one point.
+template <int WHICH>
+__global__ __launch_bounds__(256) void k_explicit2(GridDev g, const double *__restrict__ qt,
+                                                   const double *__restrict__ qr,
+                                                   const double *__restrict__ qz,
+                                                   double *__restrict__ out) {
+  const int n = g.nthm, h = n / 2, l = blockIdx.x * 256 + threadIdx.x;
+  const int j = l / h, i = 2 * (l - j * h);
+  if (j >= g.nzm) return;
+  const int kc = blockIdx.y + (WHICH == 1 ? 2 : 1);
+  const long long base = IX(g, kc, j, i);
+  const int jm = (wrap_m(j, g.nzm) - j) * n, jp = (wrap_p(j, g.nzm) - j) * n;
+  const int im = wrap_m(i, n) - i, ip = wrap_p(i + 1, n) - i;
+  const HelmPlane c = g.hp[kc];
+  auto at = [&](auto u, const double *f) {
+    return PairAcc<decltype(u)::value>{f, base, g.P, jm, jp, im, ip};
+  };
+  using U0 = std::integral_constant<int, 0>;
+  using U1 = std::integral_constant<int, 1>;
+  const double v0 = explicit_g<WHICH>(g, c, at(U0{}, qt), at(U0{}, qr), at(U0{}, qz), kc);
+  const double v1 = explicit_g<WHICH>(g, c, at(U1{}, qt), at(U1{}, qr), at(U1{}, qz), kc);
+  *reinterpret_cast<double2 *>(out + base) = make_double2(v0, v1);
 }
 
 static dim3 point_grid(const tc_ctx *c, int planes) {
   return dim3((unsigned)((c->nthm + 63) / 64), (unsigned)((c->nzm + 3) / 4), (unsigned)planes);
 }
 
-void launch_explicit_qt(tc_ctx *c) {
-  timer_begin(c, "explicit_qt");
-  hipLaunchKernelGGL(k_explicit<0>, point_grid(c, c->nrm), dim3(64, 4), 0, c->stream, c->gd,
-                     c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->f[TC_DQ]);
+template <int WHICH>
+static void launch_explicit(tc_ctx *c, const char *name, int out) {
+  const int planes = WHICH == 1 ? c->nrm - 1 : c->nrm;
+  timer_begin(c, name);
+  if (c->nthm % 2 == 0)
+    hipLaunchKernelGGL(k_explicit2<WHICH>, dim3((unsigned)((c->P / 2 + 255) / 256), (unsigned)planes),
+                       dim3(256), 0, c->stream, c->gd, c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->f[out]);
+  else
+    hipLaunchKernelGGL(k_explicit<WHICH>, point_grid(c, planes), dim3(64, 4), 0, c->stream, c->gd,
+                       c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->f[out]);
   timer_end(c);
 }
-void launch_explicit_qr(tc_ctx *c) {
-  timer_begin(c, "explicit_qr");
-  hipLaunchKernelGGL(k_explicit<1>, point_grid(c, c->nrm - 1), dim3(64, 4), 0, c->stream, c->gd,
-                     c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->f[TC_DPH]);
-  timer_end(c);
-}
-void launch_explicit_qz(tc_ctx *c) {
-  timer_begin(c, "explicit_qz");
-  hipLaunchKernelGGL(k_explicit<2>, point_grid(c, c->nrm), dim3(64, 4), 0, c->stream, c->gd,
-                     c->f[TC_QT], c->f[TC_QR], c->f[TC_QZ], c->f[TC_QCAP]);
-  timer_end(c);
-}
+void launch_explicit_qt(tc_ctx *c) { launch_explicit<0>(c, "explicit_qt", TC_DQ); }
+void launch_explicit_qr(tc_ctx *c) { launch_explicit<1>(c, "explicit_qr", TC_DPH); }
+void launch_explicit_qz(tc_ctx *c) { launch_explicit<2>(c, "explicit_qz", TC_QCAP); }
 
 // ---------------------------------------------------------------------------
 // Helmholtz solves.  The LU factors (dgttrf with partial pivoting of the
