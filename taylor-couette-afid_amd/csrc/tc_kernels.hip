@@ -413,7 +413,14 @@ DEVI double rlane(double v, int i) {
 
 // comp: 0 q_theta, 1 q_r (rows 2..nrm; both walls are set to zero), 2 q_z.
 // lu: the line's table, the same for all lines of the block with UNIFORM.
-template <int R, bool UNIFORM, bool FOLD>
+// CHUNKS: lines of more rows than the block's registers hold (R a wave) go
+// in chunks, the first of what the full ones leave over.  L needs only the
+// value that enters a chunk, so the chunks are read downwards once for those
+// (kept in LDS), the last one is solved while it is held, and the others are
+// read a second time on the way up: 1025 rows move 6.7 passes instead of 6.
+// The serial form, 12 passes and one dependent chain a line, took 1337 us at
+// 256x256x1025 and 5450 us at 512x512x1025; this one takes 820 and 3533.
+template <int R, bool UNIFORM, bool FOLD, bool CHUNKS>
 DEVI void helm_solve_lines(const long long lgrp, const int comp, const GridDev &g,
                            double *__restrict__ q, const double *__restrict__ y,
                            const double *__restrict__ lu, double *ex) {
@@ -423,98 +430,131 @@ DEVI void helm_solve_lines(const long long lgrp, const int comp, const GridDev &
   const bool ok = l < P;
   const long long lc = ok ? l : P - 1;
   const int first = comp == 1 ? 1 : 0, n = g.nrm - first, last = first + n - 1;
-  const int lo = first + p * n / NS, S = first + (p + 1) * n / NS - lo;
   const LUView T = lu_view(lu);
-  // -dl_(r-1), rd_r and -du_r rd_r of row lo + i (UNIFORM: of rows lo + lane
-  // and, past 64 rows, lo + 64 + lane, loaded before the rows so that their
-  // latency is not behind them).  Past the segment's S rows they are those
-  // of rows that pass a value on unchanged in both sweeps (right-hand side
-  // zero), so the sweeps carry no conditions.
-  constexpr int NK = (R + 63) / 64;
-  double kdl[NK], kdu[NK], krd[NK];
-  if constexpr (UNIFORM) {
+  double *exc = ex, *exw = ex + NS * 64;  // outgoing values and factors, L
+  double *uxc = ex + 2 * NS * 64, *uxw = ex + 3 * NS * 64;  // and U
+  double *enter = ex + 4 * NS * 64;       // CHUNKS: value entering each chunk
+  const int cap = R * NS, nc = CHUNKS ? (n + cap - 1) / cap : 1, n0 = n - (nc - 1) * cap;
+  if (CHUNKS && p == 0) enter[lane] = 0.0;
+  double below = 0.0;  // solution of the row below the chunk
+  for (int pass = 0; pass < 2 * nc - 1; pass++) {
+    const int ch = pass < nc ? pass : 2 * (nc - 1) - pass;
+    const int r0 = first + (ch > 0 ? n0 + (ch - 1) * cap : 0), rn = ch > 0 ? cap : n0;
+    const int lo = r0 + p * rn / NS, S = r0 + (p + 1) * rn / NS - lo, Sm = max(S - 1, 0);
+    // -dl_(r-1), rd_r and -du_r rd_r of row lo + i (UNIFORM: of rows lo + lane
+    // and, past 64 rows, lo + 64 + lane, loaded before the rows so that their
+    // latency is not behind them).  Past the segment's S rows they are those
+    // of rows that pass a value on unchanged in both sweeps (right-hand side
+    // zero), so the sweeps carry no conditions.
+    constexpr int NK = (R + 63) / 64;
+    double kdl[NK], kdu[NK], krd[NK];
+    if constexpr (UNIFORM) {
 #pragma unroll
-    for (int u = 0; u < NK; u++) {
-      const int r = lo + min(lane + 64 * u, S - 1);
-      kdl[u] = T.dl(max(r - 1, 0));
-      kdu[u] = T.du(r);
-      krd[u] = T.rd(r);
+      for (int u = 0; u < NK; u++) {
+        const int r = lo + min(lane + 64 * u, Sm);
+        kdl[u] = T.dl(max(r - 1, 0));
+        kdu[u] = T.du(r);
+        krd[u] = T.rd(r);
+      }
     }
-  }
-  double v[R];
-  {
-    const double *yp = y + (long long)lo * P + lc;
+    double v[R];
+    {
+      const double *yp = y + (long long)lo * P + lc;
+      if constexpr (CHUNKS) {
+        constexpr int B = 20;  // the first chunk's segments may be short
+        static_assert(R % B == 0, "row batches");
 #pragma unroll
-    for (int i = 0; i < R; i++) v[i] = ld_nt(yp + (long long)min(i, S - 1) * P);
-  }
-  if constexpr (UNIFORM) {
+        for (int b = 0; b < R; b += B) {
+          if (b < S) {
 #pragma unroll
-    for (int u = 0; u < NK; u++) {
-      const int i = lane + 64 * u, r = lo + i;
-      kdl[u] = i < S ? (r > first ? -kdl[u] : 0.0) : 1.0;
-      kdu[u] = i < S ? (r < last ? -kdu[u] * krd[u] : 0.0) : 1.0;
-      krd[u] = i < S ? krd[u] : 0.0;
+            for (int i = b; i < b + B; i++) v[i] = yp[(long long)min(i, Sm) * P];
+          } else {
+#pragma unroll
+            for (int i = b; i < b + B; i++) v[i] = 0.0;
+          }
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < R; i++) v[i] = ld_nt(yp + (long long)min(i, Sm) * P);
+      }
     }
-  }
-  auto dl = [&](int i) {
-    if constexpr (UNIFORM) return rlane(kdl[i >> 6], i & 63);
-    else return lo + i > first ? -T.dl(lo + i - 1) : 0.0;
-  };
-  auto rd = [&](int i) {
-    if constexpr (UNIFORM) return rlane(krd[i >> 6], i & 63);
-    else return T.rd(lo + i);
-  };
-  auto ud = [&](int i) {
-    if constexpr (UNIFORM) return rlane(kdu[i >> 6], i & 63);
-    else return lo + i < last ? -T.du(lo + i) * T.rd(lo + i) : 0.0;
-  };
-  double *exc = ex, *exw = ex + NS * 64;  // outgoing values and factors
-  double c = 0.0, w = 1.0;
+    if constexpr (UNIFORM) {
 #pragma unroll
-  for (int i = 0; i < R; i++) {
-    if (!UNIFORM && i >= S) continue;
-    const double d = dl(i);
-    c = (i < S ? v[i] : 0.0) + d * c;
-    v[i] = c;
-    w = w * d;
-  }
-  exc[p * 64 + lane] = c;
-  exw[p * 64 + lane] = w;
-  __syncthreads();
-  w = 0.0;
-  for (int s = 0; s < p; s++) w = exc[s * 64 + lane] + exw[s * 64 + lane] * w;
-#pragma unroll
-  for (int i = 0; i < R; i++) {
-    if (!UNIFORM && i >= S) continue;
-    w = w * dl(i);
-    v[i] = v[i] + w;
-  }
-  exc += 2 * NS * 64;
-  exw += 2 * NS * 64;
-  c = 0.0;
-  w = 1.0;
-#pragma unroll
-  for (int i = R - 1; i >= 0; i--) {
-    if (!UNIFORM && i >= S) continue;
-    const double u = ud(i);
-    c = v[i] * rd(i) + u * c;
-    v[i] = c;
-    w = w * u;
-  }
-  exc[p * 64 + lane] = c;
-  exw[p * 64 + lane] = w;
-  __syncthreads();
-  w = 0.0;
-  for (int s = NS - 1; s > p; s--) w = exc[s * 64 + lane] + exw[s * 64 + lane] * w;
-  double *qp = q + (long long)lo * P + l;
-#pragma unroll
-  for (int i = R - 1; i >= 0; i--) {
-    if (!UNIFORM && i >= S) continue;
-    w = w * ud(i);
-    if (i < S && ok) {
-      double *o = qp + (long long)i * P;
-      st_nt(o, FOLD ? v[i] + w : *o + (v[i] + w));
+      for (int u = 0; u < NK; u++) {
+        const int i = lane + 64 * u, r = lo + i;
+        kdl[u] = i < S ? (r > first ? -kdl[u] : 0.0) : 1.0;
+        kdu[u] = i < S ? (r < last ? -kdu[u] * krd[u] : 0.0) : 1.0;
+        krd[u] = i < S ? krd[u] : 0.0;
+      }
     }
+    auto dl = [&](int i) {
+      if constexpr (UNIFORM) return rlane(kdl[i >> 6], i & 63);
+      else return lo + i > first ? -T.dl(lo + i - 1) : 0.0;
+    };
+    auto rd = [&](int i) {
+      if constexpr (UNIFORM) return rlane(krd[i >> 6], i & 63);
+      else return T.rd(lo + i);
+    };
+    auto ud = [&](int i) {
+      if constexpr (UNIFORM) return rlane(kdu[i >> 6], i & 63);
+      else return lo + i < last ? -T.du(lo + i) * T.rd(lo + i) : 0.0;
+    };
+    double c = 0.0, w = 1.0;
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+      if (!UNIFORM && i >= S) continue;
+      const double d = dl(i);
+      c = (i < S ? v[i] : 0.0) + d * c;
+      v[i] = c;
+      w = w * d;
+    }
+    exc[p * 64 + lane] = c;
+    exw[p * 64 + lane] = w;
+    __syncthreads();
+    w = CHUNKS ? enter[ch * 64 + lane] : 0.0;
+    if (CHUNKS && pass < nc - 1) {
+      // downwards: only the value that enters the next chunk
+      for (int s = 0; s < NS; s++) w = exc[s * 64 + lane] + exw[s * 64 + lane] * w;
+      if (p == 0) enter[(ch + 1) * 64 + lane] = w;
+      __syncthreads();
+      continue;
+    }
+    for (int s = 0; s < p; s++) w = exc[s * 64 + lane] + exw[s * 64 + lane] * w;
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+      if (!UNIFORM && i >= S) continue;
+      w = w * dl(i);
+      v[i] = v[i] + w;
+    }
+    c = 0.0;
+    w = 1.0;
+#pragma unroll
+    for (int i = R - 1; i >= 0; i--) {
+      if (!UNIFORM && i >= S) continue;
+      const double u = ud(i);
+      c = v[i] * rd(i) + u * c;
+      v[i] = c;
+      w = w * u;
+    }
+    uxc[p * 64 + lane] = c;
+    uxw[p * 64 + lane] = w;
+    __syncthreads();
+    w = below;
+    for (int s = NS - 1; s > p; s--) w = uxc[s * 64 + lane] + uxw[s * 64 + lane] * w;
+    if constexpr (CHUNKS) {
+      for (int s = NS - 1; s >= 0; s--) below = uxc[s * 64 + lane] + uxw[s * 64 + lane] * below;
+    }
+    double *qp = q + (long long)lo * P + l;
+#pragma unroll
+    for (int i = R - 1; i >= 0; i--) {
+      if (!UNIFORM && i >= S) continue;
+      w = w * ud(i);
+      if (i < S && ok) {
+        double *o = qp + (long long)i * P;
+        st_nt(o, FOLD ? v[i] + w : *o + (v[i] + w));
+      }
+    }
+    if constexpr (CHUNKS) __syncthreads();  // exc and uxc are written again
   }
   if (comp == 1 && ok) {  // ImplicitAndUpdateQR.F90:70-71
     if (p == 0) q[l] = 0.0;
@@ -525,21 +565,22 @@ DEVI void helm_solve_lines(const long long lgrp, const int comp, const GridDev &
 // The table of a block's lines: one for all of them where their wall masks
 // agree (always with no-slip walls, and for the lines of a wave along a
 // groove), else one for each lane.
-template <int R, bool UNIFORM, bool FOLD>
+template <int R, bool UNIFORM, bool FOLD, bool CHUNKS>
 DEVI void helm_solve_body(const long long lgrp, const int comp, const GridDev &g,
                           double *__restrict__ q, const double *__restrict__ y,
                           const unsigned char *__restrict__ icyl,
                           const unsigned char *__restrict__ ocyl, const double *__restrict__ lu,
                           int nt, double *ex) {
   if (UNIFORM || comp == 1) {
-    helm_solve_lines<R, true, FOLD>(lgrp, comp, g, q, y, lu + (size_t)(comp == 1 ? 0 : 3) * nt, ex);
+    helm_solve_lines<R, true, FOLD, CHUNKS>(lgrp, comp, g, q, y, lu + (size_t)(comp == 1 ? 0 : 3) * nt,
+                                            ex);
   } else {
     const long long l = lgrp * 64 + threadIdx.x, lc = l < g.P ? l : g.P - 1;
     const int var = icyl[lc] + 2 * ocyl[lc], v0 = __builtin_amdgcn_readfirstlane(var);
     if (__all(var == v0))  // the same lines in every wave of the block
-      helm_solve_lines<R, true, FOLD>(lgrp, comp, g, q, y, lu + (size_t)v0 * nt, ex);
+      helm_solve_lines<R, true, FOLD, CHUNKS>(lgrp, comp, g, q, y, lu + (size_t)v0 * nt, ex);
     else
-      helm_solve_lines<R, false, FOLD>(lgrp, comp, g, q, y, lu + (size_t)var * nt, ex);
+      helm_solve_lines<R, false, FOLD, CHUNKS>(lgrp, comp, g, q, y, lu + (size_t)var * nt, ex);
   }
 }
 
@@ -552,21 +593,21 @@ struct SolveIO {
 // The components of a line group are consecutive, and the groups contiguous
 // per XCD: the six arrays then move together (1024x1024x769: 7.8 ms against
 // 8.2 with one component after the other, 512x512x385: 885 against 960 us).
-template <int R, bool UNIFORM, bool FOLD>
+template <int R, bool UNIFORM, bool FOLD, bool CHUNKS>
 __global__ __launch_bounds__(R > 32 ? 512 : 1024) void k_helm_solve(
     GridDev g, SolveIO io, const unsigned char *__restrict__ icyl,
     const unsigned char *__restrict__ ocyl, int nt, int comp0) {
   extern __shared__ double ex[];
   const int lin = xcd_tile(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
   const int comp = lin % (int)gridDim.y + comp0;
-  helm_solve_body<R, UNIFORM, FOLD>(lin / (int)gridDim.y, comp, g,
-                              comp == 0 ? io.q[0] : (comp == 1 ? io.q[1] : io.q[2]),
-                              comp == 0 ? io.y[0] : (comp == 1 ? io.y[1] : io.y[2]), icyl, ocyl,
-                              comp == 0 ? io.lu[0] : (comp == 1 ? io.lu[1] : io.lu[2]), nt, ex);
+  helm_solve_body<R, UNIFORM, FOLD, CHUNKS>(
+      lin / (int)gridDim.y, comp, g, comp == 0 ? io.q[0] : (comp == 1 ? io.q[1] : io.q[2]),
+      comp == 0 ? io.y[0] : (comp == 1 ? io.y[1] : io.y[2]), icyl, ocyl,
+      comp == 0 ? io.lu[0] : (comp == 1 ? io.lu[1] : io.lu[2]), nt, ex);
 }
 
 // Grouped: blockIdx.z = instance; right-hand sides in rhs, dq, qcap.
-template <int R, bool UNIFORM>
+template <int R, bool UNIFORM, bool CHUNKS>
 __global__ __launch_bounds__(R > 32 ? 512 : 1024) void k_helm_solve_g(
     const StepDesc *__restrict__ tab) {
   extern __shared__ double ex[];
@@ -574,7 +615,7 @@ __global__ __launch_bounds__(R > 32 ? 512 : 1024) void k_helm_solve_g(
   if (inst_stopped(d)) return;
   const int lin = xcd_tile(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * 3);
   const int comp = lin % 3;
-  helm_solve_body<R, UNIFORM, true>(
+  helm_solve_body<R, UNIFORM, true, CHUNKS>(
       lin / 3, comp, glob(d.g),
       glob(d.f[comp == 0 ? TC_QT : (comp == 1 ? TC_QR : TC_QZ)]),
       glob(d.f[comp == 0 ? TC_RHS : (comp == 1 ? TC_DQ : TC_QCAP)]), glob(d.icyl), glob(d.ocyl),
@@ -582,8 +623,7 @@ __global__ __launch_bounds__(R > 32 ? 512 : 1024) void k_helm_solve_g(
 }
 
 // Serial form, one line per lane: dgttrs as it is, for factors with row
-// exchanges and for lines longer than the partitioned form holds.  y is
-// overwritten by the forward sweep.  Loads are issued a chunk of rows ahead
+// exchanges.  y is overwritten by the forward sweep.  Loads are issued a chunk of rows ahead
 // of the dependent recurrence.
 DEVI void helm_solve_serial_body(const long long l, const int comp, const GridDev &g,
                                  double *__restrict__ q, double *__restrict__ y,
@@ -1338,35 +1378,45 @@ static unsigned line_blocks(const tc_ctx *c) { return (unsigned)((c->P + 255) / 
 
 // Shape of the partitioned solve: waves per block and the row capacity R of
 // its kernel, by the grid's shape alone (an instance's bits must not depend
-// on what it shares a launch with).  ns = 0: the serial form.  Few rows a
+// on what it shares a launch with).  ns = 0: the serial form.  Past eight
+// waves of 100 rows a line goes in chunks.  Few rows a
 // wave shorten the chain where there are few lines, many keep more loads in
 // flight where there are many: measured us with R = 25 / 50 / 100,
 // 128x128x97 18 / 21 / 32, 256x256x193 110 / 118 / 131, 256x256x385 257 /
 // 239 / 254, 512x512x385 970 / 953 / 887.
 struct SolveShape {
   int ns, rows;
+  bool chunks;  // lines of more than ns*rows rows
 };
 static SolveShape solve_shape(const tc_ctx *c) {
   const int n = c->nrm;
-  if (c->lu_pivots) return {0, 0};
+  if (c->lu_pivots) return {0, 0, false};
   const int R = n <= 72 ? 8 : (n <= 256 ? 25 : (n <= 400 && c->P < (1 << 17) ? 50 : 100));
-  const int ns = (n + R - 1) / R;
-  return ns <= (R > 32 ? 8 : 16) ? SolveShape{ns, R} : SolveShape{0, 0};
+  const int ns = (n + R - 1) / R, most = R > 32 ? 8 : 16;
+  return {std::min(ns, most), R, ns > most};
+}
+// LDS of a block: what its waves pass on in L and in U, and for a line in
+// chunks what enters each of them
+static size_t solve_lds(const SolveShape s, int n) {
+  const size_t chunks = s.chunks ? (size_t)((n + s.ns * s.rows - 1) / (s.ns * s.rows)) : 0;
+  return sizeof(double) * 64 * (4 * (size_t)s.ns + chunks);
 }
 
 template <bool U, bool FOLD>
 static void launch_solve_u(const SolveShape s, dim3 grid, hipStream_t st, const tc_ctx *c,
                            const SolveIO &io, int comp0) {
   const dim3 block(64, (unsigned)s.ns);
-  const size_t lds = sizeof(double) * 4 * 64 * (size_t)s.ns;
-#define TC_SOLVE(R)                                                                          \
-  hipLaunchKernelGGL((k_helm_solve<R, U, FOLD>), grid, block, lds, st, c->gd, io, c->mask,           \
-                     c->mask + c->P, c->lu_nt, comp0)
+  const size_t lds = solve_lds(s, c->nrm);
+#define TC_SOLVE(R, CHUNKS)                                                              \
+  hipLaunchKernelGGL((k_helm_solve<R, U, FOLD, CHUNKS>), grid, block, lds, st, c->gd, io, \
+                     c->mask, c->mask + c->P, c->lu_nt, comp0)
   switch (s.rows) {
-    case 8: TC_SOLVE(8); break;
-    case 25: TC_SOLVE(25); break;
-    case 50: TC_SOLVE(50); break;
-    default: TC_SOLVE(100); break;
+    case 8: TC_SOLVE(8, false); break;
+    case 25: TC_SOLVE(25, false); break;
+    case 50: TC_SOLVE(50, false); break;
+    default:
+      if (s.chunks) TC_SOLVE(100, true);
+      else TC_SOLVE(100, false);
   }
 #undef TC_SOLVE
 }
@@ -2496,15 +2546,19 @@ static void launch_rhs_g(tc_ctx *c, const StepDesc *tab, const BatchDyn *dyn, in
 }
 
 template <bool U>
-static void launch_solve_g(const SolveShape s, dim3 grid, hipStream_t st, const StepDesc *tab) {
+static void launch_solve_g(const SolveShape s, dim3 grid, hipStream_t st, const tc_ctx *c,
+                           const StepDesc *tab) {
   const dim3 block(64, (unsigned)s.ns);
-  const size_t lds = sizeof(double) * 4 * 64 * (size_t)s.ns;
-#define TC_SOLVE(R) hipLaunchKernelGGL((k_helm_solve_g<R, U>), grid, block, lds, st, tab)
+  const size_t lds = solve_lds(s, c->nrm);
+#define TC_SOLVE(R, CHUNKS) \
+  hipLaunchKernelGGL((k_helm_solve_g<R, U, CHUNKS>), grid, block, lds, st, tab)
   switch (s.rows) {
-    case 8: TC_SOLVE(8); break;
-    case 25: TC_SOLVE(25); break;
-    case 50: TC_SOLVE(50); break;
-    default: TC_SOLVE(100); break;
+    case 8: TC_SOLVE(8, false); break;
+    case 25: TC_SOLVE(25, false); break;
+    case 50: TC_SOLVE(50, false); break;
+    default:
+      if (s.chunks) TC_SOLVE(100, true);
+      else TC_SOLVE(100, false);
   }
 #undef TC_SOLVE
 }
@@ -2526,8 +2580,8 @@ void launch_helmholtz_fused_g(tc_ctx *c, const StepDesc *tab, const BatchDyn *dy
     return;
   }
   const dim3 grid((unsigned)((c->P + 63) / 64), 3, (unsigned)n);
-  if (c->masks_uniform_one) launch_solve_g<true>(s, grid, st, tab);
-  else launch_solve_g<false>(s, grid, st, tab);
+  if (c->masks_uniform_one) launch_solve_g<true>(s, grid, st, c, tab);
+  else launch_solve_g<false>(s, grid, st, c, tab);
 }
 
 void launch_correct_both_g(tc_ctx *c, const StepDesc *tab, int n, hipStream_t st) {

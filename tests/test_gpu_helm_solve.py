@@ -74,3 +74,40 @@ def test_masks_set_between_steps_are_replaced(tc):
     s.begin_step()
     got = s.masks()
     assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("defer", ["0", "2"])
+@pytest.mark.parametrize("nrm", [1025, 1601])
+def test_step_with_lines_in_chunks(tc, oracle, monkeypatch, nrm, defer):
+    """Lines past the 800 rows that a block holds: a first chunk of 225 rows,
+    and three chunks of which the first is one row (for q_r two full ones)."""
+    monkeypatch.setenv("TC_DEFER_CORRECTION", defer)
+    p = small_params(tc, 20, 9, nrm, ntst=1000, dtmin=1e-4, dtmax=1e-4, sizepert=0.1,
+                     omegapert=0.5, virotext=-0.3)
+    dev, orc = start_pair(tc, oracle, p, 11, 1e-2)
+    for n in range(2):
+        assert dev.step(n)[0] == orc.step(n)[0] == 0
+    compare_fields(dev, orc, nrm, 1e-10)
+
+
+@pytest.mark.parametrize("nrm", [801, 1030])
+def test_slip_walls_with_lines_in_chunks(tc, oracle, nrm):
+    p = small_params(tc, 20, 9, nrm, ren=500.0)
+    _implicit(tc, oracle, p, 1e-6, nrm)
+
+
+def test_batched_lines_in_chunks_equal_the_single_run(tc):
+    p = small_params(tc, 20, 9, 801, idtv=0, ntst=1000, dtmin=1e-4, dtmax=1e-4, limitcfl=1e30)
+    f = tc.init_perturbed_couette(p, 3, 1e-2)
+    s = tc.Solver(p)
+    with tc.Batch() as b:
+        ids = [b.add(p) for _ in range(2)]
+        for t in [s] + [b.solver(i) for i in ids]:
+            for n, a in zip(("qt", "qr", "qz"), f):
+                t.set(n, a)
+            t.project()
+        s.run(0, 3)
+        b.advance(3)
+        for i in ids:
+            for n in ("qt", "qr", "qz", "pr"):
+                assert np.array_equal(b.solver(i).get(n), s.get(n)), n
