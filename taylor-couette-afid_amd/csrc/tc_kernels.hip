@@ -1382,8 +1382,12 @@ static unsigned line_blocks(const tc_ctx *c) { return (unsigned)((c->P + 255) / 
 // waves of 100 rows a line goes in chunks.  Few rows a
 // wave shorten the chain where there are few lines, many keep more loads in
 // flight where there are many: measured us with R = 25 / 50 / 100,
-// 128x128x97 18 / 21 / 32, 256x256x193 110 / 118 / 131, 256x256x385 257 /
-// 239 / 254, 512x512x385 970 / 953 / 887.
+// 128x128x97 18 / 21 / 32, 256x256x193 123 / 125 / 129, 512x512x193 474 / 497
+// / 483, 1024x512x193 939 / 973 / 957, 256x256x385 257 / 239 / 254,
+// 512x512x385 970 / 953 / 887.  Nine waves of 25 and more no longer pair up
+// on a compute unit: 96x96x250 27 / 23, 128x128x225 39.5 / 37.8, 192x128x240
+// 66 / 61, 256x256x205 161 / 140, 256x256x250 179 / 160 / 164, 512x512x225
+// 631 / 569, 480x512x250 640 / 582 / 589 (64x64x225 17.7 / 18.5).
 struct SolveShape {
   int ns, rows;
   bool chunks;  // lines of more than ns*rows rows
@@ -1391,7 +1395,8 @@ struct SolveShape {
 static SolveShape solve_shape(const tc_ctx *c) {
   const int n = c->nrm;
   if (c->lu_pivots) return {0, 0, false};
-  const int R = n <= 72 ? 8 : (n <= 256 ? 25 : (n <= 400 && c->P < (1 << 17) ? 50 : 100));
+  const int R =
+      n <= 72 ? 8 : (n <= 200 ? 25 : (n <= 256 || (n <= 400 && c->P < (1 << 17)) ? 50 : 100));
   const int ns = (n + R - 1) / R, most = R > 32 ? 8 : 16;
   return {std::min(ns, most), R, ns > most};
 }

@@ -111,3 +111,12 @@ def test_batched_lines_in_chunks_equal_the_single_run(tc):
         for i in ids:
             for n in ("qt", "qr", "qz", "pr"):
                 assert np.array_equal(b.solver(i).get(n), s.get(n)), n
+
+
+@pytest.mark.parametrize("nrm", [200, 201])
+def test_step_where_the_rows_a_wave_change(tc, oracle, nrm):
+    """Eight waves of 25 rows, and the first length with 50 a wave."""
+    p = small_params(tc, 20, 9, nrm, ntst=1000, dtmin=1e-4, dtmax=1e-4)
+    dev, orc = start_pair(tc, oracle, p, 11, 1e-2)
+    assert dev.step(0)[0] == orc.step(0)[0] == 0
+    compare_fields(dev, orc, nrm, 1e-10)
