@@ -1478,25 +1478,31 @@ static long long helm_tiles(const tc_ctx *c, int lpt) {
 }
 
 // r segments of the fused front over n instances of this shape.  A launch
-// takes (rounds of resident blocks) x (planes per segment and about three
-// that a segment stages before its first), and its blocks, which run apart,
-// end within about a quarter of a segment of each other; the segment count
-// with the least of that, of at least two planes each.  Measured with one
-// line per thread, one segment against the chosen count: 64x64x65 133 -> 15
-// us, 256x256x193 400 -> 212 us, 512x512x385 1775 -> 1674 us.
+// takes (rounds of resident blocks) x (planes per segment and about four for
+// what a segment stages before its first and for its start), and its blocks,
+// which run apart, end within about a sixth of a segment of each other.  Of
+// the counts within 2% of the least of that, the largest, of at least two
+// planes each; up to 128 planes one segment where no count saves 2.5% (longer
+// ones drift apart, and tiles no longer find their neighbours' halo rows in
+// cache).  Measured us, one segment / the count taken (with the correction from the second pair on):
+// 64x64x65 133 / 16, 256x256x193 553 / 207 and 810 / 303, 512x512x385 1912 /
+// 1632 and 2728 / 2465, 1024x1024x769 14082 / 12488 and 20394 / 18653; one is
+// the best where the tiles fill the device and there are few planes (two:
+// 512x512x97 412 / 428 and 614 / 631, 512x512x65 281 / 330 and 414 / 502).
+// Over 30 sizes it is at most 3.4% over the best count.
 static int helm_segments(const tc_ctx *c, int lpt, bool corr, int n) {
   const long long tiles = n * helm_tiles(c, lpt), slots = c->helm_slots[corr];
-  int best = 1;
-  long long cost = 0;
-  for (int s = 1; s <= c->nrm / 2; s++) {
+  auto cost = [&](int s) {
     const long long len = (c->nrm + s - 1) / s, rounds = (tiles * s + slots - 1) / slots;
-    const long long t = 4 * rounds * (len + 3) + len;
-    if (s == 1 || t < cost) {
-      cost = t;
-      best = s;
-    }
-  }
-  return best;
+    return 32 * rounds * (len + 4) + 5 * len;
+  };
+  const int most = std::max(c->nrm / 2, 1);
+  long long least = cost(1);
+  for (int s = 2; s <= most; s++) least = std::min(least, cost(s));
+  if (c->nrm <= 128 && 40 * least > 39 * cost(1)) return 1;
+  int s = most;
+  while (50 * cost(s) > 51 * least) s--;
+  return s;
 }
 
 // Fused path: right-hand sides of q_theta -> rhs, q_r -> dq, q_z -> qcap (the
