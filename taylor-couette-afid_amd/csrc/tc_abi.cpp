@@ -166,21 +166,22 @@ void build_qr_table(const tc::Grid &g, double betadx, double *T, int nt, tc::Rhs
 
 int refresh_tables(tc_ctx *c) {
   const int nsst = c->p.nsst;
-  // with every wall mask 1 only the no-slip variant (3) is ever read
-  const bool all_variants = !c->masks_uniform_one;
-  bool any = !c->lu_valid || (all_variants && !c->lu_all_variants);
+  // the no-slip variant (3) and those that some line's masks ask for
+  const unsigned vars = c->mask_vars | 8u;
+  bool any = !c->lu_valid || (vars & ~c->lu_vars) != 0;
   for (int s = 0; s < nsst; s++)
     if (c->lu_key[s] != c->beta * c->g.alm[s + 1]) any = true;
   if (!any) return 0;
   // the previous upload must have left the staging buffer
   HIPCHK(hipEventSynchronize(c->lu_copied));
   const size_t per_slot = tc::lu_slot_doubles(c);
-  bool pivots = false;
+  unsigned pivots[3] = {0, 0, 0};
   for (int s = 0; s < nsst; s++) {
     const double betadx = c->beta * c->g.alm[s + 1];
     double *base = c->lu_host + (size_t)s * per_slot;
     tc::RhsRow *rows = reinterpret_cast<tc::RhsRow *>(base + (size_t)3 * 4 * c->lu_nt);
-    for (int v = all_variants ? 0 : 3; v < 4; v++) {
+    for (int v = 0; v < 4; v++) {
+      if (!(vars >> v & 1)) continue;
       build_wall_table(c->g, tc::LU_QT, v & 1, v >> 1, betadx,
                        base + ((size_t)tc::LU_QT * 4 + v) * c->lu_nt, c->lu_nt, rows);
       build_wall_table(c->g, tc::LU_QZ, v & 1, v >> 1, betadx,
@@ -188,9 +189,9 @@ int refresh_tables(tc_ctx *c) {
     }
     build_qr_table(c->g, betadx, base + (size_t)tc::LU_QR * 4 * c->lu_nt, c->lu_nt, rows);
     for (int t = 0; t < 12; t++) {
-      const bool used = t / 4 == tc::LU_QR ? t % 4 == 0 : (all_variants || t % 4 == 3);
+      const bool used = t / 4 == tc::LU_QR ? t % 4 == 0 : (vars >> t % 4 & 1) != 0;
       for (int r = 0; used && r < c->nr; r++)
-        pivots = pivots || base[(size_t)t * c->lu_nt + tc::LU_ROW * r + 5] != 0.0;
+        if (base[(size_t)t * c->lu_nt + tc::LU_ROW * r + 5] != 0.0) pivots[t / 4] |= 1u << t % 4;
     }
     c->lu_key[s] = betadx;
   }
@@ -198,23 +199,24 @@ int refresh_tables(tc_ctx *c) {
                         c->stream));
   HIPCHK(hipEventRecord(c->lu_copied, c->stream));
   c->lu_valid = true;
-  c->lu_all_variants = all_variants;
-  c->lu_pivots = pivots;
+  c->lu_vars = vars;
+  std::copy(pivots, pivots + 3, c->lu_pivots);
   return 0;
 }
 
 int upload_masks(tc_ctx *c) {
   std::vector<unsigned char> m((size_t)2 * c->P);
-  bool ones = true;
+  unsigned vars = 0;
   for (int i = 0; i < c->nthm; i++)
     for (int j = 0; j < c->nzm; j++) {
       const size_t f = (size_t)j + (size_t)c->nzm * i;
       const size_t d = (size_t)j * c->nthm + i;
       m[d] = (unsigned char)(c->icyl[f] != 0);
       m[c->P + d] = (unsigned char)(c->ocyl[f] != 0);
-      ones = ones && c->icyl[f] == 1 && c->ocyl[f] == 1;
+      vars |= 1u << (m[d] + 2 * m[c->P + d]);
     }
-  c->masks_uniform_one = ones;
+  c->mask_vars = vars;
+  c->masks_uniform_one = vars == 8u;
   HIPCHK(hipMemcpyAsync(c->mask, m.data(), m.size(), hipMemcpyHostToDevice, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
   return 0;

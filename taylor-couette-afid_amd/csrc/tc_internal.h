@@ -234,8 +234,10 @@ struct tc_ctx {
   int lu_nt = 0;               // doubles per table = LU_ROW*(nrm+1)
   double lu_key[3] = {-1, -1, -1};
   bool lu_valid = false;
-  bool lu_all_variants = false;  // all four mask variants built (else only variant 3)
-  bool lu_pivots = false;        // some table exchanges rows (helm_solve needs the serial sweep)
+  // bit v: the lines' wall masks hold variant v = icyl + 2 ocyl; the variants
+  // whose tables are built; those of them, per component (q_theta, q_r, q_z),
+  // whose factors exchange rows
+  unsigned mask_vars = 8, lu_vars = 0, lu_pivots[3] = {0, 0, 0};
   // FFT
   tc::FFTPlan plan_t, plan_z;
   double2 *tw_t = nullptr, *tw_z = nullptr;
@@ -329,6 +331,8 @@ int set_deferral(tc_ctx *c, int mode);
 // the dt and step recorded in a restart file's header (nothing else is read)
 int restart_file_info(const char *path, double *dt, int *ntime);
 size_t lu_slot_doubles(const tc_ctx *c);
+// bit q: component q is solved by the serial form
+unsigned serial_comps(const tc_ctx *c);
 const double *lu_table(const tc_ctx *c, int ns, int comp);
 const RhsRow *rhs_rows(const tc_ctx *c, int ns);
 void launch_helmholtz_fused_g(tc_ctx *c, const StepDesc *tab, const BatchDyn *dyn, int ns, int n,

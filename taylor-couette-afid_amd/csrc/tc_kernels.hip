@@ -609,14 +609,14 @@ __global__ __launch_bounds__(R > 32 ? 512 : 1024) void k_helm_solve(
 // Grouped: blockIdx.z = instance; right-hand sides in rhs, dq, qcap.
 template <int R, bool UNIFORM, bool CHUNKS>
 __global__ __launch_bounds__(R > 32 ? 512 : 1024) void k_helm_solve_g(
-    const StepDesc *__restrict__ tab) {
+    const StepDesc *__restrict__ tab, int comp0) {
   extern __shared__ double ex[];
   const StepDesc &d = tab[blockIdx.z];
   if (inst_stopped(d)) return;
-  const int lin = xcd_tile(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * 3);
-  const int comp = lin % 3;
+  const int lin = xcd_tile(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
+  const int comp = lin % (int)gridDim.y + comp0;
   helm_solve_body<R, UNIFORM, true, CHUNKS>(
-      lin / 3, comp, glob(d.g),
+      lin / (int)gridDim.y, comp, glob(d.g),
       glob(d.f[comp == 0 ? TC_QT : (comp == 1 ? TC_QR : TC_QZ)]),
       glob(d.f[comp == 0 ? TC_RHS : (comp == 1 ? TC_DQ : TC_QCAP)]), glob(d.icyl), glob(d.ocyl),
       glob(comp == 0 ? d.lut : (comp == 1 ? d.lur : d.luz)), d.lu_nt, ex);
@@ -680,18 +680,18 @@ DEVI void helm_solve_serial_body(const long long l, const int comp, const GridDe
 __global__ __launch_bounds__(256) void k_helm_solve_serial(GridDev g, SolveIO io,
                                                            const unsigned char *__restrict__ icyl,
                                                            const unsigned char *__restrict__ ocyl,
-                                                           int nt, int comp0, bool fold) {
-  const int comp = blockIdx.y + comp0;
+                                                           int nt, int comp, bool fold) {
   helm_solve_serial_body((long long)blockIdx.x * 256 + threadIdx.x, comp, g,
                          comp == 0 ? io.q[0] : (comp == 1 ? io.q[1] : io.q[2]),
                          const_cast<double *>(comp == 0 ? io.y[0] : (comp == 1 ? io.y[1] : io.y[2])),
                          icyl, ocyl, comp == 0 ? io.lu[0] : (comp == 1 ? io.lu[1] : io.lu[2]), nt, fold);
 }
 
-__global__ __launch_bounds__(256) void k_helm_solve_serial_g(const StepDesc *__restrict__ tab) {
-  const StepDesc &d = tab[blockIdx.z];
+// Grouped: blockIdx.y = instance.
+__global__ __launch_bounds__(256) void k_helm_solve_serial_g(const StepDesc *__restrict__ tab,
+                                                             int comp) {
+  const StepDesc &d = tab[blockIdx.y];
   if (inst_stopped(d)) return;
-  const int comp = blockIdx.y;
   helm_solve_serial_body((long long)blockIdx.x * 256 + threadIdx.x, comp, glob(d.g),
                          glob(d.f[comp == 0 ? TC_QT : (comp == 1 ? TC_QR : TC_QZ)]),
                          glob(d.f[comp == 0 ? TC_RHS : (comp == 1 ? TC_DQ : TC_QCAP)]),
@@ -1376,10 +1376,21 @@ const RhsRow *rhs_rows(const tc_ctx *c, int ns) {
 
 static unsigned line_blocks(const tc_ctx *c) { return (unsigned)((c->P + 255) / 256); }
 
+// Components whose factors exchange rows on some line.  Only those take the
+// serial form, and only while the masks hold such lines: tables that no line
+// reads (of a free-slip outer wall, which SlipBCs never sets) or that a former
+// pattern read do not count.  (They did: 192x128x129 with grooves at beta*ac
+// of a few took 87 us a solve instead of 38.)
+unsigned serial_comps(const tc_ctx *c) {
+  unsigned s = c->lu_pivots[LU_QR] ? 1u << LU_QR : 0u;
+  for (int q : {LU_QT, LU_QZ})
+    if (c->lu_pivots[q] & c->mask_vars) s |= 1u << q;
+  return s;
+}
+
 // Shape of the partitioned solve: waves per block and the row capacity R of
 // its kernel, by the grid's shape alone (an instance's bits must not depend
-// on what it shares a launch with).  ns = 0: the serial form.  Past eight
-// waves of 100 rows a line goes in chunks.  Few rows a
+// on what it shares a launch with).  Past eight waves of 100 rows a line goes in chunks.  Few rows a
 // wave shorten the chain where there are few lines, many keep more loads in
 // flight where there are many: measured us with R = 25 / 50 / 100,
 // 128x128x97 18 / 21 / 32, 256x256x193 123 / 125 / 129, 512x512x193 474 / 497
@@ -1394,7 +1405,6 @@ struct SolveShape {
 };
 static SolveShape solve_shape(const tc_ctx *c) {
   const int n = c->nrm;
-  if (c->lu_pivots) return {0, 0, false};
   const int R =
       n <= 72 ? 8 : (n <= 200 ? 25 : (n <= 256 || (n <= 400 && c->P < (1 << 17)) ? 50 : 100));
   const int ns = (n + R - 1) / R, most = R > 32 ? 8 : 16;
@@ -1426,17 +1436,22 @@ static void launch_solve_u(const SolveShape s, dim3 grid, hipStream_t st, const 
 #undef TC_SOLVE
 }
 
-// FOLD: all three components; otherwise the one component comp0
+// FOLD: all three components (one by one where some take the serial form);
+// otherwise the one component comp0
 template <bool FOLD>
-static void launch_solve(tc_ctx *c, const SolveIO &io, int comp0) {
-  const SolveShape s = solve_shape(c);
-  const unsigned ncomp = FOLD ? 3 : 1;
-  if (s.ns == 0) {
-    hipLaunchKernelGGL(k_helm_solve_serial, dim3(line_blocks(c), ncomp), dim3(256), 0, c->stream,
-                       c->gd, io, c->mask, c->mask + c->P, c->lu_nt, comp0, FOLD);
+static void launch_solve(tc_ctx *c, const SolveIO &io, int comp0, int ncomp) {
+  const unsigned serial = serial_comps(c);
+  if (ncomp > 1 && serial) {
+    for (int q = 0; q < ncomp; q++) launch_solve<FOLD>(c, io, comp0 + q, 1);
     return;
   }
-  const dim3 grid((unsigned)((c->P + 63) / 64), ncomp);
+  if (serial >> comp0 & 1) {
+    hipLaunchKernelGGL(k_helm_solve_serial, dim3(line_blocks(c)), dim3(256), 0, c->stream, c->gd, io,
+                       c->mask, c->mask + c->P, c->lu_nt, comp0, FOLD);
+    return;
+  }
+  const SolveShape s = solve_shape(c);
+  const dim3 grid((unsigned)((c->P + 63) / 64), (unsigned)ncomp);
   if (c->masks_uniform_one)
     launch_solve_u<true, FOLD>(s, grid, c->stream, c, io, comp0);
   else
@@ -1466,7 +1481,7 @@ static void launch_implicit(tc_ctx *c, const char *name, int q, int expl, int ru
   timer_end(c);
   SolveIO io = solve_io(c);
   io.y[WHICH] = c->f[TC_RHS];
-  launch_solve<false>(c, io, WHICH);
+  launch_solve<false>(c, io, WHICH, 1);
 }
 void launch_implicit_qt(tc_ctx *c) { launch_implicit<0>(c, "implicit_qt", TC_QT, TC_DQ, TC_RU1); }
 void launch_implicit_qr(tc_ctx *c) { launch_implicit<1>(c, "implicit_qr", TC_QR, TC_DPH, TC_RU2); }
@@ -1569,7 +1584,7 @@ void launch_helmholtz_fused(tc_ctx *c) {
   }
   timer_end(c);
   timer_begin(c, "helm_bwd");
-  launch_solve<true>(c, solve_io(c), 0);
+  launch_solve<true>(c, solve_io(c), 0, 3);
   timer_end(c);
 }
 
@@ -1589,7 +1604,7 @@ void launch_helmholtz_fused_corr(tc_ctx *c, const double *pr_in, double *pr_out,
   }
   timer_end(c);
   timer_begin(c, "helm_bwd");
-  launch_solve<true>(c, solve_io(c), 0);
+  launch_solve<true>(c, solve_io(c), 0, 3);
   timer_end(c);
 }
 
@@ -2558,11 +2573,11 @@ static void launch_rhs_g(tc_ctx *c, const StepDesc *tab, const BatchDyn *dyn, in
 
 template <bool U>
 static void launch_solve_g(const SolveShape s, dim3 grid, hipStream_t st, const tc_ctx *c,
-                           const StepDesc *tab) {
+                           const StepDesc *tab, int comp0) {
   const dim3 block(64, (unsigned)s.ns);
   const size_t lds = solve_lds(s, c->nrm);
 #define TC_SOLVE(R, CHUNKS) \
-  hipLaunchKernelGGL((k_helm_solve_g<R, U, CHUNKS>), grid, block, lds, st, tab)
+  hipLaunchKernelGGL((k_helm_solve_g<R, U, CHUNKS>), grid, block, lds, st, tab, comp0)
   switch (s.rows) {
     case 8: TC_SOLVE(8, false); break;
     case 25: TC_SOLVE(25, false); break;
@@ -2585,14 +2600,17 @@ void launch_helmholtz_fused_g(tc_ctx *c, const StepDesc *tab, const BatchDyn *dy
     else launch_rhs_g<false, 1>(c, tab, dyn, ns, n, st, corr);
   }
   const SolveShape s = solve_shape(c);
-  if (s.ns == 0) {
-    hipLaunchKernelGGL(k_helm_solve_serial_g, dim3(line_blocks(c), 3, (unsigned)n), dim3(256), 0,
-                       st, tab);
-    return;
+  const unsigned serial = serial_comps(c), ncomp = serial ? 1 : 3;
+  const dim3 grid((unsigned)((c->P + 63) / 64), ncomp, (unsigned)n);
+  for (int q = 0; q < 3; q += (int)ncomp) {
+    if (serial >> q & 1)
+      hipLaunchKernelGGL(k_helm_solve_serial_g, dim3(line_blocks(c), (unsigned)n), dim3(256), 0, st,
+                         tab, q);
+    else if (c->masks_uniform_one)
+      launch_solve_g<true>(s, grid, st, c, tab, q);
+    else
+      launch_solve_g<false>(s, grid, st, c, tab, q);
   }
-  const dim3 grid((unsigned)((c->P + 63) / 64), 3, (unsigned)n);
-  if (c->masks_uniform_one) launch_solve_g<true>(s, grid, st, c, tab);
-  else launch_solve_g<false>(s, grid, st, c, tab);
 }
 
 void launch_correct_both_g(tc_ctx *c, const StepDesc *tab, int n, hipStream_t st) {
