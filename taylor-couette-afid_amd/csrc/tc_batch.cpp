@@ -45,7 +45,19 @@ struct Inst {
   int group = -1, slot = -1;
 };
 
+// What the grouped launches of an instance depend on.
+using Key = std::tuple<int, int, int, int, int, int, int, int, int, int, int, int, int, int>;
+
+Key group_key(const tc_ctx *c) {
+  return Key(c->nthm, c->nzm, c->nrm, c->p.nsst, c->helm_lpt, c->poisson_pq,
+             (c->masks_uniform_one ? 1 : 0) + 2 * (int)tc::serial_comps(c), c->plan_t.lines,
+             c->plan_t.me, c->plan_t.padsh,
+             c->plan_z.lines, c->plan_z.me * 1000 + c->plan_z.nt, c->plan_z.padsh,
+             tc::defers_correction(c) ? 1 : 0);
+}
+
 struct Group {
+  Key key;
   std::vector<int> ids;
   tc_ctx *rep = nullptr;
   StepDesc *tab[3] = {nullptr, nullptr, nullptr};
@@ -56,16 +68,6 @@ struct Group {
   hipEvent_t join = nullptr;
   size_t dyn_off = 0;  // offset of this group's entries in the staging slot
 };
-
-using Key = std::tuple<int, int, int, int, int, int, int, int, int, int, int, int, int, int>;
-
-Key group_key(const tc_ctx *c) {
-  return Key(c->nthm, c->nzm, c->nrm, c->p.nsst, c->helm_lpt, c->poisson_pq,
-             (c->masks_uniform_one ? 1 : 0) + 2 * (int)tc::serial_comps(c), c->plan_t.lines,
-             c->plan_t.me, c->plan_t.padsh,
-             c->plan_z.lines, c->plan_z.me * 1000 + c->plan_z.nt, c->plan_z.padsh,
-             tc::defers_correction(c) ? 1 : 0);
-}
 
 // a failed call is also cleared from the runtime's last-error state
 #define BCHK(x)                                                                  \
@@ -251,6 +253,7 @@ int rebuild(tc_batch *b) {
   size_t total = 0;
   for (auto &kv : by) {
     Group g;
+    g.key = kv.first;
     g.ids = kv.second;
     g.rep = b->inst[(size_t)g.ids[0]].c;
     const int n = (int)g.ids.size();
@@ -428,6 +431,12 @@ int tc_batch_advance(tc_batch *b, int nsteps, int use_graph, int sync_every) {
   // work the caller queued on the instances' own streams comes first
   for (Inst &I : b->inst)
     if (I.live && I.c) BCHK(hipStreamSynchronize(I.c->stream));
+  // as are masks or a tuning set on an instance since the groups were built
+  for (const Group &g : b->groups)
+    for (int id : g.ids) {
+      const Inst &I = b->inst[(size_t)id];
+      if (I.live && I.c && group_key(I.c) != g.key) b->dirty = true;
+    }
   int rc = 0;
   for (int s = 0; s < nsteps; s++) {
     if (b->dirty) {
