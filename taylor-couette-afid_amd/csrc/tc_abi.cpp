@@ -62,137 +62,202 @@ int launch_status() {
 // Helmholtz LU tables (SolveImpEqnUpdate_QT.F90:37-63,
 // SolveImpEqnUpdate_QR.F90:27-44, SolveImpEqnUpdate_QZ.F90:35-58)
 // ---------------------------------------------------------------------------
-void write_table(double *T, int nt, int n, std::vector<double> &dl, std::vector<double> &d,
-                 std::vector<double> &du, const std::vector<double> &sc) {
-  constexpr int W = tc::LU_ROW;
-  std::vector<double> du2((size_t)std::max(n, 1), 0.0);
-  std::vector<int> ipiv((size_t)n);
-  tc::dgttrf(n, dl.data(), d.data(), du.data(), du2.data(), ipiv.data());
-  std::fill(T, T + nt, 0.0);
-  for (int q = 0; q < n - 1; q++) {
-    T[W * q] = dl[q];
-    T[W * q + 1] = du[q];
-    T[W * q + 5] = (ipiv[q] != q) ? 1.0 : 0.0;
-  }
-  for (int q = 0; q < n - 2; q++) T[W * q + 2] = du2[q];
-  for (int q = 0; q < n; q++) {
-    T[W * q + 3] = 1.0 / d[q];
-    T[W * q + 4] = sc[q];
-    T[W * q + 6] = d[q];
-  }
-}
+// Row-normalised matrix (unit diagonal) of one component: row q couples to
+// q-1 with lo[q] and to q+1 with up[q].
+struct Matrix {
+  std::vector<double> lo, up;
+  explicit Matrix(int n) : lo((size_t)n, 0.0), up((size_t)n, 0.0) {}
+  // row sum, rounded once
+  double sum(int q) const { return (double)((long double)1 + lo[q] + up[q]); }
+};
 
-// Row-normalised matrix of the q_theta / q_z solves (mask variant ic, oc).
-// rows: the records of the right-hand sides, filled by the no-slip variant.
-void build_wall_table(const tc::Grid &g, int comp, int ic, int oc, double betadx, double *T, int nt,
-                      tc::RhsRow *rows) {
-  const int n = g.nrm;
+// Off-diagonals of row kc of q_theta / q_z; slip: the wall that the row is
+// beside is free-slip.
+void wall_row(const tc::Grid &g, int comp, int kc, bool slip, double betadx, double &lo, double &up) {
   const bool is_qt = (comp == tc::LU_QT);
   const std::vector<double> &ap = is_qt ? g.ap1j : g.ap3j;
   const std::vector<double> &am = is_qt ? g.am1j : g.am3j;
   const std::vector<double> &ac = is_qt ? g.ac1j : g.ac3j;
-  const double ac_fs1 = is_qt ? g.ac1j_fs[1] : g.ac3j_fs[1];
-  const double ac_fs2 = is_qt ? g.ac1j_fs[2] : g.ac3j_fs[2];
-  std::vector<double> amkl((size_t)n + 2), ackl((size_t)n + 2), apkl((size_t)n + 2);
-  const double fic = (double)ic, foc = (double)oc;
-  double actot = (ac[1] * fic + ac_fs1 * (1 - fic));
-  double ackl_b = 1.0 / (1.0 - actot * betadx);
-  ackl[1] = 1.0;
-  apkl[1] = -ap[1] * betadx * ackl_b;
-  for (int kc = 2; kc <= n - 1; kc++) {
-    ackl_b = 1.0 / (1.0 - ac[kc] * betadx);
-    amkl[kc] = -am[kc] * betadx * ackl_b;
-    ackl[kc] = 1.0;
-    apkl[kc] = -ap[kc] * betadx * ackl_b;
-  }
-  actot = (ac[n] * foc + ac_fs2 * (1 - foc));
-  ackl_b = 1.0 / (1.0 - actot * betadx);
-  amkl[n] = -am[n] * betadx * ackl_b;
-  ackl[n] = 1.0;
-  apkl[n] = 0.0;
-  std::vector<double> dl((size_t)n), d((size_t)n), du((size_t)n), sc((size_t)n);
-  for (int q = 0; q < n - 1; q++) {
-    dl[q] = amkl[q + 2];
-    du[q] = apkl[q + 1];
-  }
-  for (int q = 0; q < n; q++) d[q] = ackl[q + 1];
-  // right-hand side row scaling uses the unblended diagonal
-  for (int kc = 1; kc <= n; kc++) sc[kc - 1] = 1.0 / (1. - ac[kc] * betadx);
-  if (ic == 1 && oc == 1) {
-    double tc::RhsRow::*const f[4] = {is_qt ? &tc::RhsRow::sc_t : &tc::RhsRow::sc_z,
-                                      is_qt ? &tc::RhsRow::am_t : &tc::RhsRow::am_z,
-                                      is_qt ? &tc::RhsRow::ap_t : &tc::RhsRow::ap_z,
-                                      is_qt ? &tc::RhsRow::x_t : &tc::RhsRow::x_z};
-    for (int kc = 1; kc <= n; kc++) {
-      rows[kc].*f[0] = sc[kc - 1];
-      rows[kc].*f[1] = kc > 1 ? amkl[kc] : 0.0;
-      rows[kc].*f[2] = kc < n ? apkl[kc] : 0.0;
-    }
-    rows[1].*f[3] = -ap[1] * betadx * (1.0 / (1.0 - ac_fs1 * betadx));
-    rows[n].*f[3] = -am[n] * betadx * (1.0 / (1.0 - ac_fs2 * betadx));
-  }
-  write_table(T, nt, n, dl, d, du, sc);
+  const double *ac_fs = is_qt ? g.ac1j_fs : g.ac3j_fs;
+  const double ackl_b = 1.0 / (1.0 - (slip ? ac_fs[kc == 1 ? 1 : 2] : ac[kc]) * betadx);
+  lo = kc > 1 ? -am[kc] * betadx * ackl_b : 0.0;
+  up = kc < g.nrm ? -ap[kc] * betadx * ackl_b : 0.0;
 }
 
-void build_qr_table(const tc::Grid &g, double betadx, double *T, int nt, tc::RhsRow *rows) {
-  const int n = g.nr, nrm = g.nrm;
-  std::vector<double> amkl((size_t)n + 2), ackl((size_t)n + 2), apkl((size_t)n + 2);
-  amkl[1] = 0.;
-  apkl[1] = 0.;
-  ackl[1] = 1.;
-  for (int kc = 2; kc <= nrm; kc++) {
+// q_theta / q_z, mask variant ic, oc
+Matrix wall_matrix(const tc::Grid &g, int comp, int ic, int oc, double betadx) {
+  const int n = g.nrm;
+  Matrix A(n);
+  for (int kc = 1; kc <= n; kc++)
+    wall_row(g, comp, kc, (kc == 1 && !ic) || (kc == n && !oc), betadx, A.lo[kc - 1], A.up[kc - 1]);
+  return A;
+}
+
+// q_r, nr rows: q_r is fixed at both walls, rows of their own that the rows
+// beside them do not couple to
+Matrix qr_matrix(const tc::Grid &g, double betadx) {
+  Matrix A(g.nr);
+  for (int kc = 2; kc <= g.nrm; kc++) {
     const double ackl_b = 1.0 / (1.0 - g.ac2j[kc] * betadx);
-    amkl[kc] = -g.am2j[kc] * betadx * ackl_b;
-    ackl[kc] = 1.0;
-    apkl[kc] = -g.ap2j[kc] * betadx * ackl_b;
+    if (kc > 2) A.lo[kc - 1] = -g.am2j[kc] * betadx * ackl_b;
+    if (kc < g.nrm) A.up[kc - 1] = -g.ap2j[kc] * betadx * ackl_b;
   }
-  amkl[n] = 0.;
-  apkl[n] = 0.;
-  ackl[n] = 1.;
-  std::vector<double> dl((size_t)n), d((size_t)n), du((size_t)n), sc((size_t)n, 0.0);
-  for (int q = 0; q < n - 1; q++) {
-    dl[q] = amkl[q + 2];
-    du[q] = apkl[q + 1];
+  return A;
+}
+
+// scaling of the right-hand side of row kc: by the unblended diagonal
+double rhs_scale(const tc::Grid &g, int comp, int kc, double betadx) {
+  const std::vector<double> &ac = comp == tc::LU_QT ? g.ac1j : (comp == tc::LU_QR ? g.ac2j : g.ac3j);
+  return 1.0 / (1.0 - ac[kc] * betadx);
+}
+
+// Factors of A with row exchanges, as dgttrf forms them: rows of dl, du, du2,
+// rd, pv for the serial solve.  True where a row was exchanged.  A matrix
+// whose row sums are not negative (its off-diagonals are not positive) is
+// diagonally dominant and needs no exchange.
+bool write_serial(const Matrix &A, double *T, bool write) {
+  constexpr int W = tc::LU_ROW;
+  const int n = (int)A.lo.size();
+  bool dominant = true;
+  for (int q = 0; q < n && !write; q++) dominant = dominant && A.sum(q) >= 0.0;
+  if (!write && dominant) return false;
+  std::vector<double> dl(A.lo.begin() + 1, A.lo.end()), d((size_t)n, 1.0), du(A.up), du2((size_t)n, 0.0);
+  std::vector<int> ipiv((size_t)n);
+  dl.push_back(0.0);
+  tc::dgttrf(n, dl.data(), d.data(), du.data(), du2.data(), ipiv.data());
+  bool exchanged = false;
+  for (int q = 0; q < n; q++) {
+    const bool pv = q < n - 1 && ipiv[q] != q;
+    exchanged = exchanged || pv;
+    if (!write) continue;
+    T[W * q] = q < n - 1 ? dl[q] : 0.0;
+    T[W * q + 1] = q < n - 1 ? du[q] : 0.0;
+    T[W * q + 2] = q < n - 2 ? du2[q] : 0.0;
+    T[W * q + 3] = 1.0 / d[q];
+    T[W * q + 4] = pv ? 1.0 : 0.0;
   }
-  for (int q = 0; q < n; q++) d[q] = ackl[q + 1];
-  for (int kc = 2; kc <= nrm; kc++) {
-    sc[kc - 1] = 1.0 / (1.0 - g.ac2j[kc] * betadx);
-    rows[kc].sc_r = sc[kc - 1];
-    rows[kc].am_r = kc > 2 ? amkl[kc] : 0.0;
-    rows[kc].ap_r = kc < nrm ? apkl[kc] : 0.0;
+  return exchanged;
+}
+
+// Factors of D A without row exchanges for the partitioned solve, rows of m,
+// u, r: y_q = g_q + m_q y_(q-1) down, x_q = y_q r_q + u_q x_(q+1) up.  The
+// pivots are formed from the row sums, d_q = s_q + m_q sigma_(q-1) - up_q
+// with sigma_q = d_q + up_q, all terms of one sign, so that each factor is
+// accurate to an ulp; as 1 - lo up / d they lose what cancels, and with
+// clustered rows (beta*ac >> 1) nearly all of d_q + up_q does.  The rows are
+// scaled by the reciprocal pivots of the no-slip matrix, D = 1 / d, so that r
+// is 1 there and y is rounded once a row.  first: the first row that is
+// solved.  sum: the row sums of the matrix that the rounded factors multiply
+// out to.  The right-hand sides fold q in by that matrix: by D A itself every
+// solve of a steady flow moves it the same way by what the factors round
+// (after 30 steps of 256x256x193 q_theta was off by 1.8e-15 and the inner
+// torque by 3.7e-13).
+void write_partitioned(const Matrix &A, int first, int last, std::vector<double> &D, bool own,
+                       double *T, std::vector<long double> &sum) {
+  constexpr int W = tc::LU_ROW;
+  double sigma = 0.0, d = 1.0;
+  for (int q = first; q <= last; q++) {
+    const double m = q > first ? -A.lo[q] / d : 0.0;
+    sigma = A.sum(q) + m * sigma;
+    d = sigma - A.up[q];
+    const double rd = 1.0 / d;
+    if (own) D[q] = rd;
+    if (q > first) T[W * q] = own ? -A.lo[q] * rd : m * D[q] / D[q - 1];
+    T[W * q + 1] = -A.up[q] * rd;
+    T[W * q + 3] = own ? 1.0 : rd / D[q];
+    const long double r = T[W * q + 3], u = T[W * q + 1];
+    sum[q] = (1 - u) / r;
+    if (q > first) sum[q] -= T[W * q] / (long double)T[W * (q - 1) + 3] * (1 - (long double)T[W * (q - 1) + 1]);
   }
-  write_table(T, nt, n, dl, d, du, sc);
+}
+
+// Tables and right-hand side records of component comp of one substep slot;
+// A: its matrix of each mask variant in vars (q_r: the last).
+void build_component(const tc::Grid &g, int comp, unsigned vars, const Matrix *A, double betadx,
+                     bool serial, double *T, int nt, tc::RhsRow *rows) {
+  using R = tc::RhsRow;
+  double R::*const f[3][4] = {{&R::sc_t, &R::am_t, &R::ap_t, &R::s_t},
+                              {&R::sc_r, &R::am_r, &R::ap_r, &R::s_r},
+                              {&R::sc_z, &R::am_z, &R::ap_z, &R::s_z}};
+  const bool wall = comp != tc::LU_QR, qt = comp == tc::LU_QT;
+  double R::*const et[4] = {&R::e0_t, &R::e1_t, &R::e2_t, &R::e3_t};
+  double R::*const ez[4] = {&R::e0_z, &R::e1_z, &R::e2_z, &R::e3_z};
+  double R::*const x = qt ? &R::x_t : &R::x_z, R::*const xs = qt ? &R::xs_t : &R::xs_z;
+  const int k0 = wall ? 1 : 2, nrm = g.nrm;
+  std::vector<double> D((size_t)g.nr, 1.0);
+  std::vector<long double> sum((size_t)g.nr, 0.0L);
+  // the no-slip variant first: its pivots scale the rows
+  for (int v : {3, 0, 1, 2}) {
+    if (!(wall ? vars >> v & 1 : v == 3)) continue;
+    double *Tv = T + (size_t)(wall ? v : 0) * nt;
+    std::fill(Tv, Tv + nt, 0.0);
+    if (serial)
+      write_serial(A[v], Tv, true);
+    else
+      write_partitioned(A[v], k0 - 1, nrm - 1, D, v == 3, Tv, sum);
+    for (int kc = k0; kc <= nrm; kc++) {
+      tc::RhsRow &row = rows[kc];
+      const int q = kc - 1;
+      if (v == 3) {
+        row.*f[comp][0] = rhs_scale(g, comp, kc, betadx) * D[q];
+        // the serial form adds its solution to q
+        row.*f[comp][1] = serial ? 0.0 : -Tv[tc::LU_ROW * q];
+        row.*f[comp][2] = serial ? 0.0 : -Tv[tc::LU_ROW * q + 1];
+        row.*f[comp][3] = serial ? 0.0 : (double)sum[q];
+        if (wall && (kc == 1 || kc == nrm)) {
+          // beside a free-slip wall: one off-diagonal
+          double lo, up;
+          wall_row(g, comp, kc, true, betadx, lo, up);
+          const double off = kc == 1 ? up : lo;
+          row.*x = serial ? 0.0 : off * D[q];
+          row.*xs = serial ? 0.0 : (1.0 + off) * D[q];
+        }
+      }
+      const bool slip = wall && ((kc == 1 && !(v & 1)) || (kc == nrm && !(v >> 1)));
+      const double e = serial ? 0.0 : (double)(sum[q] - (slip ? row.*xs : row.*f[comp][3]));
+      row.*(!wall ? &R::e_r : (qt ? et[v] : ez[v])) = e;
+    }
+  }
 }
 
 int refresh_tables(tc_ctx *c) {
   const int nsst = c->p.nsst;
   // the no-slip variant (3) and those that some line's masks ask for
   const unsigned vars = c->mask_vars | 8u;
-  bool any = !c->lu_valid || (vars & ~c->lu_vars) != 0;
+  auto serial_of = [&] {
+    unsigned s = 0;
+    for (int q = 0; q < 3; q++)
+      if (c->lu_pivots[q] & (q == tc::LU_QR ? 8u : c->mask_vars)) s |= 1u << q;
+    return s;
+  };
+  bool any = !c->lu_valid || (vars & ~c->lu_vars) != 0 || serial_of() != c->lu_serial;
   for (int s = 0; s < nsst; s++)
     if (c->lu_key[s] != c->beta * c->g.alm[s + 1]) any = true;
   if (!any) return 0;
   // the previous upload must have left the staging buffer
   HIPCHK(hipEventSynchronize(c->lu_copied));
   const size_t per_slot = tc::lu_slot_doubles(c);
-  unsigned pivots[3] = {0, 0, 0};
+  std::vector<Matrix> A;  // [slot][component][variant]
+  std::fill(c->lu_pivots, c->lu_pivots + 3, 0u);
+  for (int s = 0; s < nsst; s++) {
+    const double betadx = c->beta * c->g.alm[s + 1];
+    for (int q = 0; q < 3; q++)
+      for (int v = 0; v < 4; v++) {
+        const bool used = q == tc::LU_QR ? v == 3 : (vars >> v & 1) != 0;
+        A.push_back(!used ? Matrix(0)
+                          : (q == tc::LU_QR ? qr_matrix(c->g, betadx)
+                                            : wall_matrix(c->g, q, v & 1, v >> 1, betadx)));
+        if (used && write_serial(A.back(), nullptr, false)) c->lu_pivots[q] |= 1u << v;
+      }
+  }
+  c->lu_serial = serial_of();
   for (int s = 0; s < nsst; s++) {
     const double betadx = c->beta * c->g.alm[s + 1];
     double *base = c->lu_host + (size_t)s * per_slot;
     tc::RhsRow *rows = reinterpret_cast<tc::RhsRow *>(base + (size_t)3 * 4 * c->lu_nt);
-    for (int v = 0; v < 4; v++) {
-      if (!(vars >> v & 1)) continue;
-      build_wall_table(c->g, tc::LU_QT, v & 1, v >> 1, betadx,
-                       base + ((size_t)tc::LU_QT * 4 + v) * c->lu_nt, c->lu_nt, rows);
-      build_wall_table(c->g, tc::LU_QZ, v & 1, v >> 1, betadx,
-                       base + ((size_t)tc::LU_QZ * 4 + v) * c->lu_nt, c->lu_nt, rows);
-    }
-    build_qr_table(c->g, betadx, base + (size_t)tc::LU_QR * 4 * c->lu_nt, c->lu_nt, rows);
-    for (int t = 0; t < 12; t++) {
-      const bool used = t / 4 == tc::LU_QR ? t % 4 == 0 : (vars >> t % 4 & 1) != 0;
-      for (int r = 0; used && r < c->nr; r++)
-        if (base[(size_t)t * c->lu_nt + tc::LU_ROW * r + 5] != 0.0) pivots[t / 4] |= 1u << t % 4;
-    }
+    for (int q = 0; q < 3; q++)
+      build_component(c->g, q, vars, &A[(size_t)(s * 3 + q) * 4], betadx, (c->lu_serial >> q & 1) != 0,
+                      base + (size_t)q * 4 * c->lu_nt, c->lu_nt, rows);
     c->lu_key[s] = betadx;
   }
   HIPCHK(hipMemcpyAsync(c->lu, c->lu_host, sizeof(double) * per_slot * nsst, hipMemcpyHostToDevice,
@@ -200,7 +265,6 @@ int refresh_tables(tc_ctx *c) {
   HIPCHK(hipEventRecord(c->lu_copied, c->stream));
   c->lu_valid = true;
   c->lu_vars = vars;
-  std::copy(pivots, pivots + 3, c->lu_pivots);
   return 0;
 }
 

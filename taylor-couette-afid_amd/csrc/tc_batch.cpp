@@ -50,7 +50,7 @@ using Key = std::tuple<int, int, int, int, int, int, int, int, int, int, int, in
 
 Key group_key(const tc_ctx *c) {
   return Key(c->nthm, c->nzm, c->nrm, c->p.nsst, c->helm_lpt, c->poisson_pq,
-             (c->masks_uniform_one ? 1 : 0) + 2 * (int)tc::serial_comps(c), c->plan_t.lines,
+             (c->masks_uniform_one ? 1 : 0) + 2 * (int)c->lu_serial, c->plan_t.lines,
              c->plan_t.me, c->plan_t.padsh,
              c->plan_z.lines, c->plan_z.me * 1000 + c->plan_z.nt, c->plan_z.padsh,
              tc::defers_correction(c) ? 1 : 0);

@@ -58,23 +58,26 @@ struct FFTPlan {
   int padsh = 3;  // one LDS padding slot per 2^padsh points (31: none)
 };
 
-// Helmholtz LU tables: per (substep slot, component, mask variant) a block of
-// NT rows of LU_ROW doubles: dl, du, du2, rd=1/d, row scale, pivot flag, d, 0
-// (d, du, du2 are the rows of the upper factor U).
-// One row is one 64-byte scalar load.
+// Helmholtz tables: per (substep slot, component, mask variant) a block of NT
+// rows of LU_ROW doubles (one 64-byte load): m, u, -, r of the partitioned
+// solve, or dl, du, du2, 1/d and the exchange flag of the serial one.
 enum { LU_QT = 0, LU_QR = 1, LU_QZ = 2 };
 constexpr int LU_ROW = 8;
 
 // What the right-hand sides need of the Helmholtz matrices of plane k (row
 // k of each component), one record per plane and substep slot: the scaling
-// of the right-hand side and the off-diagonals of the row-normalised matrix
-// (unit diagonal).  x_t, x_z: the off-diagonal towards the interior of the
-// two wall rows where the wall is free-slip (k = 1: ap, k = nrm: am).
-// The q_r rows next to the walls do not couple to them (q_r is fixed there).
+// of the right-hand side, the off-diagonals and the row sum s + e of the
+// matrix that the factors multiply out to (e: what s rounds away, which
+// differs between the mask variants).  x, xs: off-diagonal and s of the two
+// wall rows where the wall is free-slip (k = 1: ap, k = nrm: am).  All but sc
+// are zero for a component that takes the serial form.  The q_r rows next to
+// the walls do not couple to them (q_r is fixed there).
 struct RhsRow {
-  double sc_t, am_t, ap_t, sc_r, am_r, ap_r, sc_z, am_z, ap_z, x_t, x_z, pad;
+  double sc_t, am_t, ap_t, s_t, sc_r, am_r, ap_r, s_r, e_r, sc_z, am_z, ap_z, s_z;
+  double e0_t, e1_t, e2_t, e3_t, e0_z, e1_z, e2_z, e3_z;  // by mask variant icyl + 2 ocyl
+  double x_t, xs_t, x_z, xs_z;
 };
-static_assert(sizeof(RhsRow) == 96, "RhsRow is twelve doubles");
+static_assert(sizeof(RhsRow) == 25 * 8, "RhsRow is twenty-five doubles");
 
 struct Timer {
   std::string name;
@@ -238,6 +241,7 @@ struct tc_ctx {
   // whose tables are built; those of them, per component (q_theta, q_r, q_z),
   // whose factors exchange rows
   unsigned mask_vars = 8, lu_vars = 0, lu_pivots[3] = {0, 0, 0};
+  unsigned lu_serial = 0;  // bit q: component q's tables are those of the serial solve
   // FFT
   tc::FFTPlan plan_t, plan_z;
   double2 *tw_t = nullptr, *tw_z = nullptr;
@@ -331,8 +335,6 @@ int set_deferral(tc_ctx *c, int mode);
 // the dt and step recorded in a restart file's header (nothing else is read)
 int restart_file_info(const char *path, double *dt, int *ntime);
 size_t lu_slot_doubles(const tc_ctx *c);
-// bit q: component q is solved by the serial form
-unsigned serial_comps(const tc_ctx *c);
 const double *lu_table(const tc_ctx *c, int ns, int comp);
 const RhsRow *rhs_rows(const tc_ctx *c, int ns);
 void launch_helmholtz_fused_g(tc_ctx *c, const StepDesc *tab, const BatchDyn *dyn, int ns, int n,

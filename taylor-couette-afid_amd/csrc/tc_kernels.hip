@@ -244,8 +244,8 @@ void launch_explicit_qr(tc_ctx *c) { launch_explicit<1>(c, "explicit_qr", TC_DPH
 void launch_explicit_qz(tc_ctx *c) { launch_explicit<2>(c, "explicit_qz", TC_QCAP); }
 
 // ---------------------------------------------------------------------------
-// Helmholtz solves.  The LU factors (dgttrf with partial pivoting of the
-// row-normalised matrices of SolveImpEqnUpdate_*) do not depend on the line
+// Helmholtz solves.  The LU factors (of the row-normalised matrices of
+// SolveImpEqnUpdate_*; by dgttrf where it exchanges rows) do not depend on the line
 // (j, i) except through the wall masks, so they come from a per-substep
 // table with one entry per mask combination.  Lanes run along theta so every
 // plane access is coalesced.  The right-hand sides are formed point by point
@@ -254,12 +254,14 @@ void launch_explicit_qz(tc_ctx *c) { launch_explicit<2>(c, "explicit_qz", TC_QCA
 // ---------------------------------------------------------------------------
 
 struct LUView {
-  const double *b;  // rows of LU_ROW doubles: dl du du2 rd sc pv
+  const double *b;  // rows of LU_ROW doubles
   DEVI double dl(int r) const { return b[LU_ROW * r]; }
   DEVI double du(int r) const { return b[LU_ROW * r + 1]; }
   DEVI double du2(int r) const { return b[LU_ROW * r + 2]; }
   DEVI double rd(int r) const { return b[LU_ROW * r + 3]; }
-  DEVI double pv(int r) const { return b[LU_ROW * r + 5]; }
+  DEVI double pv(int r) const { return b[LU_ROW * r + 4]; }
+  DEVI double m(int r) const { return dl(r); }
+  DEVI double u(int r) const { return du(r); }
 };
 DEVI LUView lu_view(const double *base) {
   LUView v;
@@ -382,20 +384,30 @@ __global__ __launch_bounds__(256) void k_implicit(GridDev g, ImpArgs a, const do
 // ---------------------------------------------------------------------------
 // Tridiagonal solves of the radial Helmholtz systems.  FOLD: the right-hand
 // sides are sc*rhs + A q, so the solution of A x' = sc*rhs + A q is
-// x' = q + x, the updated velocity itself, and q is not read (a few ulps of
-// q more rounding); otherwise q += x, as the reference adds it.
+// x' = q + x, the updated velocity itself, and q is not read; otherwise
+// q += x, as the reference adds it.  What the fold rounds passes through
+// A^-1, whose norm grows with beta*max|ac|, and so does a difference between
+// the A that is folded and the one that the rounded factors solve.  Hence the
+// factors of write_partitioned and row_fold's differences.  Relative error of
+// one solve of a smooth q, a model against extended precision, at beta*ac =
+// 2 / 4e4: 8e-17 / 1.4e-16 (a fold of U q behind the forward sweep 1.2e-16 /
+// 2.7e-16, of A q as it stands 1.3e-16 / 3.6e-15, q += x 4.5e-17); the
+// explicit radial term of the right-hand side alone rounds to 7e-15 at 4e4.
+// 30 steps of 256x256x193 against plain FP64: q_theta 5.6e-16, inner torque
+// 1.2e-14 (U q 1.6e-15 and 9e-14, A q 1.7e-15 and 1.4e-13).
 //
 // Partitioned over the block: a block owns 64 lines (lanes along theta) and
 // each of its waves a segment of at most R rows of them, held in registers,
 // so a line's rows are loaded as one batch and its dependent chain is as
-// long as a segment instead of the line.  Without row exchanges the factors
-// are A = L U with y_r = g_r - dl_(r-1) y_(r-1) and x_r = (y_r - du_r x_(r+1))
-// rd_r.  Each wave sweeps its segment with a zero incoming value and leaves
+// long as a segment instead of the line.  Without row exchanges the sweeps
+// are y_q = g_q + m_q y_(q-1) and x_q = y_q r_q + u_q x_(q+1).  Each wave sweeps its segment with a zero incoming value and leaves
 // the outgoing value and the product of its factors in LDS; the waves then
 // chain those (at most 15 terms) to their true incoming value, whose
 // contribution down the segment is the same recurrence on one number.  Twice:
 // downwards for L, upwards for U.  The factor products of a diagonally
-// dominant matrix stay below one, so this is as stable as the sweeps.
+// dominant matrix stay below one, so this is as stable as the sweeps.  All
+// multiply-adds are written out: a line has the same bits whether its block
+// shares one table or reads one a lane.
 //
 // The factors of a segment's rows are the same for all lanes (UNIFORM): the
 // lanes hold those of one row each and broadcast them by readlane.
@@ -424,12 +436,13 @@ template <int R, bool UNIFORM, bool FOLD, bool CHUNKS>
 DEVI void helm_solve_lines(const long long lgrp, const int comp, const GridDev &g,
                            double *__restrict__ q, const double *__restrict__ y,
                            const double *__restrict__ lu, double *ex) {
+#pragma clang fp contract(off)
   const int lane = threadIdx.x, NS = blockDim.y;
   const int p = __builtin_amdgcn_readfirstlane(threadIdx.y);
   const long long P = g.P, l = lgrp * 64 + lane;
   const bool ok = l < P;
   const long long lc = ok ? l : P - 1;
-  const int first = comp == 1 ? 1 : 0, n = g.nrm - first, last = first + n - 1;
+  const int first = comp == 1 ? 1 : 0, n = g.nrm - first;
   const LUView T = lu_view(lu);
   double *exc = ex, *exw = ex + NS * 64;  // outgoing values and factors, L
   double *uxc = ex + 2 * NS * 64, *uxw = ex + 3 * NS * 64;  // and U
@@ -441,20 +454,20 @@ DEVI void helm_solve_lines(const long long lgrp, const int comp, const GridDev &
     const int ch = pass < nc ? pass : 2 * (nc - 1) - pass;
     const int r0 = first + (ch > 0 ? n0 + (ch - 1) * cap : 0), rn = ch > 0 ? cap : n0;
     const int lo = r0 + p * rn / NS, S = r0 + (p + 1) * rn / NS - lo, Sm = max(S - 1, 0);
-    // -dl_(r-1), rd_r and -du_r rd_r of row lo + i (UNIFORM: of rows lo + lane
-    // and, past 64 rows, lo + 64 + lane, loaded before the rows so that their
-    // latency is not behind them).  Past the segment's S rows they are those
+    // m, r and u of row lo + i (UNIFORM: of rows lo + lane and, past 64 rows,
+    // lo + 64 + lane, loaded before the rows so that their latency is not
+    // behind them).  Past the segment's S rows they are those
     // of rows that pass a value on unchanged in both sweeps (right-hand side
     // zero), so the sweeps carry no conditions.
     constexpr int NK = (R + 63) / 64;
-    double kdl[NK], kdu[NK], krd[NK];
+    double km[NK], ku[NK], kr[NK];
     if constexpr (UNIFORM) {
 #pragma unroll
       for (int u = 0; u < NK; u++) {
         const int r = lo + min(lane + 64 * u, Sm);
-        kdl[u] = T.dl(max(r - 1, 0));
-        kdu[u] = T.du(r);
-        krd[u] = T.rd(r);
+        km[u] = T.m(r);
+        ku[u] = T.u(r);
+        kr[u] = T.rd(r);
       }
     }
     double v[R];
@@ -481,30 +494,30 @@ DEVI void helm_solve_lines(const long long lgrp, const int comp, const GridDev &
     if constexpr (UNIFORM) {
 #pragma unroll
       for (int u = 0; u < NK; u++) {
-        const int i = lane + 64 * u, r = lo + i;
-        kdl[u] = i < S ? (r > first ? -kdl[u] : 0.0) : 1.0;
-        kdu[u] = i < S ? (r < last ? -kdu[u] * krd[u] : 0.0) : 1.0;
-        krd[u] = i < S ? krd[u] : 0.0;
+        const int i = lane + 64 * u;
+        km[u] = i < S ? km[u] : 1.0;
+        ku[u] = i < S ? ku[u] : 1.0;
+        kr[u] = i < S ? kr[u] : 0.0;
       }
     }
-    auto dl = [&](int i) {
-      if constexpr (UNIFORM) return rlane(kdl[i >> 6], i & 63);
-      else return lo + i > first ? -T.dl(lo + i - 1) : 0.0;
+    auto m = [&](int i) {
+      if constexpr (UNIFORM) return rlane(km[i >> 6], i & 63);
+      else return T.m(lo + i);
     };
     auto rd = [&](int i) {
-      if constexpr (UNIFORM) return rlane(krd[i >> 6], i & 63);
+      if constexpr (UNIFORM) return rlane(kr[i >> 6], i & 63);
       else return T.rd(lo + i);
     };
-    auto ud = [&](int i) {
-      if constexpr (UNIFORM) return rlane(kdu[i >> 6], i & 63);
-      else return lo + i < last ? -T.du(lo + i) * T.rd(lo + i) : 0.0;
+    auto up = [&](int i) {
+      if constexpr (UNIFORM) return rlane(ku[i >> 6], i & 63);
+      else return T.u(lo + i);
     };
     double c = 0.0, w = 1.0;
 #pragma unroll
     for (int i = 0; i < R; i++) {
       if (!UNIFORM && i >= S) continue;
-      const double d = dl(i);
-      c = (i < S ? v[i] : 0.0) + d * c;
+      const double d = m(i);
+      c = fma(d, c, i < S ? v[i] : 0.0);
       v[i] = c;
       w = w * d;
     }
@@ -514,25 +527,26 @@ DEVI void helm_solve_lines(const long long lgrp, const int comp, const GridDev &
     w = CHUNKS ? enter[ch * 64 + lane] : 0.0;
     if (CHUNKS && pass < nc - 1) {
       // downwards: only the value that enters the next chunk
-      for (int s = 0; s < NS; s++) w = exc[s * 64 + lane] + exw[s * 64 + lane] * w;
+      for (int s = 0; s < NS; s++) w = fma(exw[s * 64 + lane], w, exc[s * 64 + lane]);
       if (p == 0) enter[(ch + 1) * 64 + lane] = w;
       __syncthreads();
       continue;
     }
-    for (int s = 0; s < p; s++) w = exc[s * 64 + lane] + exw[s * 64 + lane] * w;
+    for (int s = 0; s < p; s++) w = fma(exw[s * 64 + lane], w, exc[s * 64 + lane]);
 #pragma unroll
     for (int i = 0; i < R; i++) {
       if (!UNIFORM && i >= S) continue;
-      w = w * dl(i);
-      v[i] = v[i] + w;
+      const double d = m(i);
+      v[i] = fma(w, d, v[i]);
+      w = w * d;
     }
     c = 0.0;
     w = 1.0;
 #pragma unroll
     for (int i = R - 1; i >= 0; i--) {
       if (!UNIFORM && i >= S) continue;
-      const double u = ud(i);
-      c = v[i] * rd(i) + u * c;
+      const double u = up(i);
+      c = fma(u, c, v[i] * rd(i));
       v[i] = c;
       w = w * u;
     }
@@ -540,18 +554,19 @@ DEVI void helm_solve_lines(const long long lgrp, const int comp, const GridDev &
     uxw[p * 64 + lane] = w;
     __syncthreads();
     w = below;
-    for (int s = NS - 1; s > p; s--) w = uxc[s * 64 + lane] + uxw[s * 64 + lane] * w;
+    for (int s = NS - 1; s > p; s--) w = fma(uxw[s * 64 + lane], w, uxc[s * 64 + lane]);
     if constexpr (CHUNKS) {
-      for (int s = NS - 1; s >= 0; s--) below = uxc[s * 64 + lane] + uxw[s * 64 + lane] * below;
+      for (int s = NS - 1; s >= 0; s--) below = fma(uxw[s * 64 + lane], below, uxc[s * 64 + lane]);
     }
     double *qp = q + (long long)lo * P + l;
 #pragma unroll
     for (int i = R - 1; i >= 0; i--) {
       if (!UNIFORM && i >= S) continue;
-      w = w * ud(i);
+      const double u = up(i), x = fma(w, u, v[i]);
+      w = w * u;
       if (i < S && ok) {
         double *o = qp + (long long)i * P;
-        st_nt(o, FOLD ? v[i] + w : *o + (v[i] + w));
+        st_nt(o, FOLD ? x : *o + x);
       }
     }
     if constexpr (CHUNKS) __syncthreads();  // exc and uxc are written again
@@ -623,13 +638,14 @@ __global__ __launch_bounds__(R > 32 ? 512 : 1024) void k_helm_solve_g(
 }
 
 // Serial form, one line per lane: dgttrs as it is, for factors with row
-// exchanges.  y is overwritten by the forward sweep.  Loads are issued a chunk of rows ahead
+// exchanges; q += x (the right-hand sides hold no A q).  y is overwritten by
+// the forward sweep.  Loads are issued a chunk of rows ahead
 // of the dependent recurrence.
 DEVI void helm_solve_serial_body(const long long l, const int comp, const GridDev &g,
                                  double *__restrict__ q, double *__restrict__ y,
                                  const unsigned char *__restrict__ icyl,
                                  const unsigned char *__restrict__ ocyl,
-                                 const double *__restrict__ lu, int nt, bool fold) {
+                                 const double *__restrict__ lu, int nt) {
   constexpr int CH = 16;
   if (l >= g.P) return;
   const long long P = g.P;
@@ -655,7 +671,7 @@ DEVI void helm_solve_serial_body(const long long l, const int comp, const GridDe
   double x1 = 0.0, x0 = carry * T.rd(last);
   auto put = [&](int r, double x) {
     double *o = q + (long long)r * P + l;
-    *o = fold ? x : *o + x;
+    *o = *o + x;
   };
   put(last, x0);
   for (int r0 = last - 1; r0 >= first; r0 -= CH) {
@@ -680,11 +696,11 @@ DEVI void helm_solve_serial_body(const long long l, const int comp, const GridDe
 __global__ __launch_bounds__(256) void k_helm_solve_serial(GridDev g, SolveIO io,
                                                            const unsigned char *__restrict__ icyl,
                                                            const unsigned char *__restrict__ ocyl,
-                                                           int nt, int comp, bool fold) {
+                                                           int nt, int comp) {
   helm_solve_serial_body((long long)blockIdx.x * 256 + threadIdx.x, comp, g,
                          comp == 0 ? io.q[0] : (comp == 1 ? io.q[1] : io.q[2]),
                          const_cast<double *>(comp == 0 ? io.y[0] : (comp == 1 ? io.y[1] : io.y[2])),
-                         icyl, ocyl, comp == 0 ? io.lu[0] : (comp == 1 ? io.lu[1] : io.lu[2]), nt, fold);
+                         icyl, ocyl, comp == 0 ? io.lu[0] : (comp == 1 ? io.lu[1] : io.lu[2]), nt);
 }
 
 // Grouped: blockIdx.y = instance.
@@ -696,7 +712,7 @@ __global__ __launch_bounds__(256) void k_helm_solve_serial_g(const StepDesc *__r
                          glob(d.f[comp == 0 ? TC_QT : (comp == 1 ? TC_QR : TC_QZ)]),
                          glob(d.f[comp == 0 ? TC_RHS : (comp == 1 ? TC_DQ : TC_QCAP)]),
                          glob(d.icyl), glob(d.ocyl),
-                         glob(comp == 0 ? d.lut : (comp == 1 ? d.lur : d.luz)), d.lu_nt, true);
+                         glob(comp == 0 ? d.lut : (comp == 1 ? d.lur : d.luz)), d.lu_nt);
 }
 
 // ---------------------------------------------------------------------------
@@ -731,6 +747,27 @@ DEVI double corr_pr(const GridDev &g, int kc, double p, double d, double dim, do
   return p + d -
          be * ((dip - 2.0 * d + dim) * ldk(g.udx1qm + kc) + (djp - 2.0 * d + djm) * g.dxzq +
                (dkp * app + d * acc + dkm * amm));
+}
+
+// Row k of D (sc rhs + A q) from the records' scaled entries, with A q in
+// differences: (s + e) q + am (q(k-1) - q) + ap (q(k+1) - q) with the row sum
+// s + e, which is small where beta*ac is large, as the differences are there.
+// The term of q's size is added last, so that it is rounded once.
+DEVI double row_fold(double s, double e, double am, double ap, double scr, double qm, double q0,
+                     double qp) {
+  return fma(s, q0, fma(e, q0, fma(am, qm - q0, fma(ap, qp - q0, scr))));
+}
+// e of a line's mask variant: ic, oc its bits
+DEVI double row_e(double e0, double e1, double e2, double e3, bool ic, bool oc) {
+  const double i = ic ? e3 : e2, o = ic ? e1 : e0;
+  return oc ? i : o;
+}
+
+// The same for a point beside a free-slip wall: one off-diagonal, x, towards
+// the interior value qi, and the row sum xs, read here so that the planes
+// without walls hold neither.
+DEVI double wall_fold(const double *x, const double *xs, double e, double scr, double q0, double qi) {
+  return fma(ldk(xs), q0, fma(e, q0, fma(ldk(x), qi - q0, scr)));
 }
 
 constexpr int FT_N = 256, FT_I = 64, FT_J = FT_N / FT_I, FT_W = FT_I + 2;
@@ -913,12 +950,11 @@ DEVI void helm_rhs_body(
       Z.m00 = cm[u][3]; Z.m01 = 0.0; Z.m10 = cm[u][4];
       const double pr_c = spk[base[u]], pr_im = spk[base[u] - 1], pr_jm = spk[base[u] - FT_W];
       const long long o = (long long)(k - 1) * P + l[u];
-      // the matrix rows of q_theta and q_z next to a free-slip wall
-      double am_t = rw.am_t, ap_t = rw.ap_t, am_z = rw.am_z, ap_z = rw.ap_z;
-      if constexpr (!UNIFORM) {
-        if (k == 1 && fic[u] == 0.0) ap_t = rw.x_t, ap_z = rw.x_z;
-        if (k == nrm && foc[u] == 0.0) am_t = rw.x_t, am_z = rw.x_z;
-      }
+      // whether the matrix rows of q_theta and q_z are those beside a free-slip wall
+      const bool ic = UNIFORM || fic[u] != 0.0, oc = UNIFORM || foc[u] != 0.0;
+      const bool slip1 = k == 1 && !ic, slipn = k == nrm && !oc;
+      const double e_t = row_e(rw.e0_t, rw.e1_t, rw.e2_t, rw.e3_t, ic, oc);
+      const double e_z = row_e(rw.e0_z, rw.e1_z, rw.e2_z, rw.e3_z, ic, oc);
       // q_theta
       {
         const double dqv = explicit_qt_g(g, hc, T, R, Z, k);
@@ -926,14 +962,18 @@ DEVI void helm_rhs_body(
         double r = rhs_qt<UNIFORM>(g, hc, a, k, qm, T(0, 0, 0), qp, pr_c, pr_im, dqv, h1[u], fic[u], foc[u]);
         st_nt(ru1 + o, dqv);
         if (k == 1) r = r + a.bc1;
-        st_nt(yt + o, r * rw.sc_t + (am_t * qm + T(0, 0, 0) + ap_t * qp));
+        double y = row_fold(rw.s_t, e_t, rw.am_t, rw.ap_t, r * rw.sc_t, qm, T(0, 0, 0), qp);
+        if (slip1 || slipn)
+          y = wall_fold(&rows[k].x_t, &rows[k].xs_t, e_t, r * rw.sc_t, T(0, 0, 0), slip1 ? qp : qm);
+        st_nt(yt + o, y);
       }
             // q_r (planes 2..nrm; the walls have no row)
       if (k >= 2) {
         const double dphv = explicit_qr_g(g, hc, T, R, Z, k);
         const double r = rhs_qr(hc, a, R(-1, 0, 0), R(0, 0, 0), R(1, 0, 0), pr_c, pr_km[u], dphv, h2[u]);
         st_nt(ru2 + o, dphv);
-        st_nt(yr + o, r * rw.sc_r + (rw.am_r * R(-1, 0, 0) + R(0, 0, 0) + rw.ap_r * R(1, 0, 0)));
+        st_nt(yr + o, row_fold(rw.s_r, rw.e_r, rw.am_r, rw.ap_r, r * rw.sc_r, R(-1, 0, 0), R(0, 0, 0),
+                                R(1, 0, 0)));
       }
             // q_z
       {
@@ -941,7 +981,10 @@ DEVI void helm_rhs_body(
         const double qm = (k > 1) ? Z(-1, 0, 0) : 0.0, qp = (k < nrm) ? Z(1, 0, 0) : 0.0;
         const double r = rhs_qz<UNIFORM>(g, hc, a, k, qm, Z(0, 0, 0), qp, pr_c, pr_jm, qcv, h3[u], fic[u], foc[u]);
         st_nt(ru3 + o, qcv);
-        st_nt(yz + o, r * rw.sc_z + (am_z * qm + Z(0, 0, 0) + ap_z * qp));
+        double y = row_fold(rw.s_z, e_z, rw.am_z, rw.ap_z, r * rw.sc_z, qm, Z(0, 0, 0), qp);
+        if (slip1 || slipn)
+          y = wall_fold(&rows[k].x_z, &rows[k].xs_z, e_z, r * rw.sc_z, Z(0, 0, 0), slip1 ? qp : qm);
+        st_nt(yz + o, y);
       }
             pr_km[u] = pr_c;
       cm[u][0] = T(0, 0, 0);
@@ -985,10 +1028,11 @@ DEVI void helm_rhs_body(
 // Against one line or two z-rows of lines per thread, with the correction:
 // 256x256x193 343 -> 318 us, 512x512x385 2576 -> 2491 us, 1024x1024x769 20.5
 // -> 17.95 ms (HBM bound at the larger sizes: 4.9 of the 5.7 TB/s that
-// fifteen streamed arrays reach).  The kernels ask for two waves per SIMD,
-// which the masked form leaves by a few registers when it is not asked to:
-// grooved walls, corrected, 192x128x129 125 us at one wave, 88 at two,
-// 256x256x193 447 and 335.
+// fifteen streamed arrays reach).  The kernels ask for two waves per SIMD:
+// the masked form, corrected, once left that when it was not asked to
+// (192x128x129 125 us at one wave, 88 at two).  It holds what only the two
+// wall planes need nowhere else (wall_fold) and takes 222 registers with none
+// spilled; with the wall rows' entries in every plane 24 to 53 were.
 // (The outermost column of the tile on either side is staged only to keep
 // pairs aligned; nothing reads it.)
 constexpr int PT_W = FT_I + 4, PT_P = PT_W / 2;  // tile row: i0-2 .. i0+65
@@ -1222,32 +1266,36 @@ DEVI void helm_rhs_pair_body(
         Z.m00 = cm[5 + u]; Z.m01 = 0.0; Z.m10 = cm[7 + u];
         const double fic = (double)(wall >> u & 1), foc = (double)(wall >> u >> 2 & 1);
         const double pr_c = spk[b], pr_im = spk[b - 1], pr_jm = spk[b - PT_W];
-        // the matrix rows of q_theta and q_z next to a free-slip wall
-        double am_t = rw.am_t, ap_t = rw.ap_t, am_z = rw.am_z, ap_z = rw.ap_z;
-        if constexpr (!UNIFORM) {
-          if (k == 1 && !(wall >> u & 1)) ap_t = rw.x_t, ap_z = rw.x_z;
-          if (k == nrm && !(wall >> u & 4)) am_t = rw.x_t, am_z = rw.x_z;
-        }
+        // whether the matrix rows of q_theta and q_z are those beside a free-slip wall
+        const bool ic = UNIFORM || (wall >> u & 1), oc = UNIFORM || (wall >> u & 4);
+        const bool slip1 = k == 1 && !ic, slipn = k == nrm && !oc;
+        const double e_t = row_e(rw.e0_t, rw.e1_t, rw.e2_t, rw.e3_t, ic, oc);
+        const double e_z = row_e(rw.e0_z, rw.e1_z, rw.e2_z, rw.e3_z, ic, oc);
         // q_theta
         e1[u] = explicit_qt_g(g, hc, T, R, Z, k);
         const double tm = (k > 1) ? T(-1, 0, 0) : 0.0, tp = (k < nrm) ? T(1, 0, 0) : 0.0;
         double r = rhs_qt<UNIFORM>(g, hc, a, k, tm, T(0, 0, 0), tp, pr_c, pr_im, e1[u],
                                    u ? h1.y : h1.x, fic, foc);
         if (k == 1) r = r + a.bc1;
-        g1[u] = r * rw.sc_t + (am_t * tm + T(0, 0, 0) + ap_t * tp);
+        g1[u] = row_fold(rw.s_t, e_t, rw.am_t, rw.ap_t, r * rw.sc_t, tm, T(0, 0, 0), tp);
+        if (slip1 || slipn)
+          g1[u] = wall_fold(&rows[k].x_t, &rows[k].xs_t, e_t, r * rw.sc_t, T(0, 0, 0), slip1 ? tp : tm);
         // q_r (planes 2..nrm; the walls have no row)
         if (k >= 2) {
           e2[u] = explicit_qr_g(g, hc, T, R, Z, k);
           r = rhs_qr(hc, a, R(-1, 0, 0), R(0, 0, 0), R(1, 0, 0), pr_c, u ? pkm.y : pkm.x, e2[u],
                      u ? h2.y : h2.x);
-          g2[u] = r * rw.sc_r + (rw.am_r * R(-1, 0, 0) + R(0, 0, 0) + rw.ap_r * R(1, 0, 0));
+          g2[u] = row_fold(rw.s_r, rw.e_r, rw.am_r, rw.ap_r, r * rw.sc_r, R(-1, 0, 0), R(0, 0, 0),
+                           R(1, 0, 0));
         }
         // q_z
         e3[u] = explicit_qz_g(g, hc, T, R, Z, k);
         const double zm = (k > 1) ? Z(-1, 0, 0) : 0.0, zp = (k < nrm) ? Z(1, 0, 0) : 0.0;
         r = rhs_qz<UNIFORM>(g, hc, a, k, zm, Z(0, 0, 0), zp, pr_c, pr_jm, e3[u], u ? h3.y : h3.x,
                             fic, foc);
-        g3[u] = r * rw.sc_z + (am_z * zm + Z(0, 0, 0) + ap_z * zp);
+        g3[u] = row_fold(rw.s_z, e_z, rw.am_z, rw.ap_z, r * rw.sc_z, zm, Z(0, 0, 0), zp);
+        if (slip1 || slipn)
+          g3[u] = wall_fold(&rows[k].x_z, &rows[k].xs_z, e_z, r * rw.sc_z, Z(0, 0, 0), slip1 ? zp : zm);
         if (u)
           pkm.y = pr_c;
         else
@@ -1376,18 +1424,6 @@ const RhsRow *rhs_rows(const tc_ctx *c, int ns) {
 
 static unsigned line_blocks(const tc_ctx *c) { return (unsigned)((c->P + 255) / 256); }
 
-// Components whose factors exchange rows on some line.  Only those take the
-// serial form, and only while the masks hold such lines: tables that no line
-// reads (of a free-slip outer wall, which SlipBCs never sets) or that a former
-// pattern read do not count.  (They did: 192x128x129 with grooves at beta*ac
-// of a few took 87 us a solve instead of 38.)
-unsigned serial_comps(const tc_ctx *c) {
-  unsigned s = c->lu_pivots[LU_QR] ? 1u << LU_QR : 0u;
-  for (int q : {LU_QT, LU_QZ})
-    if (c->lu_pivots[q] & c->mask_vars) s |= 1u << q;
-  return s;
-}
-
 // Shape of the partitioned solve: waves per block and the row capacity R of
 // its kernel, by the grid's shape alone (an instance's bits must not depend
 // on what it shares a launch with).  Past eight waves of 100 rows a line goes in chunks.  Few rows a
@@ -1440,14 +1476,14 @@ static void launch_solve_u(const SolveShape s, dim3 grid, hipStream_t st, const 
 // otherwise the one component comp0
 template <bool FOLD>
 static void launch_solve(tc_ctx *c, const SolveIO &io, int comp0, int ncomp) {
-  const unsigned serial = serial_comps(c);
+  const unsigned serial = c->lu_serial;
   if (ncomp > 1 && serial) {
     for (int q = 0; q < ncomp; q++) launch_solve<FOLD>(c, io, comp0 + q, 1);
     return;
   }
   if (serial >> comp0 & 1) {
     hipLaunchKernelGGL(k_helm_solve_serial, dim3(line_blocks(c)), dim3(256), 0, c->stream, c->gd, io,
-                       c->mask, c->mask + c->P, c->lu_nt, comp0, FOLD);
+                       c->mask, c->mask + c->P, c->lu_nt, comp0);
     return;
   }
   const SolveShape s = solve_shape(c);
@@ -2600,7 +2636,7 @@ void launch_helmholtz_fused_g(tc_ctx *c, const StepDesc *tab, const BatchDyn *dy
     else launch_rhs_g<false, 1>(c, tab, dyn, ns, n, st, corr);
   }
   const SolveShape s = solve_shape(c);
-  const unsigned serial = serial_comps(c), ncomp = serial ? 1 : 3;
+  const unsigned serial = c->lu_serial, ncomp = serial ? 1 : 3;
   const dim3 grid((unsigned)((c->P + 63) / 64), ncomp, (unsigned)n);
   for (int q = 0; q < 3; q += (int)ncomp) {
     if (serial >> q & 1)

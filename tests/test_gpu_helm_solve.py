@@ -156,3 +156,44 @@ def test_row_exchanges_of_other_lines_change_nothing(tc):
         assert np.array_equal(after[f], plain[f]), f
     for masked in (inner, outer):
         assert np.array_equal(masked["qr"], plain["qr"])
+
+
+@pytest.mark.parametrize("strength", [1.5, 3.5])
+def test_folded_solve_does_not_amplify_its_rounding(tc, strength):
+    """One AB2 step of a flow that is 1 in the inner half and 2 in the outer,
+    whose explicit terms vanish: the fused step folds q into the radial
+    solve, the routines add the solution to q.  Powers of two make every
+    product of the right-hand side exact, so both solve for the same one (in
+    general they contract its products differently, which alone is 6e-15 of q
+    on the clustered rows) and differ by what the fold rounds.  On rows
+    clustered so that beta*ac is some tens and some ten thousands a fold that
+    cancels loses 2e-16 and 4e-15 of q (a model of the same systems against
+    extended precision); three roundings of q's size and the solve's own give
+    3e-16 at either.  Bound: three times that."""
+    p = small_params(tc, 16, 12, 385, nsst=1, ntst=1000, ren=1e3, str=strength, dtmin=1e-2, dtmax=1e-2,
+                     virotext=0.5)
+    out = []
+    for fused in (True, False):
+        d = tc.Solver(p)
+        d.set_fused(fused)
+        q = np.zeros(d.shape, order="F")
+        q[:192], q[192:385] = 1.0, 2.0
+        d.set("qt", q), d.set("qz", q)
+        d.set_time(0.0, p["dtmax"])
+        d.TimeMarcher()
+        out.append({f: d.get(f)[:385] for f in ("qt", "qz")})
+    for f in ("qt", "qz"):
+        assert rel_l2(out[0][f], out[1][f]) <= 9e-16, f
+
+
+def test_a_line_keeps_its_bits_beside_other_lines(tc):
+    """No-slip lines beside grooves of the inner wall, where each lane reads
+    its own table, and among themselves, where a block shares one."""
+    p = small_params(tc, 20, 9, 33, ren=50.0)
+    ones = np.ones((p["nzm"], p["nthm"]), np.int32)
+    half = ones.copy()
+    half[:, ::2] = 0
+    plain = _slip_implicit(tc, p, 0.3, (ones, ones))
+    inner = _slip_implicit(tc, p, 0.3, (half, ones))
+    for f in ("qt", "qr", "qz"):
+        assert np.array_equal(inner[f][:, :, 1::2], plain[f][:, :, 1::2]), f
