@@ -21,7 +21,7 @@ ALX3D = 2 pi, VIROTINT = 1, STR3 = 1.5 with ISTR = 4, RESID = 1e-6.
 arrival order; a job is admitted when a slot is free, its device footprint
 fits the HBM budget and the resident grid points stay under ``max_cells``
 (enough to keep the device saturated; beyond it every resident job would
-only slow the others down).  A job that does not fit may be overtaken by a
+only slow the others down: one 384^2x289 job and a 256^2x193 one by default).  A job that does not fit may be overtaken by a
 later one that does (backfill).  Admitted jobs stay resident in one
 ``Batch`` per grid shape, each advanced by its own thread on its own
 streams, so small jobs do not wait for the step of a large one; each
@@ -337,7 +337,7 @@ class Server:
     each advanced by its own thread; admission is global."""
 
     def __init__(self, tc, hbm_budget=200e9, chunk=25, graph=True, tuning=None, workers=4,
-                 max_slots=16, max_cells=400e6, order="arrival", checkpoint_dir=None,
+                 max_slots=16, max_cells=60e6, order="arrival", checkpoint_dir=None,
                  checkpoint_every=0):
         # graph=True: each class worker replays its batch's whole step as a
         # hipGraph, captured again whenever jobs join or leave.
@@ -355,6 +355,10 @@ class Server:
         self.checkpoint_every = int(checkpoint_every)
         self.tc = tc
         self.budget = hbm_budget
+        # Two traces of 12 jobs, max_cells 400e6 / 60e6 / 20e6: p50 6.8 / 4.6 /
+        # 2.4 s and 5.9 / 4.3 / 2.1, p99 25.5 / 24.4 / 25.4 and 17.5 / 17.0 /
+        # 18.3, mean 9.8 / 7.3 / 6.5 and 6.6 / 5.2 / 4.1, jobs/h 1402 / 1353 /
+        # 1312 and 2144 / 2102 / 1971.
         self.max_slots = max_slots
         self.max_cells = max_cells
         self.chunk = chunk

@@ -276,3 +276,12 @@ def test_checkpoints_follow_the_cadence_and_resume_continues(tc, tmp_path):
     assert writes[-1] == 40
     with pytest.raises(ValueError):
         sw.Server(ftc, checkpoint_every=5)
+
+
+def test_default_residency_holds_one_of_the_largest_jobs(tc):
+    """Lone jobs of the larger shapes run near the device's rate, so a second
+    384^2x289 job resident beside the first only delays the short ones; a
+    256^2x193 one still fits beside it."""
+    sw = importlib.import_module("taylor-couette-afid_amd.sweep")
+    cells = [a * b * c for a, b, c in sw.SERVED_GRIDS]
+    assert max(cells) + sorted(cells)[-2] <= sw.Server(FakeTC(tc)).max_cells < 2 * max(cells)
