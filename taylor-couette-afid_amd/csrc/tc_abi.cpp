@@ -111,32 +111,48 @@ double rhs_scale(const tc::Grid &g, int comp, int kc, double betadx) {
   return 1.0 / (1.0 - ac[kc] * betadx);
 }
 
-// Factors of A with row exchanges, as dgttrf forms them: rows of dl, du, du2,
-// rd, pv for the serial solve.  True where a row was exchanged.  A matrix
-// whose row sums are not negative (its off-diagonals are not positive) is
-// diagonally dominant and needs no exchange.
-bool write_serial(const Matrix &A, double *T, bool write) {
-  constexpr int W = tc::LU_ROW;
-  const int n = (int)A.lo.size();
-  bool dominant = true;
-  for (int q = 0; q < n && !write; q++) dominant = dominant && A.sum(q) >= 0.0;
-  if (!write && dominant) return false;
-  std::vector<double> dl(A.lo.begin() + 1, A.lo.end()), d((size_t)n, 1.0), du(A.up), du2((size_t)n, 0.0);
-  std::vector<int> ipiv((size_t)n);
-  dl.push_back(0.0);
-  tc::dgttrf(n, dl.data(), d.data(), du.data(), du2.data(), ipiv.data());
-  bool exchanged = false;
-  for (int q = 0; q < n; q++) {
-    const bool pv = q < n - 1 && ipiv[q] != q;
-    exchanged = exchanged || pv;
-    if (!write) continue;
-    T[W * q] = q < n - 1 ? dl[q] : 0.0;
-    T[W * q + 1] = q < n - 1 ? du[q] : 0.0;
-    T[W * q + 2] = q < n - 2 ? du2[q] : 0.0;
-    T[W * q + 3] = 1.0 / d[q];
-    T[W * q + 4] = pv ? 1.0 : 0.0;
+// Factors of A with row exchanges, as dgttrf forms them.
+struct Exchanged {
+  std::vector<double> dl, d, du, du2;
+  std::vector<int> ipiv;
+  explicit Exchanged(const Matrix &A)
+      : dl(A.lo.begin() + 1, A.lo.end()), d(A.lo.size(), 1.0), du(A.up), du2(A.lo.size(), 0.0), ipiv(A.lo.size()) {
+    dl.push_back(0.0);
+    tc::dgttrf((int)d.size(), dl.data(), d.data(), du.data(), du2.data(), ipiv.data());
   }
+  bool at(int q) const { return q + 1 < (int)d.size() && ipiv[q] != q; }
+};
+
+// Whether A's factors exchange rows.  A matrix whose row sums are not negative
+// (its off-diagonals are not positive) is diagonally dominant and needs none.
+bool needs_exchange(const Matrix &A) {
+  const int n = (int)A.lo.size();
+  bool dominant = true, exchanged = false;
+  for (int q = 0; q < n; q++) dominant = dominant && A.sum(q) >= 0.0;
+  if (dominant) return false;
+  const Exchanged f(A);
+  for (int q = 0; q < n; q++) exchanged = exchanged || f.at(q);
   return exchanged;
+}
+
+// The serial solve's rows of dl, du, du2, rd, pv.  sum as in
+// write_partitioned: the eliminations are undone from the last row up.
+void write_serial(const Matrix &A, double *T, std::vector<long double> &sum) {
+  constexpr int W = tc::LU_ROW;
+  const Exchanged f(A);
+  const int n = (int)f.d.size();
+  for (int q = n - 1; q >= 0; q--) {
+    const double du = q < n - 1 ? f.du[q] : 0.0, du2 = q < n - 2 ? f.du2[q] : 0.0;
+    sum[q] = (long double)f.d[q] + du + du2;
+    T[W * q] = q < n - 1 ? f.dl[q] : 0.0;
+    T[W * q + 1] = du;
+    T[W * q + 2] = du2;
+    T[W * q + 3] = 1.0 / f.d[q];
+    T[W * q + 4] = f.at(q) ? 1.0 : 0.0;
+    if (q == n - 1) continue;
+    sum[q + 1] += f.dl[q] * sum[q];
+    if (f.at(q)) std::swap(sum[q], sum[q + 1]);
+  }
 }
 
 // Factors of D A without row exchanges for the partitioned solve, rows of m,
@@ -192,7 +208,7 @@ void build_component(const tc::Grid &g, int comp, unsigned vars, const Matrix *A
     double *Tv = T + (size_t)(wall ? v : 0) * nt;
     std::fill(Tv, Tv + nt, 0.0);
     if (serial)
-      write_serial(A[v], Tv, true);
+      write_serial(A[v], Tv, sum);
     else
       write_partitioned(A[v], k0 - 1, nrm - 1, D, v == 3, Tv, sum);
     for (int kc = k0; kc <= nrm; kc++) {
@@ -200,21 +216,20 @@ void build_component(const tc::Grid &g, int comp, unsigned vars, const Matrix *A
       const int q = kc - 1;
       if (v == 3) {
         row.*f[comp][0] = rhs_scale(g, comp, kc, betadx) * D[q];
-        // the serial form adds its solution to q
-        row.*f[comp][1] = serial ? 0.0 : -Tv[tc::LU_ROW * q];
-        row.*f[comp][2] = serial ? 0.0 : -Tv[tc::LU_ROW * q + 1];
-        row.*f[comp][3] = serial ? 0.0 : (double)sum[q];
+        row.*f[comp][1] = serial ? A[3].lo[q] : -Tv[tc::LU_ROW * q];
+        row.*f[comp][2] = serial ? A[3].up[q] : -Tv[tc::LU_ROW * q + 1];
+        row.*f[comp][3] = (double)sum[q];
         if (wall && (kc == 1 || kc == nrm)) {
           // beside a free-slip wall: one off-diagonal
           double lo, up;
           wall_row(g, comp, kc, true, betadx, lo, up);
           const double off = kc == 1 ? up : lo;
-          row.*x = serial ? 0.0 : off * D[q];
-          row.*xs = serial ? 0.0 : (1.0 + off) * D[q];
+          row.*x = off * D[q];
+          row.*xs = (1.0 + off) * D[q];
         }
       }
       const bool slip = wall && ((kc == 1 && !(v & 1)) || (kc == nrm && !(v >> 1)));
-      const double e = serial ? 0.0 : (double)(sum[q] - (slip ? row.*xs : row.*f[comp][3]));
+      const double e = (double)(sum[q] - (slip ? row.*xs : row.*f[comp][3]));
       row.*(!wall ? &R::e_r : (qt ? et[v] : ez[v])) = e;
     }
   }
@@ -247,7 +262,7 @@ int refresh_tables(tc_ctx *c) {
         A.push_back(!used ? Matrix(0)
                           : (q == tc::LU_QR ? qr_matrix(c->g, betadx)
                                             : wall_matrix(c->g, q, v & 1, v >> 1, betadx)));
-        if (used && write_serial(A.back(), nullptr, false)) c->lu_pivots[q] |= 1u << v;
+        if (used && needs_exchange(A.back())) c->lu_pivots[q] |= 1u << v;
       }
   }
   c->lu_serial = serial_of();

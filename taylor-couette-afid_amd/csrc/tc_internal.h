@@ -69,9 +69,8 @@ constexpr int LU_ROW = 8;
 // of the right-hand side, the off-diagonals and the row sum s + e of the
 // matrix that the factors multiply out to (e: what s rounds away, which
 // differs between the mask variants).  x, xs: off-diagonal and s of the two
-// wall rows where the wall is free-slip (k = 1: ap, k = nrm: am).  All but sc
-// are zero for a component that takes the serial form.  The q_r rows next to
-// the walls do not couple to them (q_r is fixed there).
+// wall rows where the wall is free-slip (k = 1: ap, k = nrm: am).  The q_r
+// rows next to the walls do not couple to them (q_r is fixed there).
 struct RhsRow {
   double sc_t, am_t, ap_t, s_t, sc_r, am_r, ap_r, s_r, e_r, sc_z, am_z, ap_z, s_z;
   double e0_t, e1_t, e2_t, e3_t, e0_z, e1_z, e2_z, e3_z;  // by mask variant icyl + 2 ocyl

@@ -638,14 +638,13 @@ __global__ __launch_bounds__(R > 32 ? 512 : 1024) void k_helm_solve_g(
 }
 
 // Serial form, one line per lane: dgttrs as it is, for factors with row
-// exchanges; q += x (the right-hand sides hold no A q).  y is overwritten by
-// the forward sweep.  Loads are issued a chunk of rows ahead
+// exchanges.  y is overwritten by the forward sweep.  Loads are issued a chunk of rows ahead
 // of the dependent recurrence.
 DEVI void helm_solve_serial_body(const long long l, const int comp, const GridDev &g,
                                  double *__restrict__ q, double *__restrict__ y,
                                  const unsigned char *__restrict__ icyl,
                                  const unsigned char *__restrict__ ocyl,
-                                 const double *__restrict__ lu, int nt) {
+                                 const double *__restrict__ lu, int nt, bool fold) {
   constexpr int CH = 16;
   if (l >= g.P) return;
   const long long P = g.P;
@@ -671,7 +670,7 @@ DEVI void helm_solve_serial_body(const long long l, const int comp, const GridDe
   double x1 = 0.0, x0 = carry * T.rd(last);
   auto put = [&](int r, double x) {
     double *o = q + (long long)r * P + l;
-    *o = *o + x;
+    *o = fold ? x : *o + x;
   };
   put(last, x0);
   for (int r0 = last - 1; r0 >= first; r0 -= CH) {
@@ -696,11 +695,11 @@ DEVI void helm_solve_serial_body(const long long l, const int comp, const GridDe
 __global__ __launch_bounds__(256) void k_helm_solve_serial(GridDev g, SolveIO io,
                                                            const unsigned char *__restrict__ icyl,
                                                            const unsigned char *__restrict__ ocyl,
-                                                           int nt, int comp) {
+                                                           int nt, int comp, bool fold) {
   helm_solve_serial_body((long long)blockIdx.x * 256 + threadIdx.x, comp, g,
                          comp == 0 ? io.q[0] : (comp == 1 ? io.q[1] : io.q[2]),
                          const_cast<double *>(comp == 0 ? io.y[0] : (comp == 1 ? io.y[1] : io.y[2])),
-                         icyl, ocyl, comp == 0 ? io.lu[0] : (comp == 1 ? io.lu[1] : io.lu[2]), nt);
+                         icyl, ocyl, comp == 0 ? io.lu[0] : (comp == 1 ? io.lu[1] : io.lu[2]), nt, fold);
 }
 
 // Grouped: blockIdx.y = instance.
@@ -712,7 +711,7 @@ __global__ __launch_bounds__(256) void k_helm_solve_serial_g(const StepDesc *__r
                          glob(d.f[comp == 0 ? TC_QT : (comp == 1 ? TC_QR : TC_QZ)]),
                          glob(d.f[comp == 0 ? TC_RHS : (comp == 1 ? TC_DQ : TC_QCAP)]),
                          glob(d.icyl), glob(d.ocyl),
-                         glob(comp == 0 ? d.lut : (comp == 1 ? d.lur : d.luz)), d.lu_nt);
+                         glob(comp == 0 ? d.lut : (comp == 1 ? d.lur : d.luz)), d.lu_nt, true);
 }
 
 // ---------------------------------------------------------------------------
@@ -1483,7 +1482,7 @@ static void launch_solve(tc_ctx *c, const SolveIO &io, int comp0, int ncomp) {
   }
   if (serial >> comp0 & 1) {
     hipLaunchKernelGGL(k_helm_solve_serial, dim3(line_blocks(c)), dim3(256), 0, c->stream, c->gd, io,
-                       c->mask, c->mask + c->P, c->lu_nt, comp0);
+                       c->mask, c->mask + c->P, c->lu_nt, comp0, FOLD);
     return;
   }
   const SolveShape s = solve_shape(c);

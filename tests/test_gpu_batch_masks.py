@@ -73,3 +73,20 @@ def test_masks_set_between_advances(tc, oracle, graph):
             _march(orcs[0], p, (ones, ones), n, n + 1)
             _march(orcs[1], p, masks, n, n + 1)
             _compare(b, ids, orcs, p["nrm"])
+
+
+@pytest.mark.parametrize("lpt,defer", [(1, -1), (2, -1), (1, 2), (2, 2)])
+@pytest.mark.parametrize("shape", [(20, 9, 29), (27, 10, 29), (20, 9, 101), (20, 9, 300), (16, 6, 810)])
+def test_grouped_kernels_with_masks(tc, oracle, shape, lpt, defer):
+    """Masks of their own on each member, on both walls, through every row
+    capacity; odd theta sizes have no deferred correction."""
+    p = small_params(tc, *shape, idtv=0, ntst=1000, ren=500.0, dtmin=1e-4, dtmax=1e-4, limitcfl=1e30)
+    with tc.Batch() as b:
+        ids, orcs = _batch(tc, oracle, p, b, (3, 4), dict(helm_lpt=lpt, defer=defer))
+        masks = [_masks(p, 5 + i, True) for i in ids]
+        for i, m in zip(ids, masks):
+            b.solver(i).set_masks(*m)
+        b.advance(2)
+        for o, m in zip(orcs, masks):
+            _march(o, p, m, 0, 2)
+        _compare(b, ids, orcs, p["nrm"])
