@@ -28,9 +28,9 @@ struct Grid {
 // Validates p and fills g; returns an empty string on success or the reason.
 std::string build_grid(const tc_params &p, Grid &g);
 
-// SlipBCs.F90:31-90 at time t: masks (nzm,nthm) column-major.
 // theta points the inner wall's pattern has moved by: all that slip_bcs takes from the time
 int slip_displacement(const tc_params &p, const Grid &g, double time);
+// SlipBCs.F90:31-90 at time t: masks (nzm,nthm) column-major.
 void slip_bcs(const tc_params &p, const Grid &g, double time, std::vector<int> &icyl,
               std::vector<int> &ocyl);
 

@@ -933,7 +933,7 @@ DEVI void helm_rhs_body(
 #pragma unroll
       for (int u = 0; u < LPT; u++) n1[u] = n2[u] = n3[u] = 0.0;
     }
-        const int sm = (k + 2) % 3, sc = k % 3, sn = (k + 1) % 3;  // planes k-1, k, k+1
+    const int sm = (k + 2) % 3, sc = k % 3, sn = (k + 1) % 3;  // planes k-1, k, k+1
     const double *spk = sp[k & 1];
     const HelmPlane hc = ldk_record(g.hp + k);
     const RhsRow rw = ldk_record(rows + k);
@@ -966,7 +966,7 @@ DEVI void helm_rhs_body(
           y = wall_fold(&rows[k].x_t, &rows[k].xs_t, e_t, r * rw.sc_t, T(0, 0, 0), slip1 ? qp : qm);
         st_nt(yt + o, y);
       }
-            // q_r (planes 2..nrm; the walls have no row)
+      // q_r (planes 2..nrm; the walls have no row)
       if (k >= 2) {
         const double dphv = explicit_qr_g(g, hc, T, R, Z, k);
         const double r = rhs_qr(hc, a, R(-1, 0, 0), R(0, 0, 0), R(1, 0, 0), pr_c, pr_km[u], dphv, h2[u]);
@@ -974,7 +974,7 @@ DEVI void helm_rhs_body(
         st_nt(yr + o, row_fold(rw.s_r, rw.e_r, rw.am_r, rw.ap_r, r * rw.sc_r, R(-1, 0, 0), R(0, 0, 0),
                                 R(1, 0, 0)));
       }
-            // q_z
+      // q_z
       {
         const double qcv = explicit_qz_g(g, hc, T, R, Z, k);
         const double qm = (k > 1) ? Z(-1, 0, 0) : 0.0, qp = (k < nrm) ? Z(1, 0, 0) : 0.0;
@@ -985,7 +985,7 @@ DEVI void helm_rhs_body(
           y = wall_fold(&rows[k].x_z, &rows[k].xs_z, e_z, r * rw.sc_z, Z(0, 0, 0), slip1 ? qp : qm);
         st_nt(yz + o, y);
       }
-            pr_km[u] = pr_c;
+      pr_km[u] = pr_c;
       cm[u][0] = T(0, 0, 0);
       cm[u][1] = T(0, 0, 1);
       cm[u][2] = R(0, 0, 0);

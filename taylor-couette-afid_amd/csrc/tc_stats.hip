@@ -252,7 +252,7 @@ void launch_dump(tc_ctx *c, int kind, int k) {
 }
 
 // Statistics pass over the current fields.  stats: CalcStats (with the
-// vorticity); diss: CalcDissipation, whose volume sum lands in c->red_out[0].
+// vorticity); diss: CalcDissipation, whose volume sum lands in c->red_host[0].
 void launch_stats(tc_ctx *c, bool stats, bool diss) {
   timer_begin(c, "stats");
   const dim3 grid((unsigned)(NBAND * band_blocks(c->nzm)) * (unsigned)c->nrm);
