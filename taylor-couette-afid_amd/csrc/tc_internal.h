@@ -264,7 +264,8 @@ struct tc_ctx {
   int divfft_stage = 1;  // fused divergence FFT: stage the divergence rows in LDS first
   int poisson_pq = 13;  // rows per thread of the radial Poisson solve (13 or 26)
   int helm_lpt = 1;  // tiles of 4*helm_lpt z rows in the fused Helmholtz kernel (1 or 2)
-  int helm_slots[2] = {512, 512};  // its blocks resident on the device at once (plain, corrected)
+  // its blocks resident on the device at once, [no-slip everywhere][corrected]
+  int helm_slots[2][2] = {{512, 512}, {512, 512}};
   tc_tuning tuning{};  // effective tuning (helm_lpt 0 = chosen by occupancy)
   // statistics accumulators (TC_NSTATS x nrm x nzm) and per-line partials
   double *stats = nullptr, *stat_part = nullptr;

@@ -1541,7 +1541,7 @@ static long long helm_tiles(const tc_ctx *c, int lpt) {
 // 512x512x97 412 / 428 and 614 / 631, 512x512x65 281 / 330 and 414 / 502).
 // Over 30 sizes it is at most 3.4% over the best count.
 static int helm_segments(const tc_ctx *c, int lpt, bool corr, int n) {
-  const long long tiles = n * helm_tiles(c, lpt), slots = c->helm_slots[corr];
+  const long long tiles = n * helm_tiles(c, lpt), slots = c->helm_slots[c->masks_uniform_one][corr];
   auto cost = [&](int s) {
     const long long len = (c->nrm + s - 1) / s, rounds = (tiles * s + slots - 1) / slots;
     return 32 * rounds * (len + 4) + 5 * len;
@@ -1571,12 +1571,12 @@ static void launch_rhs(tc_ctx *c, const double *pr, const CorrIn &ci, double *pr
 
 // blocks of the fused front that one compute unit holds (asked once: every
 // device this library is built for is alike)
-template <int LPT, bool CORR, bool PAIR>
+template <bool UNIFORM, int LPT, bool CORR, bool PAIR>
 static int resident_blocks(int cus) {
   static const int per_cu = [] {
     int n = 0;
     const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &n, k_helm_rhs<true, LPT, CORR, PAIR>, PAIR ? 128 * LPT : FT_N, 0);
+        &n, k_helm_rhs<UNIFORM, LPT, CORR, PAIR>, PAIR ? 128 * LPT : FT_N, 0);
     return e == hipSuccess && n > 0 ? n : 2;
   }();
   return per_cu * cus;
@@ -1596,15 +1596,20 @@ void choose_helm_schedule(tc_ctx *c, int lpt) {
   if (cus <= 0) cus = 256;
   const bool pair = c->nthm % 2 == 0;
   if (lpt == 0)
-    lpt = pair || helm_tiles(c, 2) * (c->nrm / 32) >= resident_blocks<2, false, false>(cus) ? 2 : 1;
+    lpt = pair || helm_tiles(c, 2) * (c->nrm / 32) >= resident_blocks<true, 2, false, false>(cus) ? 2 : 1;
   c->helm_lpt = lpt;
-  if (pair) {
-    c->helm_slots[0] = lpt == 2 ? resident_blocks<2, false, true>(cus) : resident_blocks<1, false, true>(cus);
-    c->helm_slots[1] = lpt == 2 ? resident_blocks<2, true, true>(cus) : resident_blocks<1, true, true>(cus);
-  } else {
-    c->helm_slots[0] = c->helm_slots[1] =
-        lpt == 2 ? resident_blocks<2, false, false>(cus) : resident_blocks<1, false, false>(cus);
-  }
+  auto ask = [&](auto uniform, int *slots) {
+    constexpr bool U = decltype(uniform)::value;
+    if (pair) {
+      slots[0] = lpt == 2 ? resident_blocks<U, 2, false, true>(cus) : resident_blocks<U, 1, false, true>(cus);
+      slots[1] = lpt == 2 ? resident_blocks<U, 2, true, true>(cus) : resident_blocks<U, 1, true, true>(cus);
+    } else {
+      slots[0] = slots[1] =
+          lpt == 2 ? resident_blocks<U, 2, false, false>(cus) : resident_blocks<U, 1, false, false>(cus);
+    }
+  };
+  ask(std::false_type{}, c->helm_slots[0]);
+  ask(std::true_type{}, c->helm_slots[1]);
 }
 
 void launch_helmholtz_fused(tc_ctx *c) {
