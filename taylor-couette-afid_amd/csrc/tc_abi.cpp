@@ -192,12 +192,10 @@ void write_partitioned(const Matrix &A, int first, int last, std::vector<double>
 void build_component(const tc::Grid &g, int comp, unsigned vars, const Matrix *A, double betadx,
                      bool serial, double *T, int nt, tc::RhsRow *rows) {
   using R = tc::RhsRow;
-  double R::*const f[3][4] = {{&R::sc_t, &R::am_t, &R::ap_t, &R::s_t},
-                              {&R::sc_r, &R::am_r, &R::ap_r, &R::s_r},
-                              {&R::sc_z, &R::am_z, &R::ap_z, &R::s_z}};
+  double R::*const f[3][5] = {{&R::sc_t, &R::am_t, &R::ap_t, &R::s_t, &R::e_t},
+                              {&R::sc_r, &R::am_r, &R::ap_r, &R::s_r, &R::e_r},
+                              {&R::sc_z, &R::am_z, &R::ap_z, &R::s_z, &R::e_z}};
   const bool wall = comp != tc::LU_QR, qt = comp == tc::LU_QT;
-  double R::*const et[4] = {&R::e0_t, &R::e1_t, &R::e2_t, &R::e3_t};
-  double R::*const ez[4] = {&R::e0_z, &R::e1_z, &R::e2_z, &R::e3_z};
   double R::*const x = qt ? &R::x_t : &R::x_z, R::*const xs = qt ? &R::xs_t : &R::xs_z;
   const int k0 = wall ? 1 : 2, nrm = g.nrm;
   std::vector<double> D((size_t)g.nr, 1.0);
@@ -211,27 +209,23 @@ void build_component(const tc::Grid &g, int comp, unsigned vars, const Matrix *A
       write_serial(A[v], Tv, sum);
     else
       write_partitioned(A[v], k0 - 1, nrm - 1, D, v == 3, Tv, sum);
+    if (v != 3) continue;
     for (int kc = k0; kc <= nrm; kc++) {
-      tc::RhsRow &row = rows[kc];
       const int q = kc - 1;
-      if (v == 3) {
-        row.*f[comp][0] = rhs_scale(g, comp, kc, betadx) * D[q];
-        row.*f[comp][1] = serial ? A[3].lo[q] : -Tv[tc::LU_ROW * q];
-        row.*f[comp][2] = serial ? A[3].up[q] : -Tv[tc::LU_ROW * q + 1];
-        row.*f[comp][3] = (double)sum[q];
-        if (wall && (kc == 1 || kc == nrm)) {
-          // beside a free-slip wall: one off-diagonal
-          double lo, up;
-          wall_row(g, comp, kc, true, betadx, lo, up);
-          const double off = kc == 1 ? up : lo;
-          row.*x = off * D[q];
-          row.*xs = (1.0 + off) * D[q];
-        }
-      }
-      const bool slip = wall && ((kc == 1 && !(v & 1)) || (kc == nrm && !(v >> 1)));
-      const double e = (double)(sum[q] - (slip ? row.*xs : row.*f[comp][3]));
-      row.*(!wall ? &R::e_r : (qt ? et[v] : ez[v])) = e;
+      rows[kc].*f[comp][0] = rhs_scale(g, comp, kc, betadx) * D[q];
+      rows[kc].*f[comp][1] = serial ? A[3].lo[q] : -Tv[tc::LU_ROW * q];
+      rows[kc].*f[comp][2] = serial ? A[3].up[q] : -Tv[tc::LU_ROW * q + 1];
+      rows[kc].*f[comp][3] = (double)sum[q];
+      rows[kc].*f[comp][4] = (double)(sum[q] - (rows[kc].*f[comp][3]));
     }
+  }
+  if (!wall) return;
+  for (int kc : {1, nrm}) {
+    double lo, up;
+    wall_row(g, comp, kc, true, betadx, lo, up);
+    const double off = kc == 1 ? up : lo;
+    rows[kc].*x = off * D[kc - 1];
+    rows[kc].*xs = (1.0 + off) * D[kc - 1];
   }
 }
 

@@ -66,17 +66,18 @@ constexpr int LU_ROW = 8;
 
 // What the right-hand sides need of the Helmholtz matrices of plane k (row
 // k of each component), one record per plane and substep slot: the scaling
-// of the right-hand side, the off-diagonals and the row sum s + e of the
-// matrix that the factors multiply out to (e: what s rounds away, which
-// differs between the mask variants).  x, xs: off-diagonal and s of the two
-// wall rows where the wall is free-slip (k = 1: ap, k = nrm: am).  The q_r
-// rows next to the walls do not couple to them (q_r is fixed there).
+// of the right-hand side, the off-diagonals and the row sum s + e (e: what s
+// rounds away) of the matrix that the no-slip factors multiply out to.  The
+// other mask variants share them but for the two wall rows, whose one
+// off-diagonal and row sum beside a free-slip wall are x and xs.  (Rows of
+// their own for each variant, chosen a lane: no closer to 64 bits, and the
+// grooved front 3-13% slower.)  The q_r rows next to the walls do not couple
+// to them (q_r is fixed there).
 struct RhsRow {
-  double sc_t, am_t, ap_t, s_t, sc_r, am_r, ap_r, s_r, e_r, sc_z, am_z, ap_z, s_z;
-  double e0_t, e1_t, e2_t, e3_t, e0_z, e1_z, e2_z, e3_z;  // by mask variant icyl + 2 ocyl
+  double sc_t, am_t, ap_t, s_t, e_t, sc_r, am_r, ap_r, s_r, e_r, sc_z, am_z, ap_z, s_z, e_z;
   double x_t, xs_t, x_z, xs_z;
 };
-static_assert(sizeof(RhsRow) == 25 * 8, "RhsRow is twenty-five doubles");
+static_assert(sizeof(RhsRow) == 19 * 8, "RhsRow is nineteen doubles");
 
 struct Timer {
   std::string name;

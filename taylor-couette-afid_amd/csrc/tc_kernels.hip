@@ -756,17 +756,11 @@ DEVI double row_fold(double s, double e, double am, double ap, double scr, doubl
                      double qp) {
   return fma(s, q0, fma(e, q0, fma(am, qm - q0, fma(ap, qp - q0, scr))));
 }
-// e of a line's mask variant: ic, oc its bits
-DEVI double row_e(double e0, double e1, double e2, double e3, bool ic, bool oc) {
-  const double i = ic ? e3 : e2, o = ic ? e1 : e0;
-  return oc ? i : o;
-}
-
 // The same for a point beside a free-slip wall: one off-diagonal, x, towards
 // the interior value qi, and the row sum xs, read here so that the planes
 // without walls hold neither.
-DEVI double wall_fold(const double *x, const double *xs, double e, double scr, double q0, double qi) {
-  return fma(ldk(xs), q0, fma(e, q0, fma(ldk(x), qi - q0, scr)));
+DEVI double wall_fold(const double *x, const double *xs, double scr, double q0, double qi) {
+  return fma(ldk(xs), q0, fma(ldk(x), qi - q0, scr));
 }
 
 constexpr int FT_N = 256, FT_I = 64, FT_J = FT_N / FT_I, FT_W = FT_I + 2;
@@ -950,10 +944,7 @@ DEVI void helm_rhs_body(
       const double pr_c = spk[base[u]], pr_im = spk[base[u] - 1], pr_jm = spk[base[u] - FT_W];
       const long long o = (long long)(k - 1) * P + l[u];
       // whether the matrix rows of q_theta and q_z are those beside a free-slip wall
-      const bool ic = UNIFORM || fic[u] != 0.0, oc = UNIFORM || foc[u] != 0.0;
-      const bool slip1 = k == 1 && !ic, slipn = k == nrm && !oc;
-      const double e_t = row_e(rw.e0_t, rw.e1_t, rw.e2_t, rw.e3_t, ic, oc);
-      const double e_z = row_e(rw.e0_z, rw.e1_z, rw.e2_z, rw.e3_z, ic, oc);
+      const bool slip1 = !UNIFORM && k == 1 && fic[u] == 0.0, slipn = !UNIFORM && k == nrm && foc[u] == 0.0;
       // q_theta
       {
         const double dqv = explicit_qt_g(g, hc, T, R, Z, k);
@@ -961,9 +952,9 @@ DEVI void helm_rhs_body(
         double r = rhs_qt<UNIFORM>(g, hc, a, k, qm, T(0, 0, 0), qp, pr_c, pr_im, dqv, h1[u], fic[u], foc[u]);
         st_nt(ru1 + o, dqv);
         if (k == 1) r = r + a.bc1;
-        double y = row_fold(rw.s_t, e_t, rw.am_t, rw.ap_t, r * rw.sc_t, qm, T(0, 0, 0), qp);
+        double y = row_fold(rw.s_t, rw.e_t, rw.am_t, rw.ap_t, r * rw.sc_t, qm, T(0, 0, 0), qp);
         if (slip1 || slipn)
-          y = wall_fold(&rows[k].x_t, &rows[k].xs_t, e_t, r * rw.sc_t, T(0, 0, 0), slip1 ? qp : qm);
+          y = wall_fold(&rows[k].x_t, &rows[k].xs_t, r * rw.sc_t, T(0, 0, 0), slip1 ? qp : qm);
         st_nt(yt + o, y);
       }
       // q_r (planes 2..nrm; the walls have no row)
@@ -980,9 +971,9 @@ DEVI void helm_rhs_body(
         const double qm = (k > 1) ? Z(-1, 0, 0) : 0.0, qp = (k < nrm) ? Z(1, 0, 0) : 0.0;
         const double r = rhs_qz<UNIFORM>(g, hc, a, k, qm, Z(0, 0, 0), qp, pr_c, pr_jm, qcv, h3[u], fic[u], foc[u]);
         st_nt(ru3 + o, qcv);
-        double y = row_fold(rw.s_z, e_z, rw.am_z, rw.ap_z, r * rw.sc_z, qm, Z(0, 0, 0), qp);
+        double y = row_fold(rw.s_z, rw.e_z, rw.am_z, rw.ap_z, r * rw.sc_z, qm, Z(0, 0, 0), qp);
         if (slip1 || slipn)
-          y = wall_fold(&rows[k].x_z, &rows[k].xs_z, e_z, r * rw.sc_z, Z(0, 0, 0), slip1 ? qp : qm);
+          y = wall_fold(&rows[k].x_z, &rows[k].xs_z, r * rw.sc_z, Z(0, 0, 0), slip1 ? qp : qm);
         st_nt(yz + o, y);
       }
       pr_km[u] = pr_c;
@@ -1266,19 +1257,17 @@ DEVI void helm_rhs_pair_body(
         const double fic = (double)(wall >> u & 1), foc = (double)(wall >> u >> 2 & 1);
         const double pr_c = spk[b], pr_im = spk[b - 1], pr_jm = spk[b - PT_W];
         // whether the matrix rows of q_theta and q_z are those beside a free-slip wall
-        const bool ic = UNIFORM || (wall >> u & 1), oc = UNIFORM || (wall >> u & 4);
-        const bool slip1 = k == 1 && !ic, slipn = k == nrm && !oc;
-        const double e_t = row_e(rw.e0_t, rw.e1_t, rw.e2_t, rw.e3_t, ic, oc);
-        const double e_z = row_e(rw.e0_z, rw.e1_z, rw.e2_z, rw.e3_z, ic, oc);
+        const bool slip1 = !UNIFORM && k == 1 && !(wall >> u & 1);
+        const bool slipn = !UNIFORM && k == nrm && !(wall >> u & 4);
         // q_theta
         e1[u] = explicit_qt_g(g, hc, T, R, Z, k);
         const double tm = (k > 1) ? T(-1, 0, 0) : 0.0, tp = (k < nrm) ? T(1, 0, 0) : 0.0;
         double r = rhs_qt<UNIFORM>(g, hc, a, k, tm, T(0, 0, 0), tp, pr_c, pr_im, e1[u],
                                    u ? h1.y : h1.x, fic, foc);
         if (k == 1) r = r + a.bc1;
-        g1[u] = row_fold(rw.s_t, e_t, rw.am_t, rw.ap_t, r * rw.sc_t, tm, T(0, 0, 0), tp);
+        g1[u] = row_fold(rw.s_t, rw.e_t, rw.am_t, rw.ap_t, r * rw.sc_t, tm, T(0, 0, 0), tp);
         if (slip1 || slipn)
-          g1[u] = wall_fold(&rows[k].x_t, &rows[k].xs_t, e_t, r * rw.sc_t, T(0, 0, 0), slip1 ? tp : tm);
+          g1[u] = wall_fold(&rows[k].x_t, &rows[k].xs_t, r * rw.sc_t, T(0, 0, 0), slip1 ? tp : tm);
         // q_r (planes 2..nrm; the walls have no row)
         if (k >= 2) {
           e2[u] = explicit_qr_g(g, hc, T, R, Z, k);
@@ -1292,9 +1281,9 @@ DEVI void helm_rhs_pair_body(
         const double zm = (k > 1) ? Z(-1, 0, 0) : 0.0, zp = (k < nrm) ? Z(1, 0, 0) : 0.0;
         r = rhs_qz<UNIFORM>(g, hc, a, k, zm, Z(0, 0, 0), zp, pr_c, pr_jm, e3[u], u ? h3.y : h3.x,
                             fic, foc);
-        g3[u] = row_fold(rw.s_z, e_z, rw.am_z, rw.ap_z, r * rw.sc_z, zm, Z(0, 0, 0), zp);
+        g3[u] = row_fold(rw.s_z, rw.e_z, rw.am_z, rw.ap_z, r * rw.sc_z, zm, Z(0, 0, 0), zp);
         if (slip1 || slipn)
-          g3[u] = wall_fold(&rows[k].x_z, &rows[k].xs_z, e_z, r * rw.sc_z, Z(0, 0, 0), slip1 ? zp : zm);
+          g3[u] = wall_fold(&rows[k].x_z, &rows[k].xs_z, r * rw.sc_z, Z(0, 0, 0), slip1 ? zp : zm);
         if (u)
           pkm.y = pr_c;
         else
