@@ -83,7 +83,7 @@ int tc_create(const tc_params *p, tc_ctx **out);
  * fields take the TC_* environment override, else the default. */
 typedef struct tc_tuning {
   int helm_lpt;   /* tiles of 4*helm_lpt z rows of the fused Helmholtz kernel: 1, 2 (0: by size) */
-  int fft_t_lds;  /* LDS bytes of a theta-FFT block (default 16384 up to NTM = 384, else 32768) */
+  int fft_t_lds;  /* LDS bytes of a theta-FFT block (default 16384 up to NTM = 256, odd 384, else 32768) */
   int fft_z_lds;  /* LDS bytes of a z-FFT block (default: 16 columns within 32768 up to
                      NZM = 256, else 65536) */
   int fft_z_nt;   /* threads of a z-FFT block: 256 (default up to NZM = 256) or 512 */

@@ -426,13 +426,18 @@ tc_tuning resolve_tuning(const tc_tuning *in, int nthm, int nzm, int nrm) {
   if (t.helm_lpt == 0) t.helm_lpt = std::max(0, std::min(2, env("TC_HELM_LPT", 0)));
   // FFT blocks: short lines need few per block, or the grid is too coarse to
   // fill the device and the last column tile mostly empty (64x64x65: 65
-  // blocks of 32 theta lines or 64 columns).  theta, us with 16 / 32 KiB
-  // (divergence fused): n = 64 11.4 / 14.7, 192 34.2 / 35.1, 375 123 / 124;
-  // inverse 375 72 / 76; 512 keeps its four lines in 32 KiB.  z, us with the
-  // default here / 64 KiB and 512 threads: n = 64 7.7 / 9.0, 128 (192 columns)
-  // 18.1 / 24.5, 240 62 / 67, 256 51 / 54; 512 keeps eight columns in 64 KiB
-  // and 512 threads.
-  if (t.fft_t_lds == 0) t.fft_t_lds = env("TC_FFT_T_LDS", nthm <= 384 ? 16384 : 32768);
+  // blocks of 32 theta lines or 64 columns).  theta, us with 16 / 32 KiB,
+  // forward with the divergence and inverse: n = 64 11.4 / 14.7, 96 15.9 /
+  // 17.2 and 10.4 / 11.7, 192 34.2 / 35.1, 240 88.8 / 94.1 and 54.1 / 57.1;
+  // past four lines in 16 KiB only odd sizes, whose rows are not staged in
+  // pairs, are no slower: 375 123 / 124 and 72 / 76, but 324 148 / 137 and 78
+  // / 83, 384 147 / 137 and 82 / 79 (a step of 384x384x289 7.74 / 7.66 ms),
+  // 512 160 / 162 and 93 / 84.  z, us with the default up to 256 / 64 KiB and
+  // 512 threads: n = 64 7.7 / 9.0, 128 (192 columns) 18.1 / 24.5, 216 31.5 /
+  // 33.7, 256 30.3 / 33.4, then even: 270 52.6 / 51.5, 320 44.8 / 46.0, 384
+  // 51.3 / 54.3, 450 74.0 / 73.0 (129 columns, 97 planes).
+  if (t.fft_t_lds == 0)
+    t.fft_t_lds = env("TC_FFT_T_LDS", nthm <= 256 || (nthm % 2 && nthm <= 384) ? 16384 : 32768);
   if (t.fft_z_lds == 0)
     t.fft_z_lds = env("TC_FFT_Z_LDS", nzm <= 256 ? std::min(32768, 16 * 16 * nzm) : 65536);
   if (t.fft_z_nt == 0) t.fft_z_nt = env("TC_FFT_Z_NT", nzm <= 256 ? 256 : 512) == 256 ? 256 : 512;
