@@ -606,8 +606,9 @@ struct SolveIO {
 };
 
 // The components of a line group are consecutive, and the groups contiguous
-// per XCD: the six arrays then move together (1024x1024x769: 7.8 ms against
-// 8.2 with one component after the other, 512x512x385: 885 against 960 us).
+// per XCD: the six arrays then move together (1024x1024x769: 7.82 ms against
+// 8.43-8.56 with one component after the other, the step alike; no difference
+// at 512x512x385 and below).
 template <int R, bool UNIFORM, bool FOLD, bool CHUNKS>
 __global__ __launch_bounds__(R > 32 ? 512 : 1024) void k_helm_solve(
     GridDev g, SolveIO io, const unsigned char *__restrict__ icyl,
@@ -638,8 +639,8 @@ __global__ __launch_bounds__(R > 32 ? 512 : 1024) void k_helm_solve_g(
 }
 
 // Serial form, one line per lane: dgttrs as it is, for factors with row
-// exchanges.  y is overwritten by the forward sweep.  Loads are issued a chunk of rows ahead
-// of the dependent recurrence.
+// exchanges.  y is overwritten by the forward sweep.  Loads are issued a chunk
+// of rows ahead of the dependent recurrence.
 DEVI void helm_solve_serial_body(const long long l, const int comp, const GridDev &g,
                                  double *__restrict__ q, double *__restrict__ y,
                                  const unsigned char *__restrict__ icyl,
@@ -1016,13 +1017,14 @@ DEVI void helm_rhs_body(
 // dph planes with one more row of halo on either side, so the corrected
 // fields are the ones the per-substep path would have stored, bit for bit.
 // Against one line or two z-rows of lines per thread, with the correction:
-// 256x256x193 343 -> 318 us, 512x512x385 2576 -> 2491 us, 1024x1024x769 20.5
-// -> 17.95 ms (HBM bound at the larger sizes: 4.9 of the 5.7 TB/s that
-// fifteen streamed arrays reach).  The kernels ask for two waves per SIMD:
-// the masked form, corrected, once left that when it was not asked to
-// (192x128x129 125 us at one wave, 88 at two).  It holds what only the two
-// wall planes need nowhere else (wall_fold) and takes 222 registers with none
-// spilled; with the wall rows' entries in every plane 24 to 53 were.
+// 256x256x193 343 -> 313 us, 512x512x385 2576 -> 2491 us, 1024x1024x769 20.5
+// -> 18.4 ms (HBM bound at the larger sizes: 4.9 of the 5.7 TB/s that fifteen
+// streamed arrays reach; with the fold in differences 303, 2490 us, 18.8 ms).
+// The kernels ask for two waves per SIMD: the masked form, corrected, once
+// left that when it was not asked to (192x128x129 125 us at one wave, 88 at
+// two).  It holds what only the two wall planes need nowhere else (wall_fold)
+// and takes 222 registers with none spilled; with the wall rows' entries in
+// every plane 24 to 53 were.
 // (The outermost column of the tile on either side is staged only to keep
 // pairs aligned; nothing reads it.)
 constexpr int PT_W = FT_I + 4, PT_P = PT_W / 2;  // tile row: i0-2 .. i0+65
@@ -1413,16 +1415,17 @@ const RhsRow *rhs_rows(const tc_ctx *c, int ns) {
 static unsigned line_blocks(const tc_ctx *c) { return (unsigned)((c->P + 255) / 256); }
 
 // Shape of the partitioned solve: waves per block and the row capacity R of
-// its kernel, by the grid's shape alone (an instance's bits must not depend
-// on what it shares a launch with).  Past eight waves of 100 rows a line goes in chunks.  Few rows a
-// wave shorten the chain where there are few lines, many keep more loads in
-// flight where there are many: measured us with R = 25 / 50 / 100,
-// 128x128x97 18 / 21 / 32, 256x256x193 123 / 125 / 129, 512x512x193 474 / 497
-// / 483, 1024x512x193 939 / 973 / 957, 256x256x385 257 / 239 / 254,
-// 512x512x385 970 / 953 / 887.  Nine waves of 25 and more no longer pair up
+// its kernel, by the grid's shape alone (an instance's bits must not depend on
+// what it shares a launch with).  Past eight waves of 100 rows a line goes in
+// chunks.  Few rows a wave shorten the chain where there are few lines, many
+// keep more loads in flight where there are many: measured us with R = 25 / 50
+// / 100, 128x128x97 19 / 19 / 24, 256x256x193 120 / 124 / 128, 512x512x193 481
+// / 490 / 485, 1024x512x193 938 / 971 / 956, 256x256x385 260 / 248 / 244,
+// 512x512x385 1016 / 955 / 970 (941 / 869 / 828 in processes where every
+// kernel of the step ran faster).  Nine waves of 25 and more no longer pair up
 // on a compute unit: 96x96x250 27 / 23, 128x128x225 39.5 / 37.8, 192x128x240
-// 66 / 61, 256x256x205 161 / 140, 256x256x250 179 / 160 / 164, 512x512x225
-// 631 / 569, 480x512x250 640 / 582 / 589 (64x64x225 17.7 / 18.5).
+// 66 / 61, 256x256x205 161 / 140, 256x256x250 178 / 164, 512x512x225 633 /
+// 571, 480x512x250 640 / 592 (64x64x225 17.7 / 19.4).
 struct SolveShape {
   int ns, rows;
   bool chunks;  // lines of more than ns*rows rows
@@ -1523,12 +1526,12 @@ static long long helm_tiles(const tc_ctx *c, int lpt) {
 // the counts within 2% of the least of that, the largest, of at least two
 // planes each; up to 128 planes one segment where no count saves 2.5% (longer
 // ones drift apart, and tiles no longer find their neighbours' halo rows in
-// cache).  Measured us, one segment / the count taken (with the correction from the second pair on):
-// 64x64x65 133 / 16, 256x256x193 553 / 207 and 810 / 303, 512x512x385 1912 /
-// 1632 and 2728 / 2465, 1024x1024x769 14082 / 12488 and 20394 / 18653; one is
-// the best where the tiles fill the device and there are few planes (two:
-// 512x512x97 412 / 428 and 614 / 631, 512x512x65 281 / 330 and 414 / 502).
-// Over 30 sizes it is at most 3.4% over the best count.
+// cache).  Measured us, one segment / the count taken (with the correction
+// from the second pair on): 64x64x65 133 / 16, 256x256x193 553 / 207 and 810 /
+// 303, 512x512x385 1912 / 1632 and 2728 / 2465, 1024x1024x769 14082 / 12488
+// and 20394 / 18653; one is the best where the tiles fill the device and there
+// are few planes (two: 512x512x97 412 / 428 and 614 / 631, 512x512x65 281 /
+// 330 and 414 / 502).  Over 30 sizes it is at most 3.4% over the best count.
 static int helm_segments(const tc_ctx *c, int lpt, bool corr, int n) {
   const long long tiles = n * helm_tiles(c, lpt), slots = c->helm_slots[c->masks_uniform_one][corr];
   auto cost = [&](int s) {
